@@ -728,8 +728,8 @@ def main():
     kcnt_all = torch.full((wl.heads, wl.nq), wl.nk, dtype=torch.int32, device=dev)
     ms_dense = timed(lambda: attend(kidx_all, kcnt_all, od), nd)
     del kidx_all, kcnt_all
-    # the masked dense walk (FVSR_ATTN_DENSE: every key block of each non-empty row, unselected ones masked; rows
-    # that select nothing are written as zeros without a walk); includes the mask -> list build (a few us)
+    # FVSR_ATTN_DENSE under the selected mask: the unselected blocks weigh exactly 0 and are not visited; includes the
+    # mask -> list build (a few us)
     ms_masked = timed(lambda: fvsr_lcsa.block_masked_attention(q, k, v, mask, wl.heads, out=od), nd)
     dense_flops = 4.0 * 128 * wl.heads * wl.lq * wl.lk
     cpu_inputs = None

@@ -42,7 +42,7 @@ typedef enum fvsr_dtype { FVSR_DTYPE_F32 = 0, FVSR_DTYPE_BF16 = 1 } fvsr_dtype;
  * reference documents it as 2-4x slower than dense and keeps it for study only. */
 typedef enum fvsr_attn_mode {
   FVSR_ATTN_AUTO = 0,    /* kernel when the expected kept fraction <= threshold, else dense (DiT.swift:517-522) */
-  FVSR_ATTN_DENSE = 1,   /* every key block visited, unselected blocks masked (blockMaskedAttention) */
+  FVSR_ATTN_DENSE = 1,   /* blockMaskedAttention's result: softmax over all keys, unselected blocks masked */
   FVSR_ATTN_KERNEL = 3   /* only the selected key blocks visited (kernelBlockAttention) */
 } fvsr_attn_mode;
 
@@ -120,9 +120,9 @@ int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t
                                 void* o, void* stream);
 
 /* Replaces `FlashVSRAttentionOps.kernel` / `.dense` (SparseAttention.swift:190-202): attention under a block mask
- * (H, Nq, Nk) f32 tested > 0.5. mode FVSR_ATTN_KERNEL visits only the selected blocks; FVSR_ATTN_DENSE is the
- * dense fallback of `blockMaskedAttention` (DiT.swift:279-313): the same kernel walks EVERY key block and masks the
- * unselected ones, so its cost is that of full attention. Both return the same values. */
+ * (H, Nq, Nk) f32 tested > 0.5. FVSR_ATTN_DENSE is the dense fallback of
+ * `blockMaskedAttention` (DiT.swift:279-313). A masked block's weights are exactly 0, so both modes walk the selected
+ * blocks only and return the same values. */
 int fvsr_lcsa_attention_mask(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
                              int64_t lk, int heads, const float* block_mask, int mode, void* o, void* stream);
 
@@ -152,8 +152,8 @@ int fvsr_kv_ring_read(fvsr_kv_ring* ring, int layer, void* k_out, void* v_out, v
 int fvsr_lcsa_select_ring(fvsr_ctx* ctx, fvsr_kv_ring* ring, int layer, const void* qW, int64_t lq, int q_slices,
                           const uint8_t* local_dev, int topk, float* mask_out, float* probs_out, int32_t* kidx_out,
                           int32_t* kcnt_out, void* stream);
-/* Attention over the ring's held keys/values of `layer` from lists (mode KERNEL) or, mode DENSE, every held block
- * with the unselected masked (kidx/kcnt still name the selection). */
+/* Attention over the ring's held keys/values of `layer` from lists. Mode KERNEL takes the lists as they stand; mode
+ * DENSE takes them as a mask over the held blocks (the distinct listed blocks inside the held range, ascending). */
 int fvsr_lcsa_attention_ring(fvsr_ctx* ctx, fvsr_kv_ring* ring, int layer, const void* q, int64_t lq,
                              const int32_t* kidx, const int32_t* kcnt, int nk_stride, int mode, void* o,
                              void* stream);

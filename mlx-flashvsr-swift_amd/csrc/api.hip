@@ -22,18 +22,16 @@ int set_error(int status, const std::string& msg) {
 }
 
 // kernels (lcsa_attn.hip, lcsa_select.hip, kv_ring.hip)
-int launch_attention(int dtype, bool dense, const AttnArgs& a, hipStream_t stream);
-int launch_lists_from_mask(const float* mask, int rows, int nk, int32_t* kidx, int32_t* kcnt, uint8_t* sel,
-                           hipStream_t stream);
-int launch_sel_from_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_stride, int nk, uint8_t* sel,
-                          hipStream_t stream);
+int launch_attention(int dtype, const AttnArgs& a, hipStream_t stream);
+int launch_lists_from_mask(const float* mask, int rows, int nk, int32_t* kidx, int32_t* kcnt, hipStream_t stream);
+int launch_set_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_stride, int nk, int32_t* kidx_out,
+                     int32_t* kcnt_out, hipStream_t stream);
 int launch_scores_softmax(const float* pq, const float* pk, KeyMap kmap, int heads, int C, int nq, int nk, int s,
                           const uint8_t* local, float* probs, unsigned* hist, int q_slices, hipStream_t stream);
 size_t hist12_bytes(int heads, int q_slices);
 size_t topk_cand_bytes(int heads, int64_t nq);
 int launch_topk_emit(const float* probs, int heads, int nq, int nk, int q_slices, int topk, unsigned* hist,
-                     unsigned* cand, float* thr, float* mask_out, uint8_t* sel, int32_t* kidx, int32_t* kcnt,
-                     hipStream_t stream);
+                     unsigned* cand, float* thr, float* mask_out, int32_t* kidx, int32_t* kcnt, hipStream_t stream);
 int launch_qkv_epilogue(int dtype, const void* q, const void* k, const void* v, int f, int h, int w, int C, int t0,
                         const void* wq, const void* wk, float eps, const float* rope, void* q_out, void* k_out,
                         void* v_out, int dst_slot0, int capacity, int slice_blocks, int64_t kv_head_stride,
@@ -62,13 +60,12 @@ int launch_window_layout(int dtype, const void* x, void* out, int f, int h, int 
                          hipStream_t stream);
 
 constexpr int kMaxSelectKeyBlocks = 1920;    // scores stage LDS: (8 x (128 + Nk) + 2 x 64 x 132) fp32 + 8 x Nk B
-constexpr double kAutoThreshold = 0.45;      // DiT.swift:210
 
 static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // workspace carve for one select + attention call
 struct Carve {
-  size_t pq, pk, probs, kidx, kcnt, sel, order, counter, thr, hist, cand, total;
+  size_t pq, pk, probs, kidx, kcnt, order, counter, thr, hist, cand, total;
 };
 static Carve carve(int heads, int64_t nq, int64_t nk, int C) {
   Carve c;
@@ -78,7 +75,6 @@ static Carve carve(int heads, int64_t nq, int64_t nk, int C) {
   c.probs = off; off += align256((size_t)heads * nq * nk * 4);
   c.kidx = off; off += align256((size_t)heads * nq * nk * 4);
   c.kcnt = off; off += align256((size_t)heads * nq * 4);
-  c.sel = off; off += align256((size_t)heads * nq * nk);
   c.order = off; off += align256((size_t)heads * nq * 4);
   c.counter = off; off += 256;
   c.thr = off; off += align256((size_t)heads * nq * 4);   // per (head, query slice) thresholds (nq >= slices)
@@ -240,7 +236,7 @@ int fvsr_attention_mode_auto(int topk, int s, int nk, double threshold, double* 
 static int select_impl(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, const float* pk_src, bool pk_ready,
                        const void* kW, int64_t lk, KeyMap kmap, int nk, int heads, int q_slices, int s,
                        const uint8_t* local, int topk, float* mask_out, float* probs_out, int32_t* kidx,
-                       int32_t* kcnt, uint8_t* sel_out, hipStream_t stream, bool q_pooled = false) {
+                       int32_t* kcnt, hipStream_t stream, bool q_pooled = false) {
   const int C = heads * kHeadDim;
   const int64_t nq = ceil_div(lq, kBlock);
   FVSR_REQUIRE(nq == (int64_t)q_slices * s, FVSR_ERR_INVALID_ARG,
@@ -254,7 +250,6 @@ static int select_impl(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, con
   char* ws = (char*)ctx->ws;
   float* pq = (float*)(ws + cv.pq);
   float* probs = probs_out ? probs_out : (float*)(ws + cv.probs);
-  uint8_t* sel = sel_out ? sel_out : (uint8_t*)(ws + cv.sel);
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
   unsigned* hist = (unsigned*)(ws + cv.hist);
   const float* pk = pk_ready ? pk_src : (const float*)(ws + cv.pk);
@@ -271,7 +266,7 @@ static int select_impl(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, con
   if ((rc = launch_scores_softmax(pq, pk, kmap, heads, C, (int)nq, nk, s, local, probs, hist, q_slices, stream)))
     return rc;
   return launch_topk_emit(probs, heads, (int)nq, nk, q_slices, topk, hist, (unsigned*)(ws + cv.cand),
-                          (float*)(ws + cv.thr), mask_out, sel, kidx, kcnt, stream);
+                          (float*)(ws + cv.thr), mask_out, kidx, kcnt, stream);
 }
 
 int fvsr_lcsa_select(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, const void* kW, int64_t lk, int heads,
@@ -288,7 +283,7 @@ int fvsr_lcsa_select(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, const
   const int64_t nk = ceil_div(lk, kBlock);
   FVSR_REQUIRE(nk <= kMaxSelectKeyBlocks, FVSR_ERR_UNSUPPORTED, "too many key blocks for selection");
   return select_impl(ctx, dtype, qW, lq, nullptr, false, kW, lk, plain_key_map(), (int)nk, heads, q_slices,
-                     s, local_dev, topk, mask_out, probs_out, kidx_out, kcnt_out, nullptr, (hipStream_t)stream);
+                     s, local_dev, topk, mask_out, probs_out, kidx_out, kcnt_out, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -296,13 +291,13 @@ int fvsr_lcsa_select(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, const
 // ---------------------------------------------------------------------------------------------------------------
 // K/V token-major (rows of heads * 128 elements of es bytes, lk rows); the ring's head-major layout is set by its caller
 static AttnArgs make_args(const void* q, int64_t lq, const void* k, const void* v, int64_t lk, int heads,
-                          const int32_t* kidx, const int32_t* kcnt, const uint8_t* sel, int nk_stride, int nk,
-                          KeyMap map, void* o, int es) {
+                          const int32_t* kidx, const int32_t* kcnt, int nk_stride, int nk, KeyMap map,
+                          void* o, int es) {
   AttnArgs a{};
   a.q = q; a.k = k; a.v = v; a.o = o;
   a.lq = lq; a.lk = lk;
   a.heads = heads; a.ld = heads * kHeadDim;
-  a.kidx = kidx; a.kcnt = kcnt; a.sel = sel;
+  a.kidx = kidx; a.kcnt = kcnt;
   a.nk_stride = nk_stride;
   a.nq = (int)ceil_div(lq, kBlock);
   a.nk = nk;
@@ -348,9 +343,9 @@ int fvsr_lcsa_attention(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, con
   FVSR_REQUIRE(nk_stride > 0, FVSR_ERR_INVALID_ARG, "nk_stride must be > 0");
   const int nk = (int)ceil_div(lk, kBlock);
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
-  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, nullptr, nk_stride, nk, plain_key_map(), o, esize(dtype));
+  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, nk_stride, nk, plain_key_map(), o, esize(dtype));
   if ((rc = attach_order(ctx, a, nk))) return rc;
-  return launch_attention(dtype, false, a, (hipStream_t)stream);
+  return launch_attention(dtype, a, (hipStream_t)stream);
 }
 
 int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
@@ -361,13 +356,13 @@ int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t
   FVSR_REQUIRE(kidx && kcnt, FVSR_ERR_INVALID_ARG, "kidx and kcnt must be non-NULL");
   FVSR_REQUIRE(nk_stride > 0, FVSR_ERR_INVALID_ARG, "nk_stride must be > 0");
   const int nk = (int)ceil_div(lk, kBlock);
-  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, nullptr, nk_stride, nk, plain_key_map(), o, esize(dtype));
+  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, nk_stride, nk, plain_key_map(), o, esize(dtype));
   // only the bf16 walk keeps a row order and a work counter; the fp32 kernel has neither, so no row cap applies
   if (dtype == FVSR_DTYPE_BF16 &&
       (rc = noalloc_scratch(ctx->device, (int64_t)heads * a.nq, &a.order, &a.counter)))
     return rc;
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
-  return launch_attention(dtype, false, a, (hipStream_t)stream);
+  return launch_attention(dtype, a, (hipStream_t)stream);
 }
 
 int fvsr_lcsa_attention_mask(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
@@ -383,13 +378,12 @@ int fvsr_lcsa_attention_mask(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq
   char* ws = (char*)ctx->ws;
   int32_t* kidx = (int32_t*)(ws + cv.kidx);
   int32_t* kcnt = (int32_t*)(ws + cv.kcnt);
-  uint8_t* sel = (uint8_t*)(ws + cv.sel);
   hipStream_t st = (hipStream_t)stream;
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
-  if ((rc = launch_lists_from_mask(block_mask, (int)(heads * nq), (int)nk, kidx, kcnt, sel, st))) return rc;
-  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, sel, (int)nk, (int)nk, plain_key_map(), o, esize(dtype));
+  if ((rc = launch_lists_from_mask(block_mask, (int)(heads * nq), (int)nk, kidx, kcnt, st))) return rc;
+  AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, (int)nk, (int)nk, plain_key_map(), o, esize(dtype));
   if ((rc = attach_order(ctx, a, nk))) return rc;
-  return launch_attention(dtype, mode == FVSR_ATTN_DENSE, a, st);
+  return launch_attention(dtype, a, st);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -650,15 +644,15 @@ int fvsr_lcsa_select_ring(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void*
   const int nk = r->count[layer] * r->s;
   return select_impl(ctx, r->dtype, qW, lq, r->layer_pooled(layer), true, nullptr, (int64_t)nk * kBlock,
                      r->map(layer), nk, r->heads, q_slices, r->s, local_dev, topk, mask_out, probs_out, kidx_out,
-                     kcnt_out, nullptr, (hipStream_t)stream);
+                     kcnt_out, (hipStream_t)stream);
 }
 
 static int attention_ring_impl(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* q, int64_t lq,
-                               const int32_t* kidx, const int32_t* kcnt, int nk_stride, const uint8_t* sel,
-                               bool dense, void* o, hipStream_t stream, bool o_grid = false) {
+                               const int32_t* kidx, const int32_t* kcnt, int nk_stride, void* o,
+                               hipStream_t stream, bool o_grid = false) {
   const int nk = r->count[layer] * r->s;
   AttnArgs a = make_args(q, lq, r->layer_k(layer), r->layer_v(layer), (int64_t)nk * kBlock, r->heads, kidx, kcnt,
-                         sel, nk_stride, nk, r->map(layer), o, esize(r->dtype));
+                         nk_stride, nk, r->map(layer), o, esize(r->dtype));
   a.kv_head_stride = r->head_stride();   // head-major
   a.kv_ld = kHeadDim;
   a.kv_bytes = (int64_t)r->heads * r->head_stride() * esize(r->dtype);
@@ -668,7 +662,7 @@ static int attention_ring_impl(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const 
   }
   int rc = attach_order(ctx, a, nk);
   if (rc) return rc;
-  return launch_attention(r->dtype, dense, a, stream);
+  return launch_attention(r->dtype, a, stream);
 }
 
 int fvsr_lcsa_attention_ring(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* q, int64_t lq,
@@ -686,14 +680,17 @@ int fvsr_lcsa_attention_ring(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const vo
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
   const int64_t nq = ceil_div(lq, kBlock);
   const int nk = r->count[layer] * r->s;
-  uint8_t* sel = nullptr;
   if (mode == FVSR_ATTN_DENSE) {
     const Carve cv = carve(r->heads, nq, nk, r->C);
     if ((rc = ensure_ws(ctx, cv.total))) return rc;
-    sel = (uint8_t*)((char*)ctx->ws + cv.sel);
-    if ((rc = launch_sel_from_lists(kidx, kcnt, (int)(r->heads * nq), nk_stride, nk, sel, st))) return rc;
+    int32_t* const set_idx = (int32_t*)((char*)ctx->ws + cv.kidx);
+    int32_t* const set_cnt = (int32_t*)((char*)ctx->ws + cv.kcnt);
+    if ((rc = launch_set_lists(kidx, kcnt, (int)(r->heads * nq), nk_stride, nk, set_idx, set_cnt, st))) return rc;
+    kidx = set_idx;
+    kcnt = set_cnt;
+    nk_stride = nk;
   }
-  return attention_ring_impl(ctx, r, layer, q, lq, kidx, kcnt, nk_stride, sel, mode == FVSR_ATTN_DENSE, o, st);
+  return attention_ring_impl(ctx, r, layer, q, lq, kidx, kcnt, nk_stride, o, st);
 }
 
 int fvsr_lcsa_layer(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* qW, int64_t lq, const void* k_new,
@@ -723,14 +720,11 @@ int fvsr_lcsa_layer(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* qW, i
   char* ws = (char*)ctx->ws;
   int32_t* kidx = (int32_t*)(ws + cv.kidx);
   int32_t* kcnt = (int32_t*)(ws + cv.kcnt);
-  uint8_t* sel = (uint8_t*)(ws + cv.sel);
   rc = select_impl(ctx, r->dtype, qW, lq, r->layer_pooled(layer), true, nullptr, (int64_t)nk * kBlock,
                    r->map(layer), nk, r->heads, q_slices, r->s, local_dev, topk, mask_out, probs_out, kidx, kcnt,
-                   sel, st);
+                   st);
   if (rc) return ring_rewind(r, layer, mark, rc);
-  int use = mode;
-  if (use == FVSR_ATTN_AUTO) fvsr_attention_mode_auto(topk, r->s, nk, kAutoThreshold, nullptr, &use);
-  rc = attention_ring_impl(ctx, r, layer, qW, lq, kidx, kcnt, nk, sel, use == FVSR_ATTN_DENSE, o, st);
+  rc = attention_ring_impl(ctx, r, layer, qW, lq, kidx, kcnt, nk, o, st);
   if (rc) return ring_rewind(r, layer, mark, rc);
   return fvsr_kv_ring_evict(r, layer);
 }
@@ -767,14 +761,11 @@ int fvsr_lcsa_layer_qkv(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* q
   const int nk = r->count[layer] * r->s;
   int32_t* kidx = (int32_t*)(ws + cv.kidx);
   int32_t* kcnt = (int32_t*)(ws + cv.kcnt);
-  uint8_t* sel = (uint8_t*)(ws + cv.sel);
   rc = select_impl(ctx, r->dtype, q_work, lq, r->layer_pooled(layer), true, nullptr, (int64_t)nk * kBlock,
                    r->map(layer), nk, r->heads, q_slices, r->s, local_dev, topk, mask_out, probs_out, kidx, kcnt,
-                   sel, st, true);
+                   st, true);
   if (rc) return ring_rewind(r, layer, mark, rc);
-  int use = mode;
-  if (use == FVSR_ATTN_AUTO) fvsr_attention_mode_auto(topk, r->s, nk, kAutoThreshold, nullptr, &use);
-  rc = attention_ring_impl(ctx, r, layer, q_work, lq, kidx, kcnt, nk, sel, use == FVSR_ATTN_DENSE, o, st, true);
+  rc = attention_ring_impl(ctx, r, layer, q_work, lq, kidx, kcnt, nk, o, st, true);
   if (rc) return ring_rewind(r, layer, mark, rc);
   return fvsr_kv_ring_evict(r, layer);
 }

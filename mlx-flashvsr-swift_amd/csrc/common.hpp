@@ -132,7 +132,6 @@ struct AttnArgs {
   int ld;                // channels per token = heads * 128
   const int32_t* kidx;   // (H, nq, nk_stride) listed key blocks
   const int32_t* kcnt;   // (H, nq)
-  const uint8_t* sel;    // (H, nq, nk) selection bytes, dense mode only
   int nk_stride;
   int nq;
   int nk;

@@ -79,8 +79,8 @@ __device__ __forceinline__ float rescale_if_grown(float mxc, float& m_run, float
 // the copies of the step before it, so a tile is in LDS a step before the step that first reads it.
 //
 // Softmax with a lazily raised reference per query row: S = K Q^T in fp32 from the bf16 inputs (keys that do not
-// take part score -2^100: in the dense walk by one extra rank-1 MFMA per tile, in the sparse walk by a select on the
-// rare tile with fewer than 32 keys: a ragged end, an index outside [0, nk), the tile past the walk's end), then
+// take part score -2^100, by a select on the rare tile with fewer than 32 keys: a ragged end, an index outside
+// [0, nk), the tile past the walk's end), then
 // P = exp2(c S - m) with one v_fma per score (c = log2(e)/sqrt(128), applied to the fp32 scores as the reference
 // does, SparseAttention.swift:96; m, the row's reference, first the exact max of its first tile). A tile whose
 // partial row sum exceeds 2^32 (its scores outgrew the reference by about 27 or more, in log2 units) raises the
@@ -163,18 +163,17 @@ __device__ __forceinline__ int next_dealt_item(int32_t* counters, int rows) {
 }
 
 // LDS operand requests of chunk / pair j >= 2 (j = 0, 1: micro-round 0), in micro-rounds of a step with QG query
-// groups per wave and EXT mask MFMAs ahead of the first QK chunk: 7 (QG 2) or 4 (QG 1) micro-rounds before the QK
-// MFMA that uses them, micro-round 0 at the earliest
-template <int QG, int EXT>
+// groups per wave: 7 (QG 2) or 4 (QG 1) micro-rounds before the QK MFMA that uses them, micro-round 0 at the earliest
+template <int QG>
 constexpr int attn_read_at(int j) {
-  const int r = EXT + 2 * QG * j - (QG == 2 ? 7 : 4);
+  const int r = 2 * QG * j - (QG == 2 ? 7 : 4);
   return r > 0 ? r : 0;
 }
 
-template <bool DENSE, int QG>
+template <int QG>
 __global__ __attribute__((amdgpu_flat_work_group_size(256 / QG, 256 / QG), amdgpu_waves_per_eu(3 - QG, 3 - QG)))
 void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
-                      const uint8_t* __restrict__ sel, const bf16* __restrict__ Q, bf16* __restrict__ O,
+                      const bf16* __restrict__ Q, bf16* __restrict__ O,
                       const int32_t* __restrict__ order, int32_t* __restrict__ counter) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * kVRing];
   __shared__ int item_s;
@@ -218,8 +217,7 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
     continue;
   }
   const int32_t* __restrict__ klist = kidx + (int64_t)row_id * a.nk_stride;
-  const uint8_t* __restrict__ srow = DENSE ? sel + (int64_t)row_id * a.nk : nullptr;
-  const int nblocks = DENSE ? a.nk : min(cnt, a.nk_stride);
+  const int nblocks = min(cnt, a.nk_stride);
 
   // Q as the B operand of S^T = K Q^T (the bf16 inputs as they are; the scale c is applied to the fp32 scores):
   // group q holds queries qb*128 + kQW*wave + 32*q + l32, lane (query, k-half g) dims 16t + 8g .. +7
@@ -283,16 +281,13 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
     dma16<kVRing + SLOT * kTileBytes + P * 4 * kRowBytes>(vrs, dma_base, voff_v[P], soff);
   };
   // walked block b: buffer offset of its first row (past the buffer past the end of the walk) and its keys taking
-  // part (0 if unselected in the dense walk or outside [0, nk); else up to 128, fewer for a ragged last block)
-  // A walked block's entry e: its key block index (sparse walk) or its selection byte (dense walk), -1 past the
-  // end. The loop loads each entry one block before it derives the offset and key count from it, so the load's
-  // wait is covered by the waits of the steps in between.
-  auto walk_entry = [&](int b) -> int { return b < nblocks ? (DENSE ? (int)srow[b] : klist[b]) : -1; };
-  auto entry_soff = [&](int b, int e) -> int { return b < nblocks ? block_soff(DENSE ? b : e) : (int)range; };
-  auto entry_keys = [&](int b, int e) -> int {
-    if (b >= nblocks) return 0;
-    const int j = DENSE ? b : e;
-    if ((unsigned)j >= (unsigned)a.nk || (DENSE && e == 0)) return 0;
+  // part (0 outside [0, nk); else up to 128, fewer for a ragged last block). A walked block's entry is its key block
+  // index, -1 past the end. The loop loads each entry one block before it derives the offset and key count from it,
+  // so the load's wait is covered by the waits of the steps in between.
+  auto walk_entry = [&](int b) -> int { return b < nblocks ? klist[b] : -1; };
+  auto entry_soff = [&](int b, int j) -> int { return b < nblocks ? block_soff(j) : (int)range; };
+  auto entry_keys = [&](int b, int j) -> int {
+    if (b >= nblocks || (unsigned)j >= (unsigned)a.nk) return 0;
     return (int)min<int64_t>(kBlock, a.lk - (int64_t)j * kBlock);
   };
   auto walk_soff = [&](int b) -> int { return entry_soff(b, walk_entry(b)); };
@@ -321,52 +316,28 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
   };
   // the reference of a raw row max (masked keys only: 0)
   auto ref_of = [&](float mx) -> float { return mx > kNoKey ? mx * c_scale : 0.f; };
-  // the extra MFMA step, a v_mfma_f32_32x32x8_bf16 (k = 8, half the cost of a k = 16 step): A lane (key l32, g = 0)
-  // holds k-slot {masked}, B lane (query, g = 0) {-2^100}, all other k-slots 0: keys that do not take part score
-  // -2^100 and their exponentials are exactly 0
-  i16x4 bext;
-  {
-    bf16x4 b = bf16x4{};
-    if (g == 0) b[0] = (bf16)kMaskedScore;
-    bext = __builtin_bit_cast(i16x4, b);
-  }
-  auto aext = [&](int valid) -> i16x4 {
-    bf16x4 x = bf16x4{};
-    if (g == 0) x[0] = l32 >= valid ? (bf16)1.0f : (bf16)0.0f;
-    return __builtin_bit_cast(i16x4, x);
-  };
-  auto mfma_ext = [&](const i16x4& ax, const i16x4& bx) -> f32x16 {
-    return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(ax, bx, f32x16{}, 0, 0, 0);
-  };
-  // The sparse walk lists selected blocks only, so its tiles are whole (32 keys) but for a ragged last block, a listed
-  // index outside [0, nk) and the tile past the end of the walk, whose rows all load as zeros. It starts S at zero
-  // (no mask MFMA) and, on a tile with fewer than 32 keys taking part (a wave-uniform branch), sets the scores of the
-  // keys at or past `valid` to -2^100 afterwards: the values the mask MFMA gives there (their K rows are zeros).
+  // The walk lists selected blocks only, so its tiles are whole (32 keys) but for a ragged last block, a listed
+  // index outside [0, nk) and the tile past the end of the walk, whose rows all load as zeros. S starts at zero and,
+  // on a tile with fewer than 32 keys taking part (a wave-uniform branch), the scores of the keys at or past `valid`
+  // are set to -2^100 afterwards: their exponentials are exactly 0.
   // Lane element i of a 32 x 32 MFMA result is key row 8 (i / 4) + 4 g + i % 4.
   auto mask_tile = [&](f32x16& s, int valid) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + 4 * g + (i & 3) >= valid ? kMaskedScore : s[i];
   };
-  // mask MFMAs per step: the dense walk's tiles mix selected and unselected blocks
-  constexpr int kExt = DENSE ? QG : 0;
   lds_char* const lds = (lds_char*)(uintptr_t)smem_lds;
-  // S^T = K Q^T (keys that do not take part: - 2^100) for both groups, K from ring slot SLOT
+  // S^T = K Q^T (keys that do not take part: -2^100) for every group, K from ring slot SLOT
   auto qk = [&](auto slot_c, int valid, f32x16 (&s)[QG]) {
     constexpr int SLOT = decltype(slot_c)::value;
     bf16x8 kk[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) kk[t] = *(const lds_bf16x8*)(lds + SLOT * kTileBytes + k_off[t]);
-    if constexpr (DENSE) {
-      const i16x4 ax = aext(valid);
-#pragma unroll
-      for (int q = 0; q < QG; ++q) s[q] = mfma_ext(ax, bext);
-    }
 #pragma unroll
     for (int t = 0; t < 8; ++t)
 #pragma unroll
       for (int q = 0; q < QG; ++q)
-        s[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk[t], qop[q][t], (DENSE || t > 0) ? s[q] : f32x16{}, 0, 0, 0);
-    if (!DENSE && valid < kTileKeys) {
+        s[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk[t], qop[q][t], t > 0 ? s[q] : f32x16{}, 0, 0, 0);
+    if (valid < kTileKeys) {
 #pragma unroll
       for (int q = 0; q < QG; ++q) mask_tile(s[q], valid);
     }
@@ -430,20 +401,6 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
     int o0 = walk_soff(0), o1 = walk_soff(1), o2 = walk_soff(2);
     int n0 = walk_keys(0), n1 = walk_keys(1), n2 = walk_keys(2);
     int e3 = walk_entry(3);
-    if (MODE == 0 && DENSE) {
-      // the reference comes from the tile the sparse walk starts with (the first tile of the first listed block),
-      // so both walks do the same arithmetic on every selected tile and agree bit for bit
-      const int jr = klist[0];
-      issue_k(C0{}, block_soff(jr));
-      FVSR_WAIT_VM_LGKM0(0);
-      __builtin_amdgcn_s_barrier();
-      qk(C0{}, (unsigned)jr < (unsigned)a.nk ? sub_valid((int)min<int64_t>(kBlock, a.lk - (int64_t)jr * kBlock), 0)
-                                             : 0,
-         sA);
-#pragma unroll
-      for (int q = 0; q < QG; ++q) set_ref(q, ref_of(row_max(sA[q])));
-      __builtin_amdgcn_s_barrier();   // every wave is done with K slot 0 before the walk refills it
-    }
     // prologue = virtual steps -4 .. -1: K(0..3) and V(-2..1); V(-2), V(-1) are zeros, so step 0's PV of the
     // (zero) previous P adds exact zeros
     issue_k(C0{}, o0);                issue_v(C2{}, (int)range);
@@ -452,8 +409,8 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
     issue_k(C3{}, o0 + 3 * sub_bytes); issue_v(C1{}, o0 + sub_bytes);
     sync_steps(3);   // K(0) landed
     qk(C0{}, sub_valid(n0, 0), sA);
-    if (MODE == 0 && !DENSE) {
-      // reference = the exact row max of tile 0 (scaled), as the dense walk's pre-step computes it
+    if (MODE == 0) {
+      // reference = the exact row max of tile 0 (scaled)
 #pragma unroll
       for (int q = 0; q < QG; ++q) set_ref(q, ref_of(row_max(sA[q])));
     }
@@ -490,11 +447,11 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
 #pragma unroll
         for (int q = 0; q < QG; ++q) m_row[q] = fmaxf(m_row[q], row_max(s_cur[q]));
       } else {
-        // 16 * QG micro-rounds with one MFMA each (17 * QG in the dense walk), fenced so the order below is the
-        // issue order, then one more for the last exponential. A wave issues in order and an MFMA occupies the
+        // 16 * QG micro-rounds with one MFMA each, fenced so the order below is the issue order, then one more for the
+        // last exponential. A wave issues in order and an MFMA occupies the
         // matrix core for 32 cycles: every MFMA is followed by a slice of the other work, which issues while it runs
-        // (MFMAs grouped back to back would leave that work unoverlapped). MFMA order: (dense walk) the mask MFMA of
-        // QK(T+1) for each query group, then for c = 0..7 QK chunk c (each group) and PV pair c (each group).
+        // (MFMAs grouped back to back would leave that work unoverlapped). MFMA order: for c = 0..7 QK chunk c (each
+        // group) and PV pair c (each group).
         // Slices: exponential I of S(T) in micro-round I (pairs packed to bf16 and summed a micro-round later); the
         // LDS operands of chunk / pair j requested up to 4 micro-rounds before use (attn_read_at); one of the step's
         // buffer->LDS copies every 4 micro-rounds.
@@ -520,8 +477,6 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
           if constexpr (R < kDmaK) dma_k(KS{}, std::integral_constant<int, R>{}, soff_k);
           else dma_v(VS{}, std::integral_constant<int, R - kDmaK>{}, soff_v);
         };
-        i16x4 ax{};
-        if constexpr (DENSE) ax = aext(valid_next);
         float sum[QG][2];
         float xv[2];   // the exponentials of the last two micro-rounds
         auto micro = [&](auto i_c) {
@@ -532,14 +487,12 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
           }
           static_for<2, 8>([&](auto j_c) {
             constexpr int J = decltype(j_c)::value;
-            if constexpr (attn_read_at<QG, kExt>(J) == I) read_ops(J);
+            if constexpr (attn_read_at<QG>(J) == I) read_ops(J);
           });
-          if constexpr (I < kExt) {
-            s_nxt[I] = mfma_ext(ax, bext);
-          } else if constexpr (I < kExt + 16 * QG) {
-            constexpr int c = (I - kExt) / (2 * QG), w = (I - kExt) % (2 * QG);
+          if constexpr (I < 16 * QG) {
+            constexpr int c = I / (2 * QG), w = I % (2 * QG);
             if constexpr (w < QG) {
-              if constexpr (DENSE || c > 0)
+              if constexpr (c > 0)
                 s_nxt[w] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk[c], qop[w][c], s_nxt[w], 0, 0, 0);
               else
                 s_nxt[w] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk[0], qop[w][0], f32x16{}, 0, 0, 0);
@@ -572,11 +525,11 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
             xv[I & 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_cur[q][idx], c_scale, negm[q]));
           }
           if constexpr ((I & 3) == 1 && I / 4 < kDmaStep) dma(std::integral_constant<int, I / 4>{});
-          if constexpr (I == kExt + 16 * QG - (DENSE ? 1 : 0))
+          if constexpr (I == 16 * QG)
             read_first(std::integral_constant<int, (SUB + 2) & 3>{}, std::integral_constant<int, SUB>{});
           __builtin_amdgcn_sched_barrier(0);
         };
-        static_for<0, kExt + 16 * QG + (DENSE ? 0 : 1)>(micro);
+        static_for<0, 16 * QG + 1>(micro);
         float part[QG];
         bool grow = false;
 #pragma unroll
@@ -618,7 +571,7 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
           part_max[q] = fmaxf(part_max[q], part[q]);
         }
         // last in the step: a branch before the row sums would let the compiler sink the exponentials past it
-        if (!DENSE && valid_next < kTileKeys) {
+        if (valid_next < kTileKeys) {
 #pragma unroll
           for (int q = 0; q < QG; ++q) mask_tile(s_nxt[q], valid_next);
         }
@@ -698,7 +651,7 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
 
 // Rows (head, query block) for the persistent bf16 walk, and the per-XCD queue counters. One workgroup. First a
 // counting sort by decreasing key-list length in 255 bins of ceil(longest / 255) blocks (exact lengths up to 255
-// blocks; the dense walk: every non-empty row is a full walk). Then every wave of `grid` consecutive items of that order (one
+// blocks). Then every wave of `grid` consecutive items of that order (one
 // item per workgroup) is re-sorted by row id (head-major, neighbouring query blocks together) and dealt so that XCD x
 // (workgroups b with b % 8 == x, dispatch is round-robin over the XCDs) holds positions x, x + 8, .. of the wave:
 // one contiguous range of rows, whose key lists overlap, so the XCD's L2 serves the key blocks they share.
@@ -710,7 +663,7 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
 // already and is dealt as it stands.
 constexpr int kOrderLdsRows = 8192;
 __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restrict__ kcnt, int rows, int nk_stride,
-                                                          int dense, int grid, int32_t* __restrict__ order,
+                                                          int grid, int32_t* __restrict__ order,
                                                           int32_t* __restrict__ counters) {
   constexpr int kBins = 256;
   constexpr int kWords = 4096;   // row-id bitmap words: the bitmap rank serves up to 32 x 4096 rows
@@ -756,14 +709,14 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
     if (__ballot(mixed) != 0 && lane == 0) s_mixed = 1;
   }
   __syncthreads();
-  // every list of one length (the cross-attention's and the dense fallback's lists): the row-id order is already
+  // every list of one length (the cross-attention's lists): the row-id order is already
   // sorted by length and each of its waves by row id, so the sort and the ranking are skipped and the rows are dealt
   // where they stand
   const bool one_len = s_mixed == 0;
   if (!one_len) {
     const int width = max(1, (s_longest + kBins - 2) / (kBins - 1));   // blocks per bin
     auto bin_len = [&](int c) -> int {   // bin 0 = the longest lists
-      const int len = c <= 0 ? 0 : (dense ? 1 : min((c + width - 1) / width, kBins - 1));
+      const int len = c <= 0 ? 0 : min((c + width - 1) / width, kBins - 1);
       return kBins - 1 - len;
     };
     auto bin_of = [&](int r) -> int { return bin_len(list_len(r)); };
@@ -884,7 +837,6 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 // ------------------------------------------------------------------------------------------------------------
 // fp32 (parity lane)
 // ------------------------------------------------------------------------------------------------------------
-template <bool DENSE>
 __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
   constexpr int BK = 32;          // keys per tile
   constexpr int LDR = 132;        // padded fp32 row stride (floats): conflict-free operand reads
@@ -911,8 +863,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
     return;
   }
   const int32_t* __restrict__ klist = a.kidx + (int64_t)row_id * a.nk_stride;
-  const uint8_t* __restrict__ srow = DENSE ? a.sel + (int64_t)row_id * a.nk : nullptr;
-  const int nblocks = DENSE ? a.nk : min(cnt, a.nk_stride);
+  const int nblocks = min(cnt, a.nk_stride);
   const int ntiles = nblocks * (kBlock / BK);
   auto valid_keys = [&](int j, int part) -> int64_t {
     return (unsigned)j < (unsigned)a.nk ? a.lk - ((int64_t)j * kBlock + part * BK) : 0;
@@ -931,7 +882,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
   const int ld_row = tid >> 5, ld_c4 = tid & 31;
   auto load_tile = [&](int T) {
     const int jj = T >> 2, part = T & 3;
-    const int j = DENSE ? jj : klist[jj];
+    const int j = klist[jj];
     const int64_t valid = valid_keys(j, part);
     const int64_t row0 = valid > 0 ? a.map.row(j) + part * BK : 0;
 #pragma unroll
@@ -983,15 +934,8 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
       for (int b = 0; b < 4; ++b) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[b], qf[i][b], s, 0, 0, 0);
     }
 
-    const int jj = T >> 2;
-    bool dead = false;
-    if (DENSE) dead = srow[jj] == 0;
-    const int j = DENSE ? jj : klist[jj];
-    const int64_t valid = valid_keys(j, T & 3);
-    if (dead) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = -INFINITY;
-    } else if (valid < BK) {
+    const int64_t valid = valid_keys(klist[T >> 2], T & 3);
+    if (valid < BK) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (8 * (r >> 2) + 4 * g + (r & 3) >= valid) s[r] = -INFINITY;
@@ -1047,11 +991,10 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
 // key lists
 // ------------------------------------------------------------------------------------------------------------
 // Mask (rows, nk) f32 -> kcnt, kidx (selected ascending, then unselected ascending: argSort(!sel) of
-// SparseAttention.swift:175-177 with a stable order), sel bytes. One wave per row.
+// SparseAttention.swift:175-177 with a stable order). One wave per row.
 __global__ __launch_bounds__(256) void lists_from_mask_kernel(const float* __restrict__ mask, int rows, int nk,
                                                               int32_t* __restrict__ kidx,
-                                                              int32_t* __restrict__ kcnt,
-                                                              uint8_t* __restrict__ sel) {
+                                                              int32_t* __restrict__ kcnt) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -1064,7 +1007,6 @@ __global__ __launch_bounds__(256) void lists_from_mask_kernel(const float* __res
     const bool s = j < nk && mrow[j] > 0.5f;
     const uint64_t b = __ballot(s);
     if (s) krow[n_sel + __popcll(b & lt)] = j;
-    if (j < nk) sel[(int64_t)row * nk + j] = s ? 1 : 0;
     n_sel += __popcll(b);
   }
   int n_un = n_sel;
@@ -1078,22 +1020,34 @@ __global__ __launch_bounds__(256) void lists_from_mask_kernel(const float* __res
   if (lane == 0) kcnt[row] = n_sel;
 }
 
-// (kidx, kcnt) -> sel bytes (rows, nk), for the dense walk over caller-supplied lists. One wave per row.
-__global__ __launch_bounds__(256) void sel_from_lists_kernel(const int32_t* __restrict__ kidx,
-                                                             const int32_t* __restrict__ kcnt, int rows,
-                                                             int nk_stride, int nk, uint8_t* __restrict__ sel) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  uint8_t* srow = sel + (int64_t)row * nk;
-  for (int j = lane; j < nk; j += 64) srow[j] = 0;
-  __builtin_amdgcn_wave_barrier();
-  __threadfence_block();
+// Caller-supplied lists as the set they name: the distinct listed blocks inside [0, nk), ascending (kidx_out rows of
+// nk entries, kcnt_out). The dense fallback takes lists so: its mask holds a block once, whatever the order, the
+// repeats and the indices outside the key range of the list. One wave per row; the set is a bitmap in LDS.
+constexpr int kSetWords = 2048;   // 65,536 blocks: K/V buffers and ring layers are below 2 GiB, so nk < 2^16
+__global__ __launch_bounds__(64) void set_lists_kernel(const int32_t* __restrict__ kidx,
+                                                       const int32_t* __restrict__ kcnt, int nk_stride, int nk,
+                                                       int32_t* __restrict__ kidx_out,
+                                                       int32_t* __restrict__ kcnt_out) {
+  __shared__ unsigned bits[kSetWords];
+  const int row = blockIdx.x, lane = threadIdx.x;
+  const int words = (nk + 31) / 32;
+  for (int w = lane; w < words; w += 64) bits[w] = 0u;
+  __syncthreads();
   const int c = min(kcnt[row], nk_stride);
-  for (int jj = lane; jj < c; jj += 64) {
-    const int j = kidx[(int64_t)row * nk_stride + jj];
-    if (j >= 0 && j < nk) srow[j] = 1;
+  for (int i = lane; i < c; i += 64) {
+    const int j = kidx[(int64_t)row * nk_stride + i];
+    if ((unsigned)j < (unsigned)nk) atomicOr(&bits[j >> 5], 1u << (j & 31));
   }
+  __syncthreads();
+  int32_t* const out = kidx_out + (int64_t)row * nk;
+  int base = 0;
+  for (int w0 = 0; w0 < words; w0 += 64) {
+    unsigned m = w0 + lane < words ? bits[w0 + lane] : 0u;
+    const unsigned n = __popc(m), incl = wave_incl_scan(n);
+    for (int at = base + (int)(incl - n); m != 0u; m &= m - 1u) out[at++] = 32 * (w0 + lane) + __ffs(m) - 1;
+    base += (int)__shfl(incl, 63);
+  }
+  if (lane == 0) kcnt_out[row] = base;
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -1122,7 +1076,7 @@ static int attn_query_groups() {
   return qg;
 }
 
-int launch_attention(int dtype, bool dense, const AttnArgs& a, hipStream_t stream) {
+int launch_attention(int dtype, const AttnArgs& a, hipStream_t stream) {
   const int nwg = a.heads * a.nq;
   if (nwg <= 0) return FVSR_OK;
   dim3 grid(nwg), block(256);
@@ -1130,27 +1084,17 @@ int launch_attention(int dtype, bool dense, const AttnArgs& a, hipStream_t strea
     if (!a.order || !a.counter) return set_error(FVSR_ERR_INVALID_ARG, "attention: no workspace for the row order");
     // two workgroups (64 KB of LDS each) are resident per CU
     const int pwgs = std::min(nwg, std::min(2 * device_cus(), kMaxPersistentWgs));
-    hipLaunchKernelGGL(attn_order_kernel, dim3(1), dim3(1024), 0, stream, a.kcnt, nwg, a.nk_stride, dense ? 1 : 0,
-                       pwgs, a.order, a.counter);
+    hipLaunchKernelGGL(attn_order_kernel, dim3(1), dim3(1024), 0, stream, a.kcnt, nwg, a.nk_stride, pwgs, a.order,
+                       a.counter);
     const dim3 pgrid(pwgs);
-    if (attn_query_groups() == 2) {
-      if (dense)
-        hipLaunchKernelGGL((attn_bf16_kernel<true, 2>), pgrid, dim3(128), 0, stream, a, a.kidx, a.kcnt, a.sel,
-                           (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
-      else
-        hipLaunchKernelGGL((attn_bf16_kernel<false, 2>), pgrid, dim3(128), 0, stream, a, a.kidx, a.kcnt, a.sel,
-                           (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
-    } else {
-      if (dense)
-        hipLaunchKernelGGL((attn_bf16_kernel<true, 1>), pgrid, dim3(256), 0, stream, a, a.kidx, a.kcnt, a.sel,
-                           (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
-      else
-        hipLaunchKernelGGL((attn_bf16_kernel<false, 1>), pgrid, dim3(256), 0, stream, a, a.kidx, a.kcnt, a.sel,
-                           (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
-    }
+    if (attn_query_groups() == 2)
+      hipLaunchKernelGGL(attn_bf16_kernel<2>, pgrid, dim3(128), 0, stream, a, a.kidx, a.kcnt, (const bf16*)a.q,
+                         (bf16*)a.o, (const int32_t*)a.order, a.counter);
+    else
+      hipLaunchKernelGGL(attn_bf16_kernel<1>, pgrid, dim3(256), 0, stream, a, a.kidx, a.kcnt, (const bf16*)a.q,
+                         (bf16*)a.o, (const int32_t*)a.order, a.counter);
   } else {
-    if (dense) hipLaunchKernelGGL(attn_f32_kernel<true>, grid, block, 0, stream, a);
-    else hipLaunchKernelGGL(attn_f32_kernel<false>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL(attn_f32_kernel, grid, block, 0, stream, a);
   }
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
@@ -1205,20 +1149,18 @@ int noalloc_scratch(int device, int64_t rows, int32_t** order, int32_t** counter
   return FVSR_OK;
 }
 
-int launch_lists_from_mask(const float* mask, int rows, int nk, int32_t* kidx, int32_t* kcnt, uint8_t* sel,
-                           hipStream_t stream) {
+int launch_lists_from_mask(const float* mask, int rows, int nk, int32_t* kidx, int32_t* kcnt, hipStream_t stream) {
   if (rows <= 0) return FVSR_OK;
-  hipLaunchKernelGGL(lists_from_mask_kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, mask, rows, nk, kidx,
-                     kcnt, sel);
+  hipLaunchKernelGGL(lists_from_mask_kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, mask, rows, nk, kidx, kcnt);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }
 
-int launch_sel_from_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_stride, int nk, uint8_t* sel,
-                          hipStream_t stream) {
+int launch_set_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_stride, int nk, int32_t* kidx_out,
+                     int32_t* kcnt_out, hipStream_t stream) {
   if (rows <= 0) return FVSR_OK;
-  hipLaunchKernelGGL(sel_from_lists_kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, kidx, kcnt, rows,
-                     nk_stride, nk, sel);
+  if (nk > 32 * kSetWords) return set_error(FVSR_ERR_UNSUPPORTED, "more than 65,536 key blocks");
+  hipLaunchKernelGGL(set_lists_kernel, dim3(rows), dim3(64), 0, stream, kidx, kcnt, nk_stride, nk, kidx_out, kcnt_out);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }

@@ -23,7 +23,7 @@
 //                         bin, each workgroup gathers the bin's elements of its share of the row (held in
 //                         registers), and the last to arrive finishes the low 19 bits by three radix passes in LDS
 //                         (full-row 4-pass radix select when the bin is too large)
-//   topk_emit_kernel     one wave per query row: mask, selection bytes and compacted key lists (ballot + popcount),
+//   topk_emit_kernel     one wave per query row: mask and compacted key lists (ballot + popcount),
 //                        the row's probs loaded into registers at once
 #include "common.hpp"
 
@@ -568,7 +568,7 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
   if (tid == 0) thr_out[row] = __uint_as_float(prefix);
 }
 
-// Mask, selection bytes and key lists from the row thresholds: one wave per query row (head, query block). Lists
+// Mask and key lists from the row thresholds: one wave per query row (head, query block). Lists
 // hold the selected key blocks ascending, then the unselected ascending (argSort(!sel) of SparseAttention.swift:177
 // with a stable order). A row of up to 64 * kEmitChunks key blocks is loaded into registers first, every load in
 // flight at once (the probs were just written on other XCDs, so each load waits on the memory-side cache); longer
@@ -577,7 +577,7 @@ constexpr int kEmitChunks = 12;
 __global__ __launch_bounds__(256) void topk_emit_kernel(const float* __restrict__ probs,
                                                         const float* __restrict__ thr, int heads, int nq, int nk,
                                                         int q_slices, float* __restrict__ mask_out,
-                                                        uint8_t* __restrict__ sel, int32_t* __restrict__ kidx,
+                                                        int32_t* __restrict__ kidx,
                                                         int32_t* __restrict__ kcnt) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);   // h * nq + qi
@@ -595,10 +595,7 @@ __global__ __launch_bounds__(256) void topk_emit_kernel(const float* __restrict_
     const bool s = j < nk && p > th;
     const uint64_t b = __ballot(s);
     if (s) krow[n_sel + __popcll(b & lt)] = j;
-    if (j < nk) {
-      sel[roff + j] = s ? 1 : 0;
-      if (mask_out) mask_out[roff + j] = s ? 1.f : 0.f;
-    }
+    if (j < nk && mask_out) mask_out[roff + j] = s ? 1.f : 0.f;
     n_sel += __popcll(b);
   };
   auto emit_unselected = [&](int j0, float p, int& n_un) {
@@ -688,8 +685,7 @@ size_t hist12_bytes(int heads, int q_slices) {
 size_t topk_cand_bytes(int heads, int64_t nq) { return (size_t)heads * nq * kCandPerBlock * sizeof(unsigned); }
 
 int launch_topk_emit(const float* probs, int heads, int nq, int nk, int q_slices, int topk, unsigned* hist,
-                     unsigned* cand, float* thr, float* mask_out, uint8_t* sel, int32_t* kidx, int32_t* kcnt,
-                     hipStream_t stream) {
+                     unsigned* cand, float* thr, float* mask_out, int32_t* kidx, int32_t* kcnt, hipStream_t stream) {
   if (nq <= 0 || nk <= 0) return FVSR_OK;
   // enough workgroups per row that each one's share fits its registers (kThrRegs elements per thread)
   const int64_t row_n = (int64_t)(nq / q_slices) * nk;
@@ -699,7 +695,7 @@ int launch_topk_emit(const float* probs, int heads, int nq, int nk, int q_slices
                      nq, nk, q_slices, topk, ceil_div(row_n, (int64_t)parts), hist, cand, thr);
   FVSR_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(topk_emit_kernel, dim3((heads * nq + 3) / 4), dim3(256), 0, stream, probs, thr, heads, nq, nk,
-                     q_slices, mask_out, sel, kidx, kcnt);
+                     q_slices, mask_out, kidx, kcnt);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }

@@ -285,7 +285,7 @@ def kernel_block_attention(q, k, v, block_mask, heads: int, stream=None, out=Non
 
 
 def block_masked_attention(q, k, v, block_mask, heads: int, stream=None, out=None) -> torch.Tensor:
-    """Dense fallback: the same kernel walks every key block, unselected ones masked. DiT.swift:279-313."""
+    """The dense fallback's result (unselected blocks weigh exactly 0, so they are not visited). DiT.swift:279-313."""
     return _attn_mask(q, k, v, block_mask, heads, ATTN_DENSE, stream, out)
 
 

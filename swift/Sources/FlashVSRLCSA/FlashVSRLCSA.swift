@@ -100,7 +100,7 @@ public func kernelBlockAttention(_ c: LCSAContext, q: DeviceTensor, k: DeviceTen
                                        stream), "fvsr_lcsa_attention_mask")
 }
 
-/// `blockMaskedAttention` (DiT.swift:279-313): the dense fallback (same values, every key block visited).
+/// `blockMaskedAttention` (DiT.swift:279-313): the dense fallback (same values and, here, the same walk).
 public func blockMaskedAttention(_ c: LCSAContext, q: DeviceTensor, k: DeviceTensor, v: DeviceTensor,
                                  blockMask: DeviceTensor, heads: Int, out: DeviceTensor, stream: HIPStream = nil) {
     fvsrCheck(fvsr_lcsa_attention_mask(c.ctx, q.dtype, q.ptr, Int64(q.rows), k.ptr, v.ptr, Int64(k.rows),

@@ -84,6 +84,35 @@ def test_select_and_attention_over_ring_equal_plain(dev, dtype):
         ring.evict(0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,bh,bw", [(1, 1, 1), (2, 2, 3), (2, 5, 7)])
+def test_dense_mode_takes_lists_as_a_set(dev, dtype, heads, bh, bw):
+    """Mode DENSE reads caller-supplied lists as a mask: any order, repeats, indices outside the held range, a count
+    past the row stride and an empty row give, bit for bit, the kernel's result on the ascending distinct blocks
+    (key counts 3, 18 and 105: within one bitmap word, one word short of full, several words)."""
+    s = bh * bw
+    nk = 3 * s
+    gen = torch.Generator().manual_seed(100 * heads + nk)
+    ring = fvsr_lcsa.KVRing(1, heads, bh, bw, capacity=4, kv_len=3, dtype=dtype)
+    kn, vn, q = (torch.randn((n * 128, heads * 128), generator=gen).to(dtype).to(dev) for n in (nk, nk, s))
+    ring.append(0, kn, vn, 3)
+    stride = 2 * nk + 3
+    kidx = torch.randint(-2, nk + 3, (heads, s, stride), generator=gen, dtype=torch.int32)
+    kcnt = torch.randint(1, stride + 9, (heads, s), generator=gen, dtype=torch.int32)
+    kcnt[0, 0] = 0
+    mask = torch.zeros((heads, s, nk))
+    for h in range(heads):
+        for i in range(s):
+            for j in kidx[h, i, :min(int(kcnt[h, i]), stride)].tolist():
+                if 0 <= j < nk:
+                    mask[h, i, j] = 1.0
+    o = ring.attention(0, q, kidx.to(dev), kcnt.to(dev), fvsr_lcsa.ATTN_DENSE)
+    want_idx, want_cnt = O.block_lists(mask.numpy())
+    ref = ring.attention(0, q, torch.from_numpy(want_idx).to(dev), torch.from_numpy(want_cnt).to(dev))
+    assert torch.equal(o, ref)
+    assert (o[:128, :128] == 0).all()
+
+
 # AUTO with top-k 3 n s keeps an expected (3 n s + 1) / (s nk) of the pairs: over 0.45 in chunk 0 (dense walk), under
 # it afterwards (the kernel walk); both walks give the kernel's result bit for bit (DiT.swift:517-522)
 @pytest.mark.parametrize("mode", ["kernel", "auto"])
