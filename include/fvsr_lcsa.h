@@ -108,13 +108,13 @@ int fvsr_lcsa_attention(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, con
 
 /* No counterpart in the reference: fvsr_lcsa_attention for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). Same arguments and results as
- * fvsr_lcsa_attention; the persistent walk's row order and work counter live in a static device array of the
- * library (1 MiB + 256 B per GPU, held until the process ends) instead of the context workspace, so the call
- * allocates nothing. For bf16, heads * ceil(lq / 128) must be <= 262144 (FVSR_ERR_UNSUPPORTED otherwise, before any
- * device work); the fp32 kernel keeps no row order, so fp32 calls have no such cap. The context must exist
+ * fvsr_lcsa_attention; the walk's row order and work counter and the partial results of split rows live in a static
+ * device array of the library (34 MiB per GPU, held until the process ends) instead of the context workspace, so the
+ * call allocates nothing. For bf16, heads * ceil(lq / 128) must be <= 262144 (FVSR_ERR_UNSUPPORTED otherwise, before any
+ * device work); fp32 calls past that many rows run without the order. The context must exist
  * (fvsr_ctx_create takes the array's device address). Calls that overlap on one GPU share the array and race:
- * serialise them (one stream, or events). The call may be captured into a HIP graph: the order kernel rewrites the
- * row order and the work counter on every launch, so each replay starts from a clean scratch. */
+ * serialise them (one stream, or events). The call may be captured into a HIP graph: every launch writes
+ * what it reads of the scratch, so each replay starts clean. */
 int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
                                 int64_t lk, int heads, const int32_t* kidx, const int32_t* kcnt, int nk_stride,
                                 void* o, void* stream);

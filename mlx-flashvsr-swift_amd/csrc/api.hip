@@ -22,7 +22,8 @@ int set_error(int status, const std::string& msg) {
 }
 
 // kernels (lcsa_attn.hip, lcsa_select.hip, kv_ring.hip)
-int launch_attention(int dtype, const AttnArgs& a, hipStream_t stream);
+int launch_attention(int dtype, AttnArgs a, hipStream_t stream);
+int64_t attn_partial_items(int64_t rows, int nk);
 int launch_lists_from_mask(const float* mask, int rows, int nk, int32_t* kidx, int32_t* kcnt, hipStream_t stream);
 int launch_set_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_stride, int nk, int32_t* kidx_out,
                      int32_t* kcnt_out, hipStream_t stream);
@@ -49,7 +50,7 @@ int launch_residual_norm(void* x, const void* y, const void* gate, int64_t L, in
 int launch_rms_norm(const void* x, int64_t L, int C, float eps, const void* w, void* out, hipStream_t stream);
 int launch_full_lists(int rows, int nkc, int32_t* kidx, int32_t* kcnt, hipStream_t stream);
 int noalloc_scratch_init(int device);
-int noalloc_scratch(int device, int64_t rows, int32_t** order, int32_t** counter);
+int noalloc_scratch(int device, int dtype, AttnArgs& a);
 void rope_tables_host(double theta, float* out);
 int launch_ring_append(int dtype, const void* k_new, const void* v_new, int n_blocks, int C, bool grid_layout,
                        int nbh, int nbw, int slot0, int capacity, void* ring_k, void* ring_v, int64_t head_stride,
@@ -65,7 +66,7 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // workspace carve for one select + attention call
 struct Carve {
-  size_t pq, pk, probs, kidx, kcnt, order, counter, thr, hist, cand, total;
+  size_t pq, pk, probs, kidx, kcnt, order, counter, thr, hist, cand, part, total;
 };
 static Carve carve(int heads, int64_t nq, int64_t nk, int C) {
   Carve c;
@@ -80,6 +81,7 @@ static Carve carve(int heads, int64_t nq, int64_t nk, int C) {
   c.thr = off; off += align256((size_t)heads * nq * 4);   // per (head, query slice) thresholds (nq >= slices)
   c.hist = off; off += align256(hist12_bytes(heads, (int)nq));   // nq >= query slices
   c.cand = off; off += align256(topk_cand_bytes(heads, nq));
+  c.part = off; off += align256((size_t)attn_partial_items(heads * nq, (int)nk) * kPartialFloats * 4);
   c.total = off;
   return c;
 }
@@ -309,13 +311,15 @@ static AttnArgs make_args(const void* q, int64_t lq, const void* k, const void* 
   return a;
 }
 
-// the persistent walk's row order and work counter, carved from the context workspace (grown if needed)
+// the attention's row order, work counter and partial results, carved from the context workspace (grown if needed)
 static int attach_order(fvsr_ctx* ctx, AttnArgs& a, int64_t nk) {
   const Carve cv = carve(a.heads, a.nq, nk, a.ld);
   int rc = ensure_ws(ctx, cv.total);
   if (rc) return rc;
   a.order = (int32_t*)((char*)ctx->ws + cv.order);
   a.counter = (int32_t*)((char*)ctx->ws + cv.counter);
+  a.part_o = (float*)((char*)ctx->ws + cv.part);
+  a.part_items = attn_partial_items((int64_t)a.heads * a.nq, (int)nk);
   return FVSR_OK;
 }
 
@@ -357,10 +361,7 @@ int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t
   FVSR_REQUIRE(nk_stride > 0, FVSR_ERR_INVALID_ARG, "nk_stride must be > 0");
   const int nk = (int)ceil_div(lk, kBlock);
   AttnArgs a = make_args(q, lq, k, v, lk, heads, kidx, kcnt, nk_stride, nk, plain_key_map(), o, esize(dtype));
-  // only the bf16 walk keeps a row order and a work counter; the fp32 kernel has neither, so no row cap applies
-  if (dtype == FVSR_DTYPE_BF16 &&
-      (rc = noalloc_scratch(ctx->device, (int64_t)heads * a.nq, &a.order, &a.counter)))
-    return rc;
+  if ((rc = noalloc_scratch(ctx->device, dtype, a))) return rc;
   FVSR_HIP_CHECK(hipSetDevice(ctx->device));
   return launch_attention(dtype, a, (hipStream_t)stream);
 }

@@ -120,6 +120,8 @@ struct PoolDst {
   int nb, slot0, capacity, slice_blocks;
 };
 
+constexpr int kPartialFloats = kBlock * kHeadDim + 2 * kBlock;   // one item's partial attention result
+
 // Arguments of the attention kernels (lcsa_attn.hip).
 struct AttnArgs {
   const void* q;
@@ -144,6 +146,10 @@ struct AttnArgs {
   int32_t* order;        // (H * nq) rows, longest key list first (bf16 persistent walk; workspace)
   int32_t* counter;      // per-XCD queue counters of the walk, counter[8 x] for XCD x (workspace, 256 bytes; set by
                          // the order kernel)
+  int pieces;            // > 1: each row's key list is split into that many items (set by launch_attention)
+  float* part_o;         // workspace of part_items partial results (kPartialFloats each): the accumulators of the items
+  float* part_ml;        // (128 x 128 floats each), then their references and sums (2 x 128 floats each)
+  int64_t part_items;
   int o_nbh, o_nbw;      // > 0: write o in natural (f, h, w) token order of an (8 o_nbh, 8 o_nbw) grid (the
                          // reference's windowReverse, DiT.swift:121-126) instead of window order
   // output row of window-order query row r

@@ -7,9 +7,9 @@
 // bf16 (the production lane): a persistent walk over rows (head, 128-query block); a workgroup = 4 wave64s x 32
 // queries, two waves per SIMD; K/V tiles of 32 keys reach LDS by direct buffer->LDS copies into 4-slot rings;
 // S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16_bf16 so each lane owns one query row; the softmax keeps a fixed
-// reference per row (see the kernel's comment). fp32 (the parity lane): 4 wave64s x 32 queries on
-// v_mfma_f32_32x32x2_f32 with a lazy online-softmax rescale; workgroup ids are remapped so each XCD (own L2) walks a
-// contiguous run of (head, query block) items.
+// reference per row (see the kernel's comment). fp32 (the parity lane): 4 wave64s x 32 queries, every fp32 operand
+// split into three bf16 parts and multiplied on the same matrix instruction, with a lazy online-softmax rescale. In
+// both, calls with few rows split the rows' key lists into pieces that a second kernel merges.
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
@@ -30,6 +30,7 @@ __device__ __forceinline__ float pair_sum(float x) {
 
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) char lds_char;
 
 
@@ -162,6 +163,100 @@ __device__ __forceinline__ int next_dealt_item(int32_t* counters, int rows) {
   return rows;
 }
 
+// The next item of this workgroup. DIRECT (every item has a workgroup of its own): one item, the XCD-remapped workgroup
+// index. Else the row at its position of the order's first wave, then of its XCD's queue. Called by the whole workgroup;
+// false when nothing is left.
+template <bool DIRECT>
+__device__ __forceinline__ bool next_item(const int32_t* __restrict__ order, int32_t* __restrict__ counter, int rows,
+                                          bool first, int tid, int* item_s, int& item) {
+  if constexpr (DIRECT) {
+    item = xcd_remap(blockIdx.x, gridDim.x);
+    return first;
+  }
+  int p = blockIdx.x;
+  if (!first) {
+    if (tid == 0) *item_s = next_dealt_item(counter, rows);
+    __syncthreads();
+    p = *item_s;
+    __syncthreads();
+  }
+  if (p >= rows) return false;
+  item = order[p];
+  return true;
+}
+
+// An item: a row (head-major, 128 queries), or with a.pieces > 1 (DIRECT only) piece `item / rows` of row
+// `item % rows`: entries [b0, b0 + nblocks) of the row's list. Neighbouring items are neighbouring rows' same pieces,
+// whose key blocks overlap.
+struct AttnItem {
+  int row, h, qb, b0, nblocks;
+};
+template <bool DIRECT>
+__device__ __forceinline__ AttnItem attn_item(const AttnArgs& a, const int32_t* __restrict__ kcnt, int rows, int item) {
+  AttnItem it;
+  const int piece = DIRECT ? item / rows : 0;
+  it.row = item - piece * rows;
+  it.h = it.row / a.nq;
+  it.qb = it.row - it.h * a.nq;
+  const int n = max(0, min(kcnt[it.row], a.nk_stride));
+  it.b0 = DIRECT ? (int)((int64_t)n * piece / a.pieces) : 0;
+  it.nblocks = (DIRECT ? (int)((int64_t)n * (piece + 1) / a.pieces) : n) - it.b0;
+  return it;
+}
+
+// An item that lists no block: an unsplit row is zeros (SparseAttention.swift:47-53; DiT.swift:300-304), a piece is a
+// partial result of weight 0.
+template <bool DIRECT, typename T>
+__device__ __forceinline__ void attn_empty_item(const AttnArgs& a, const AttnItem& it, int item, T* __restrict__ O,
+                                                int tid, int threads) {
+  constexpr int VN = 16 / sizeof(T), kVecs = kHeadDim / VN;
+  if (DIRECT && a.pieces > 1) {
+    if (tid < kBlock) a.part_ml[(int64_t)item * 2 * kBlock + kBlock + tid] = 0.f;
+    return;
+  }
+  for (int e = tid; e < kBlock * kVecs; e += threads) {
+    const int64_t row = (int64_t)it.qb * kBlock + e / kVecs;
+    if (row < a.lq) *(u32x4*)(O + a.out_row(row) * a.ld + it.h * kHeadDim + (e % kVecs) * VN) = u32x4{0, 0, 0, 0};
+  }
+}
+
+// The result of 32 queries (group `group` of the item's four; lane l holds query l % 32, dims 32 dt + 8 r4 + 4 (l / 32) + e
+// at acc[dt][4 r4 + e]) from the unnormalised accumulator, the softmax sum l and the reference m (log2 units): the output
+// row, or the piece's partial result in register order (1 KB per store instruction).
+template <bool DIRECT, typename T>
+__device__ __forceinline__ void attn_store(const AttnArgs& a, const AttnItem& it, int item, int group,
+                                           const f32x16 (&acc)[4], float m, float l, T* __restrict__ O) {
+  typedef T Tx4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
+  if (DIRECT && a.pieces > 1) {
+    float* const po = a.part_o + ((int64_t)item * 4 + group) * (32 * kHeadDim) + 4 * lane;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[i >> 2][4 * (i & 3) + e];
+      *(f32x4*)(po + i * 256) = v;
+    }
+    if (g == 0) {
+      float* const ml = a.part_ml + (int64_t)item * 2 * kBlock + group * 32 + l32;
+      ml[0] = m;
+      ml[kBlock] = l;
+    }
+    return;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int64_t qrow = (int64_t)it.qb * kBlock + group * 32 + l32;
+  if (qrow >= a.lq) return;
+  T* const orow = O + a.out_row(qrow) * a.ld + it.h * kHeadDim;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    Tx4 ov;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[i >> 2][4 * (i & 3) + e] * inv);
+    *(Tx4*)(orow + 8 * i + 4 * g) = ov;
+  }
+}
+
 // LDS operand requests of chunk / pair j >= 2 (j = 0, 1: micro-round 0), in micro-rounds of a step with QG query
 // groups per wave: 7 (QG 2) or 4 (QG 1) micro-rounds before the QK MFMA that uses them, micro-round 0 at the earliest
 template <int QG>
@@ -170,7 +265,7 @@ constexpr int attn_read_at(int j) {
   return r > 0 ? r : 0;
 }
 
-template <int QG>
+template <int QG, bool DIRECT>
 __global__ __attribute__((amdgpu_flat_work_group_size(256 / QG, 256 / QG), amdgpu_waves_per_eu(3 - QG, 3 - QG)))
 void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
                       const bf16* __restrict__ Q, bf16* __restrict__ O,
@@ -185,39 +280,23 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
   const int rows = a.heads * a.nq;
-  // Persistent: the grid is sized to the resident workgroups. attn_order_kernel sorts the rows longest key list
+  // With more rows than resident workgroups the walk is persistent. attn_order_kernel sorts the rows longest key list
   // first and deals every wave of gridDim.x of them by XCD (re-sorted by row id, XCD x holds positions x, x + 8, ..
   // of the wave: one contiguous row range, whose key lists overlap). Workgroup b starts on position b of the first
   // wave; after that it takes the next position of its XCD's queue (positions x, x + 8, .. of the first wave, then
   // of the second, ...) and, once that queue is empty, of the other XCDs' queues in turn. So the long rows start
   // early, the rows running together on one XCD share key blocks in its L2, and the short ones balance the tail.
-  bool first_item = true;
-  for (;;) {
+  for (bool first = true;; first = false) {
   int item;
-  if (first_item) {
-    item = blockIdx.x;
-    first_item = false;
-  } else {
-    if (tid == 0) item_s = next_dealt_item(counter, rows);
-    __syncthreads();
-    item = item_s;
-    __syncthreads();
-  }
-  if (item >= rows) break;
-  const int row_id = order[item];
-  const int h = row_id / a.nq, qb = row_id - h * a.nq;
-  const int hc = h * kHeadDim;
-  const int cnt = kcnt[row_id];
-
-  if (cnt <= 0) {   // empty query block -> zeros (SparseAttention.swift:47-53; DiT.swift:300-304)
-    for (int e = tid; e < kBlock * 16; e += kThreads) {
-      const int64_t row = (int64_t)qb * kBlock + (e >> 4);
-      if (row < a.lq) *(u32x4*)(O + a.out_row(row) * a.ld + hc + (e & 15) * 8) = u32x4{0, 0, 0, 0};
-    }
+  if (!next_item<DIRECT>(order, counter, rows, first, tid, &item_s, item)) break;
+  const AttnItem it = attn_item<DIRECT>(a, kcnt, rows, item);
+  if (it.nblocks <= 0) {
+    attn_empty_item<DIRECT, bf16>(a, it, item, O, tid, kThreads);
     continue;
   }
-  const int32_t* __restrict__ klist = kidx + (int64_t)row_id * a.nk_stride;
-  const int nblocks = min(cnt, a.nk_stride);
+  const int h = it.h, qb = it.qb, nblocks = it.nblocks;
+  const int hc = h * kHeadDim;
+  const int32_t* __restrict__ klist = kidx + (int64_t)it.row * a.nk_stride + it.b0;
 
   // Q as the B operand of S^T = K Q^T (the bf16 inputs as they are; the scale c is applied to the fp32 scores):
   // group q holds queries qb*128 + kQW*wave + 32*q + l32, lane (query, k-half g) dims 16t + 8g .. +7
@@ -629,24 +708,8 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
   }
 
 #pragma unroll
-  for (int q = 0; q < QG; ++q) {
-    const float l = pair_sum(l_run[q]);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int64_t qrow = (int64_t)qb * kBlock + wave * kQW + q * 32 + l32;
-    if (qrow < a.lq) {
-      bf16* orow = O + a.out_row(qrow) * a.ld + hc;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          bf16x4 ov;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ov[e] = (bf16)(acc[q][dt][4 * r4 + e] * inv);
-          *(bf16x4*)(orow + 32 * dt + 8 * r4 + 4 * g) = ov;
-        }
-    }
-  }
-  }   // next row
+  for (int q = 0; q < QG; ++q) attn_store<DIRECT, bf16>(a, it, item, wave * QG + q, acc[q], m_ref[q], pair_sum(l_run[q]), O);
+  }   // next item
 }
 
 // Rows (head, query block) for the persistent bf16 walk, and the per-XCD queue counters. One workgroup. First a
@@ -837,153 +900,353 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 // ------------------------------------------------------------------------------------------------------------
 // fp32 (parity lane)
 // ------------------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
-  constexpr int BK = 32;          // keys per tile
-  constexpr int LDR = 132;        // padded fp32 row stride (floats): conflict-free operand reads
-  constexpr int TILE = BK * LDR;  // floats per tile
-  __shared__ __attribute__((aligned(16))) float smem[2 * 2 * TILE];
+// The products run on the bf16 matrix cores: every fp32 operand is the exact sum of three bf16 parts (24 significand
+// bits = 8 + 8 + 8, each part the rounded remainder of the ones before it), and a product takes the six partial
+// products above 2^-24 of it, hi*lo and lo*hi and mid*mid first, hi*hi last, accumulated in fp32. The three left out
+// (mid*lo, lo*mid, lo*lo) are at most 2^-23 of the product and lie below the rounding of the fp32 sum. Six k = 16
+// products cost 192 matrix-core cycles per 32 x 32 x 16 block of products, against 512 for the eight k = 2 fp32 ones.
+//
+// A workgroup = 4 wave64s x 32 queries, two per CU (48 KB of tile LDS, at most 256 registers a wave), so that one
+// workgroup's staging, softmax and waits run under the other's products. Keys stream in tiles of 32: a tile's fp32
+// rows are loaded into registers half a step ahead (raw buffer loads, rows past the buffer read 0), split once per
+// workgroup and stored as three bf16 planes with the 16-byte chunk swizzles of the bf16 walk. K and V planes each have
+// one buffer: K(T+1) is stored while PV(T) runs, V(T+1) while QK(T+1) runs, with one barrier after each product.
+// S^T = K Q^T leaves each lane one query's scores; the lazy online softmax is in fp32, and P is split in registers.
+//
+// The split cannot hold values past the largest bf16 (3.39e38, infinities), and the parts of values near the smallest
+// normal number are lost: a workgroup that met the one, or a thread that saw only such V, redoes its item on the fp32
+// matrix cores (f32_exact_walk). NaNs propagate through the parts.
+//
+// Bound by the matrix cores (58 % busy) with the split's and the softmax's VALU work and the two barriers a tile.
+// 504 rows x 32 blocks: 705 us, 192 TFLOP/s of fp32 products, past the 157 of the fp32 matrix instructions, on which the
+// former kernel reached 90 to 120; 512 x 512 two-chunk clip 2813 -> 1528 us. Its error against 64 bits is the smaller one:
+// 1.4e-6 against 1.9e-6 on that clip, 5.3e-7 against 8.1e-7 on a sparse 512 x 512 layer.
+constexpr int kF32Plane = kTileBytes;              // one bf16 plane of a 32-key tile
+constexpr float kSplitMax = 3.3895314e38f;         // the largest finite bf16
+constexpr float kSplitMin = 1.2621775e-29f;        // 2^-96: the parts of smaller values near the normal range's end
+constexpr int kExactLd = 132;                      // padded fp32 row of the exact walk's tiles (floats)
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = lid / a.nq, qb = lid - h * a.nq;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int g = lane >> 5, l32 = lane & 31;
-  const int hc = h * kHeadDim;
-  const float* __restrict__ Q = (const float*)a.q;
-  const float* __restrict__ K = (const float*)a.k;
-  const float* __restrict__ V = (const float*)a.v;
-  float* __restrict__ O = (float*)a.o;
-  const int row_id = h * a.nq + qb;
-  const int cnt = a.kcnt[row_id];
+// two values as their packed parts h + m + l
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  auto pack = [](float x, float y) -> unsigned {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
+  };
+  auto lo = [](unsigned u) { return __uint_as_float(u << 16); };
+  auto hi = [](unsigned u) { return __uint_as_float(u & 0xffff0000u); };
+  h = pack(a, b);
+  const float ra = a - lo(h), rb = b - hi(h);
+  m = pack(ra, rb);
+  l = pack(ra - lo(m), rb - hi(m));
+}
 
-  if (cnt <= 0) {
-    for (int e = tid; e < kBlock * 32; e += 256) {
-      const int64_t row = (int64_t)qb * kBlock + (e >> 5);
-      if (row < a.lq) *(f32x4*)(O + a.out_row(row) * a.ld + hc + (e & 31) * 4) = f32x4{0, 0, 0, 0};
-    }
-    return;
+struct Planes8 {   // eight values as three bf16 parts
+  u32x4 h, m, l;
+};
+__device__ __forceinline__ Planes8 split8(const f32x4& x, const f32x4& y, float& mag) {
+  Planes8 p;
+  unsigned h, m, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = i < 2 ? x[2 * i] : y[2 * i - 4], b = i < 2 ? x[2 * i + 1] : y[2 * i - 3];
+    split_pair(a, b, h, m, l);
+    p.h[i] = h;
+    p.m[i] = m;
+    p.l[i] = l;
+    mag = fmaxf(mag, fmaxf(fabsf(a), fabsf(b)));
   }
-  const int32_t* __restrict__ klist = a.kidx + (int64_t)row_id * a.nk_stride;
-  const int nblocks = min(cnt, a.nk_stride);
-  const int ntiles = nblocks * (kBlock / BK);
-  auto valid_keys = [&](int j, int part) -> int64_t {
-    return (unsigned)j < (unsigned)a.nk ? a.lk - ((int64_t)j * kBlock + part * BK) : 0;
-  };
+  return p;
+}
 
-  // Q as the B operand of 32x32x2 steps: step (a, b) pairs dim 8a + 4g + b with k-index g
-  const int64_t qrow = (int64_t)qb * kBlock + wave * 32 + l32;
-  f32x4 qf[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (qrow < a.lq) qf[i] = *(const f32x4*)(Q + qrow * a.ld + hc + 8 * i + 4 * g);
-    else qf[i] = f32x4{0, 0, 0, 0};
-  }
+// The six partial products of one k = 16 step, smallest first.
+__device__ __forceinline__ void mfma_split(f32x16& acc, const bf16x8& ah, const bf16x8& am, const bf16x8& al,
+                                           const bf16x8& bh, const bf16x8& bm, const bf16x8& bl) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bm, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bh, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bm, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc, 0, 0, 0);
+}
 
-  f32x4 kreg[4], vreg[4];
-  const int ld_row = tid >> 5, ld_c4 = tid & 31;
-  auto load_tile = [&](int T) {
-    const int jj = T >> 2, part = T & 3;
-    const int j = klist[jj];
-    const int64_t valid = valid_keys(j, part);
-    const int64_t row0 = valid > 0 ? a.map.row(j) + part * BK : 0;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int r = p * 8 + ld_row;
-      if (r < valid) {
-        const int64_t off = (row0 + r) * a.kv_ld + h * a.kv_head_stride + ld_c4 * 4;
-        kreg[p] = *(const f32x4*)(K + off);
-        vreg[p] = *(const f32x4*)(V + off);
-      } else {
-        kreg[p] = f32x4{0, 0, 0, 0};
-        vreg[p] = f32x4{0, 0, 0, 0};
-      }
-    }
-  };
-  auto store_tile = [&](int st) {
-    float* ks = smem + st * 2 * TILE;
-    float* vs = ks + TILE;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int r = p * 8 + ld_row;
-      *(f32x4*)(ks + r * LDR + ld_c4 * 4) = kreg[p];
-      *(f32x4*)(vs + r * LDR + ld_c4 * 4) = vreg[p];
-    }
-  };
-
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-
-  f32x16 acc_o[4];
+// One item on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), for operands the split cannot hold. Every wave of the
+// workgroup calls it together; smem holds 2 x 32 x kExactLd floats. Same lazy softmax and output layout as the kernel.
+__device__ __forceinline__ void f32_exact_walk(const AttnArgs& a, int h, int64_t qrow,
+                                                         const int32_t* __restrict__ klist, int nblocks, float* smem,
+                                                         f32x16 (&acc_o)[4], float& m_run, float& l_run) {
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const float* __restrict__ Q = (const float*)a.q + h * kHeadDim;
+  const float* __restrict__ K = (const float*)a.k + h * a.kv_head_stride;
+  const float* __restrict__ V = (const float*)a.v + h * a.kv_head_stride;
+  float* const ks = smem;
+  float* const vs = smem + kTileKeys * kExactLd;
+  m_run = -INFINITY;
+  l_run = 0.f;
 #pragma unroll
   for (int d = 0; d < 4; ++d) acc_o[d] = f32x16{};
-  float m_run = -INFINITY, l_run = 0.f;
-  const float c = a.c;
-
-  for (int T = 0; T < ntiles; ++T) {
-    const int st = T & 1;
-    const bool has_next = T + 1 < ntiles;
-    if (has_next) load_tile(T + 1);
-    const float* ks = smem + st * 2 * TILE;
-    const float* vs = ks + TILE;
-
+  for (int T = 0; T < 4 * nblocks; ++T) {
+    const int j = klist[T >> 2], sub = T & 3;
+    const int64_t valid = (unsigned)j < (unsigned)a.nk ? a.lk - ((int64_t)j * kBlock + sub * kTileKeys) : 0;
+    const int64_t row0 = valid > 0 ? a.map.row(j) + sub * kTileKeys : 0;
+    __syncthreads();   // the tile before has been read
+    for (int e = tid; e < kTileKeys * 32; e += 256) {
+      const int r = e >> 5, c4 = (e & 31) * 4;
+      f32x4 kv = f32x4{0, 0, 0, 0}, vv = f32x4{0, 0, 0, 0};
+      if (r < valid) {
+        kv = *(const f32x4*)(K + (row0 + r) * a.kv_ld + c4);
+        vv = *(const f32x4*)(V + (row0 + r) * a.kv_ld + c4);
+      }
+      *(f32x4*)(ks + r * kExactLd + c4) = kv;
+      *(f32x4*)(vs + r * kExactLd + c4) = vv;
+    }
+    __syncthreads();
     f32x16 s = f32x16{};
-#pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const f32x4 kf = *(const f32x4*)(ks + l32 * LDR + 8 * i + 4 * g);
+      const f32x4 kf = *(const f32x4*)(ks + l32 * kExactLd + 8 * i + 4 * g);
+      f32x4 qf = f32x4{0, 0, 0, 0};
+      if (qrow < a.lq) qf = *(const f32x4*)(Q + qrow * a.ld + 8 * i + 4 * g);
 #pragma unroll
-      for (int b = 0; b < 4; ++b) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[b], qf[i][b], s, 0, 0, 0);
+      for (int b = 0; b < 4; ++b) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[b], qf[b], s, 0, 0, 0);
     }
-
-    const int64_t valid = valid_keys(klist[T >> 2], T & 3);
-    if (valid < BK) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + 4 * g + (r & 3) >= valid) s[r] = -INFINITY;
-    }
-
+    for (int r = 0; r < 16; ++r)
+      if (8 * (r >> 2) + 4 * g + (r & 3) >= valid) s[r] = -INFINITY;
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
-    mx = pair_max(mx);
-    const float m_use = rescale_if_grown<4>(mx * c, m_run, l_run, acc_o);
-    float lsum = 0.f;
+    const float m_use = rescale_if_grown<4>(pair_max(mx) * a.c, m_run, l_run, acc_o);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, -m_use));
-      lsum += s[r];
+      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], a.c, -m_use));
+      l_run += s[r];
     }
-    l_run += lsum;
-
-    // O^T += V^T P^T: k-step r pairs key 8(r/4) + 4g + r%4 (this lane's P entry r) with k-index g
+    // k-step r pairs key 8(r/4) + 4g + r%4 (this lane's P entry r) with k-index g
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = 8 * (r >> 2) + 4 * g + (r & 3);
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const float vv = vs[key * LDR + 32 * dt + l32];
-        acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, s[r], acc_o[dt], 0, 0, 0);
-      }
+      for (int dt = 0; dt < 4; ++dt)
+        acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[key * kExactLd + 32 * dt + l32], s[r], acc_o[dt], 0, 0, 0);
     }
-
-    if (has_next) store_tile(st ^ 1);
-    __syncthreads();
   }
+}
 
-  const float l_tot = pair_sum(l_run);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (qrow < a.lq) {
-    float* orow = O + a.out_row(qrow) * a.ld + hc;
+template <bool DIRECT>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
+void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
+                     const float* __restrict__ Q, float* __restrict__ O, const int32_t* __restrict__ order,
+                     int32_t* __restrict__ counter) {
+  __shared__ __attribute__((aligned(1024))) char smem[6 * kF32Plane];   // K planes h, m, l, then V planes h, m, l
+  static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 6 * kF32Plane, "the exact walk's tiles fit");
+  __shared__ int item_s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5, l32 = lane & 31;
+  const int rows = a.heads * a.nq;
+  const uint32_t row_bytes = (uint32_t)a.kv_ld * 4;
+  const uint32_t range = (uint32_t)a.kv_bytes;
+  __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void*)a.k, 0, range, 0x00020000);
+  __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.v, 0, range, 0x00020000);
+  // staging: this thread loads 8 floats of rows r_ld and r_ld + 16 of a tile, one 16-byte chunk of each plane
+  const int r_ld = tid >> 4, c_ld = tid & 15;
+  const int st_k[2] = {r_ld * kRowBytes + ((c_ld ^ swz_k(r_ld)) << 4),
+                       (r_ld + 16) * kRowBytes + ((c_ld ^ swz_k(r_ld + 16)) << 4)};
+  const int st_v[2] = {r_ld * kRowBytes + ((c_ld ^ swz_v(r_ld)) << 4),
+                       (r_ld + 16) * kRowBytes + ((c_ld ^ swz_v(r_ld + 16)) << 4)};
+  // operand reads, as in the bf16 walk
+  const int kb = l32 * kRowBytes, kx = swz_k(l32);
+  const int G = lane >> 4, mm = lane & 15, vr = 4 * (G >> 1) + (mm >> 2);
+  int v_off[4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < 4; ++dt)
+    v_off[dt] = vr * kRowBytes + (((4 * dt + 2 * (G & 1) + ((mm & 3) >> 1)) ^ swz_v(vr)) << 4) + (mm & 1) * 8;
+  lds_char* const lds = (lds_char*)(uintptr_t)lds_addr(smem);
+  lds_char* const ldsv = lds + 3 * kF32Plane;
+
+  for (bool first = true;; first = false) {
+    int item;
+    if (!next_item<DIRECT>(order, counter, rows, first, tid, &item_s, item)) break;
+    const AttnItem it = attn_item<DIRECT>(a, kcnt, rows, item);
+    if (it.nblocks <= 0) {
+      attn_empty_item<DIRECT, float>(a, it, item, O, tid, 256);
+      continue;
+    }
+    const int32_t* __restrict__ klist = kidx + (int64_t)it.row * a.nk_stride + it.b0;
+    const int nblocks = it.nblocks;
+    const int64_t qrow = (int64_t)it.qb * kBlock + wave * 32 + l32;
+    float mag = 0.f, mag_v = 0.f;   // largest magnitude this thread split: Q and K, V
+    bf16x8 qh[8], qm[8], ql[8];
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        f32x4 ov;
-        ov[0] = acc_o[dt][4 * r4 + 0] * inv;
-        ov[1] = acc_o[dt][4 * r4 + 1] * inv;
-        ov[2] = acc_o[dt][4 * r4 + 2] * inv;
-        ov[3] = acc_o[dt][4 * r4 + 3] * inv;
-        *(f32x4*)(orow + 32 * dt + 8 * r4 + 4 * g) = ov;
+    for (int t = 0; t < 8; ++t) {
+      f32x4 x = f32x4{0, 0, 0, 0}, y = f32x4{0, 0, 0, 0};
+      if (qrow < a.lq) {
+        const float* p = Q + qrow * a.ld + it.h * kHeadDim + 16 * t + 8 * g;
+        x = *(const f32x4*)p;
+        y = *(const f32x4*)(p + 4);
       }
+      const Planes8 p = split8(x, y, mag);
+      qh[t] = __builtin_bit_cast(bf16x8, p.h);
+      qm[t] = __builtin_bit_cast(bf16x8, p.m);
+      ql[t] = __builtin_bit_cast(bf16x8, p.l);
+    }
+    const uint32_t ld_off = r_ld * row_bytes + (uint32_t)(it.h * a.kv_head_stride * 4) + c_ld * 32;
+    // tile T = quarter T % 4 of the T / 4-th listed block: byte offset of its first row (past the buffer for a block
+    // outside [0, nk) and past the walk's end) and its keys taking part
+    auto tile_off = [&](int T) -> uint32_t {
+      if ((T >> 2) >= nblocks) return range;
+      const int j = klist[T >> 2];
+      return (unsigned)j < (unsigned)a.nk ? (uint32_t)(a.map.row(j) + (T & 3) * kTileKeys) * row_bytes : range;
+    };
+    auto tile_valid = [&](int T) -> int {
+      const int j = klist[T >> 2];
+      if ((unsigned)j >= (unsigned)a.nk) return 0;
+      return (int)min<int64_t>(kTileKeys, a.lk - ((int64_t)j * kBlock + (T & 3) * kTileKeys));
+    };
+    f32x4 raw[4];
+    auto load_raw = [&](__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+      const uint32_t o0 = ld_off + off, o1 = o0 + 16 * row_bytes;   // < 2^31 + 2^18: no wrap
+      raw[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0, 0, 0));
+      raw[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0 + 16, 0, 0));
+      raw[2] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1, 0, 0));
+      raw[3] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1 + 16, 0, 0));
+    };
+    auto store_planes = [&](lds_char* base, const int (&at)[2], float& largest) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const Planes8 p = split8(raw[2 * i], raw[2 * i + 1], largest);
+        *(lds_u32x4*)(base + at[i]) = p.h;
+        *(lds_u32x4*)(base + kF32Plane + at[i]) = p.m;
+        *(lds_u32x4*)(base + 2 * kF32Plane + at[i]) = p.l;
+      }
+    };
+    f32x16 acc[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) acc[d] = f32x16{};
+    float m_run = -INFINITY, l_run = 0.f;
+    const int ntiles = 4 * nblocks;
+
+    load_raw(krs, tile_off(0));
+    store_planes(lds, st_k, mag);
+    load_raw(vrs, tile_off(0));
+    __syncthreads();   // K(0) stored
+    for (int T = 0; T < ntiles; ++T) {
+      // V(T) goes to LDS (PV(T-1) is done) while this tile's scores are formed; then K(T+1) is requested
+      store_planes(ldsv, st_v, mag_v);
+      const uint32_t off_next = tile_off(T + 1);
+      load_raw(krs, off_next);
+      f32x16 s = f32x16{};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        lds_char* const p = lds + kb + (((2 * t + g) ^ kx) << 4);
+        const bf16x8 kh = *(const lds_bf16x8*)p, km = *(const lds_bf16x8*)(p + kF32Plane);
+        const bf16x8 kl = *(const lds_bf16x8*)(p + 2 * kF32Plane);
+        mfma_split(s, kh, km, kl, qh[t], qm[t], ql[t]);
+      }
+      __syncthreads();   // K(T) has been read, V(T) is stored
+      store_planes(lds, st_k, mag);
+      load_raw(vrs, off_next);
+      const int valid = tile_valid(T);
+      if (valid < kTileKeys) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + 4 * g + (r & 3) >= valid) s[r] = -INFINITY;
+      }
+      float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+      for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      const float m_use = rescale_if_grown<4>(pair_max(mx) * a.c, m_run, l_run, acc);
+      float sum[2] = {0.f, 0.f};
+      bf16x8 ph[2], pm[2], pl[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        u32x4 wh, wm, wl;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i], a.c, -m_use));
+          const float y = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i + 1], a.c, -m_use));
+          sum[0] += x;
+          sum[1] += y;
+          unsigned h, m, l;
+          split_pair(x, y, h, m, l);
+          wh[i] = h;
+          wm[i] = m;
+          wl[i] = l;
+        }
+        ph[u] = __builtin_bit_cast(bf16x8, wh);
+        pm[u] = __builtin_bit_cast(bf16x8, wm);
+        pl[u] = __builtin_bit_cast(bf16x8, wl);
+      }
+      l_run += sum[0] + sum[1];
+      // O^T += V^T P^T
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          bf16x8 vv[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) {
+            lds_char* const pa = ldsv + p * kF32Plane + v_off[dt] + 16 * u * kRowBytes;
+            const i16x4 va = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)pa);
+            const i16x4 vb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + 8 * kRowBytes));
+            vv[p] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+          mfma_split(acc[dt], vv[0], vv[1], vv[2], ph[u], pm[u], pl[u]);
+        }
+      __syncthreads();   // V(T) has been read, K(T+1) is stored
+    }
+    if (__syncthreads_or(!(fmaxf(mag, mag_v) <= kSplitMax) || (mag_v > 0.f && mag_v < kSplitMin)))
+      f32_exact_walk(a, it.h, qrow, klist, nblocks, (float*)smem, acc, m_run, l_run);
+    attn_store<DIRECT, float>(a, it, item, wave, acc, m_run == -INFINITY ? 0.f : m_run, pair_sum(l_run), O);
+    __syncthreads();   // smem and item_s are free for the next item
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// merge of split rows
+// ------------------------------------------------------------------------------------------------------------
+// O of a row split into pieces: sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p, M the largest reference of the pieces
+// that listed a block. One workgroup per 32 queries of a row, one wave per 32 dims; reads 64 KB a piece and row in
+// register order, so it runs at the rate the partial results come out of the caches.
+template <typename T>
+__global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, T* __restrict__ O) {
+  typedef T Tx4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31, dt = threadIdx.x >> 6;
+  const int row = blockIdx.x >> 2, group = blockIdx.x & 3;
+  const int rows = a.heads * a.nq;
+  const int h = row / a.nq, qb = row - h * a.nq;
+  const float* const ml = a.part_ml + (int64_t)row * 2 * kBlock + group * 32 + l32;
+  const float* const po = a.part_o + ((int64_t)row * 4 + group) * (32 * kHeadDim) + 1024 * dt + 4 * lane;
+  const int64_t sml = (int64_t)rows * 2 * kBlock, so = (int64_t)rows * kBlock * kHeadDim;   // piece to piece
+  float M = -INFINITY;
+#pragma unroll 4
+  for (int p = 0; p < a.pieces; ++p) {
+    const float m = ml[p * sml];
+    M = fmaxf(M, ml[p * sml + kBlock] != 0.f ? m : -INFINITY);
+  }
+  f32x4 acc[4] = {};
+  float l = 0.f;
+#pragma unroll 4
+  for (int p = 0; p < a.pieces; ++p) {
+    const float lp = ml[p * sml + kBlock], sc = __builtin_amdgcn_exp2f(ml[p * sml] - M);
+    const bool in = lp != 0.f;   // a piece of weight 0 may hold anything
+    l += in ? sc * lp : 0.f;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const f32x4 x = *(const f32x4*)(po + p * so + 256 * r4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[r4][e] += in ? sc * x[e] : 0.f;
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int64_t qrow = (int64_t)qb * kBlock + group * 32 + l32;
+  if (qrow >= a.lq) return;
+  T* const orow = O + a.out_row(qrow) * a.ld + h * kHeadDim + 32 * dt;
+#pragma unroll
+  for (int r4 = 0; r4 < 4; ++r4) {
+    Tx4 ov;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[r4][e] * inv);
+    *(Tx4*)(orow + 8 * r4 + 4 * g) = ov;
   }
 }
 
@@ -1076,42 +1339,83 @@ static int attn_query_groups() {
   return qg;
 }
 
-int launch_attention(int dtype, const AttnArgs& a, hipStream_t stream) {
-  const int nwg = a.heads * a.nq;
-  if (nwg <= 0) return FVSR_OK;
-  dim3 grid(nwg), block(256);
-  if (dtype == FVSR_DTYPE_BF16) {
-    if (!a.order || !a.counter) return set_error(FVSR_ERR_INVALID_ARG, "attention: no workspace for the row order");
-    // two workgroups (64 KB of LDS each) are resident per CU
-    const int pwgs = std::min(nwg, std::min(2 * device_cus(), kMaxPersistentWgs));
-    hipLaunchKernelGGL(attn_order_kernel, dim3(1), dim3(1024), 0, stream, a.kcnt, nwg, a.nk_stride, pwgs, a.order,
+// Pieces per row. Few rows leave workgroup slots idle and make each row's key list one serial chain, so their lists are
+// split; a piece costs 65 KB of partial result written and read again, and the merge a launch. Measured (12 heads unless
+// said; us a call, unsplit against the pieces chosen):
+//   bf16: one workgroup per CU already runs at 70 % of what two reach together, so the split stops at one item per CU, and
+//   at 4 key blocks an item: 48 rows x 16 blocks 34.4 -> 24.3, 72 x 24 47.9 -> 30.8, 8 (2 heads) x 200 179 -> 30; 108 x 19
+//   31.9 -> 28.0; splitting on to two items per CU is slower (72 x 24 in 7: 34.6, 216 x 18 in 2: 43.1 -> 49.1) until an item
+//   holds about 24 blocks (192 x 64 in 2: 81.2 -> 75.8).
+//   fp32: a block costs 3 times as much, so every slot is filled, down to one block an item: 48 x 16 198 -> 60, 72 x 24
+//   294 -> 101, 216 x 18 226 -> 197, 192 x 64 505 -> 361.
+constexpr int kMaxSplitItems = 512;   // the partial results of a call: at most 34 MB
+constexpr int kMaxPieces = 32;        // the merge walks a row's pieces one after another
+static int split_pieces(int dtype, int64_t rows, int nk, int cus, int64_t max_items) {
+  auto fit = [&](int64_t items, int blocks) -> int64_t {   // pieces of at least `blocks` key blocks within `items`
+    return std::min(std::min(items, max_items) / rows, (int64_t)(nk / blocks));
+  };
+  const int64_t n = dtype == FVSR_DTYPE_BF16 ? std::max(fit(cus, 4), fit(2 * cus, 24)) : fit(2 * cus, 1);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(n, kMaxPieces));
+}
+
+// the most items that attentions over up to `rows` rows and nk key blocks split into
+int64_t attn_partial_items(int64_t rows, int nk) {
+  return std::min<int64_t>(kMaxSplitItems, rows * std::min(kMaxPieces, std::max(1, nk)));
+}
+
+int launch_attention(int dtype, AttnArgs a, hipStream_t stream) {
+  const int rows = a.heads * a.nq;
+  if (rows <= 0) return FVSR_OK;
+  const bool half = dtype == FVSR_DTYPE_BF16;
+  // two workgroups are resident per CU (64 KB of LDS each in the bf16 walk, 48 KB in the fp32 one)
+  const int slots = std::min(2 * device_cus(), kMaxPersistentWgs);
+  a.pieces = split_pieces(dtype, rows, a.nk, device_cus(), a.part_items);
+  a.part_ml = a.part_o + (int64_t)rows * a.pieces * kBlock * kHeadDim;
+  const bool direct = rows * a.pieces <= slots || !a.order;   // a workgroup per item
+  const dim3 grid(direct ? rows * a.pieces : slots);
+  if (!direct)
+    hipLaunchKernelGGL(attn_order_kernel, dim3(1), dim3(1024), 0, stream, a.kcnt, rows, a.nk_stride, slots, a.order,
                        a.counter);
-    const dim3 pgrid(pwgs);
-    if (attn_query_groups() == 2)
-      hipLaunchKernelGGL(attn_bf16_kernel<2>, pgrid, dim3(128), 0, stream, a, a.kidx, a.kcnt, (const bf16*)a.q,
-                         (bf16*)a.o, (const int32_t*)a.order, a.counter);
+  auto walk = [&](auto direct_c) {
+    constexpr bool DIRECT = decltype(direct_c)::value;
+    if (!half)
+      hipLaunchKernelGGL(attn_f32_kernel<DIRECT>, grid, dim3(256), 0, stream, a, a.kidx, a.kcnt, (const float*)a.q,
+                         (float*)a.o, (const int32_t*)a.order, a.counter);
+    else if (attn_query_groups() == 2)
+      hipLaunchKernelGGL((attn_bf16_kernel<2, DIRECT>), grid, dim3(128), 0, stream, a, a.kidx, a.kcnt,
+                         (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
     else
-      hipLaunchKernelGGL(attn_bf16_kernel<1>, pgrid, dim3(256), 0, stream, a, a.kidx, a.kcnt, (const bf16*)a.q,
-                         (bf16*)a.o, (const int32_t*)a.order, a.counter);
-  } else {
-    hipLaunchKernelGGL(attn_f32_kernel, grid, block, 0, stream, a);
-  }
+      hipLaunchKernelGGL((attn_bf16_kernel<1, DIRECT>), grid, dim3(256), 0, stream, a, a.kidx, a.kcnt,
+                         (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
+  };
+  if (direct) walk(std::true_type{});
+  else walk(std::false_type{});
   FVSR_HIP_CHECK(hipGetLastError());
+  if (a.pieces > 1) {
+    if (half)
+      hipLaunchKernelGGL(attn_merge_kernel<bf16>, dim3(4 * rows), dim3(256), 0, stream, a, (bf16*)a.o);
+    else
+      hipLaunchKernelGGL(attn_merge_kernel<float>, dim3(4 * rows), dim3(256), 0, stream, a, (float*)a.o);
+    FVSR_HIP_CHECK(hipGetLastError());
+  }
   return FVSR_OK;
 }
 
 // ------------------------------------------------------------------------------------------------------------
 // allocation-free scratch of fvsr_lcsa_attention_noalloc
 // ------------------------------------------------------------------------------------------------------------
-// The persistent walk's row order (one int32 per (head, query block) row) and its work counter live in a file-scope
-// device array instead of the context workspace: bytes [0, 256) hold the counter, the order starts at byte 256.
+// The persistent walk's row order (one int32 per (head, query block) row), its work counter and the partial results of
+// split rows live in a file-scope device array instead of the context workspace: bytes [0, 256) hold the counter, the
+// order starts at byte 256, the partial results follow.
 // Every GPU holds its own copy for the life of the process. In host code `scratch` names a host-side stand-in, so
 // the device address is taken once per device with hipGetSymbolAddress (noalloc_scratch_init, called by
 // fvsr_ctx_create with the device current) and only that address reaches kernels. The order kernel rewrites the
 // counter and every order entry it uses on each call, so nothing needs clearing; calls that overlap on one GPU
 // share the array and race.
 constexpr int kNoAllocRows = 1 << 18;
-constexpr size_t kNoAllocScratchBytes = 256 + (size_t)kNoAllocRows * sizeof(int32_t);
+constexpr size_t kNoAllocOrderBytes = 256 + (size_t)kNoAllocRows * sizeof(int32_t);
+constexpr size_t kNoAllocScratchBytes =
+    kNoAllocOrderBytes + (size_t)kMaxSplitItems * kPartialFloats * sizeof(float);
 static __device__ __align__(256) char scratch[kNoAllocScratchBytes];
 
 static std::mutex g_scratch_mutex;
@@ -1132,9 +1436,12 @@ int noalloc_scratch_init(int device) {
   return FVSR_OK;
 }
 
-// the row order and counter of `device`'s scratch for `rows` rows (FVSR_ERR_STATE before noalloc_scratch_init)
-int noalloc_scratch(int device, int64_t rows, int32_t** order, int32_t** counter) {
-  if (rows > kNoAllocRows)
+// `device`'s scratch as the order, counter and partial results of an attention (FVSR_ERR_STATE before
+// noalloc_scratch_init). Beyond kNoAllocRows rows the order does not fit: the bf16 walk, whose row order balances it,
+// refuses them; the fp32 one runs a workgroup per row.
+int noalloc_scratch(int device, int dtype, AttnArgs& a) {
+  const int64_t rows = (int64_t)a.heads * a.nq;
+  if (rows > kNoAllocRows && dtype == FVSR_DTYPE_BF16)
     return set_error(FVSR_ERR_UNSUPPORTED, "fvsr_lcsa_attention_noalloc: " + std::to_string(rows) +
                                                " (head, query block) rows exceed its static scratch of " +
                                                std::to_string(kNoAllocRows));
@@ -1144,8 +1451,10 @@ int noalloc_scratch(int device, int64_t rows, int32_t** order, int32_t** counter
     p = g_scratch_ptr[device];
   }
   if (!p) return set_error(FVSR_ERR_STATE, "no scratch address for this device: create its context first");
-  *counter = (int32_t*)p;
-  *order = (int32_t*)((char*)p + 256);
+  a.counter = (int32_t*)p;
+  a.order = rows <= kNoAllocRows ? (int32_t*)((char*)p + 256) : nullptr;
+  a.part_o = (float*)((char*)p + kNoAllocOrderBytes);
+  a.part_items = attn_partial_items(rows, a.nk);
   return FVSR_OK;
 }
 

@@ -478,3 +478,69 @@ def test_row_counts_beyond_the_order_kernels_lds(dev, heads, lqb, uniform):
         assert (ov[i, :, h] == 0).all()
     pairs = [(h, i) for h in range(heads) for i in (0, 1, lqb // 2, lqb - 2, lqb - 1)]
     assert _rows_vs_torch(q, k, v, m, heads, o, pairs) <= BF16_REL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,lqb,nkb", [(1, 1, 3), (1, 1, 130), (3, 5, 8), (2, 9, 50), (12, 16, 26), (16, 16, 25),
+                                           (12, 42, 9)])
+def test_split_key_lists(dev, dtype, heads, lqb, nkb):
+    """Rows whose key lists are split over workgroups and merged: one row and 3 or 130 key blocks (the most pieces),
+    rows that leave slots over, 256 rows (the last that fp32 splits) and 504 (unsplit). Lists of every length from empty
+    through fewer blocks than pieces to full, ragged ends on both sides, scores that grow along the list so that the
+    pieces' references lie far apart. Every row against a float64 softmax at the lane's bar, outputs start as NaN."""
+    gen = torch.Generator(device=dev).manual_seed(heads * 10000 + lqb * 100 + nkb)
+    lq, lk = lqb * 128 - 21, nkb * 128 - 53
+    q, k, v = (torch.randn((n, heads * 128), generator=gen, device=dev) for n in (lq, lk, lk))
+    k = k * torch.linspace(0.2, 2.0, lk, device=dev)[:, None]
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    dens = torch.rand((heads, lqb, 1), generator=gen, device=dev)
+    m = (torch.rand((heads, lqb, nkb), generator=gen, device=dev) < dens).float()
+    m[0, 0] = 1.0
+    if lqb > 1:
+        m[0, 1] = 0.0
+        m[-1, -1] = 0.0
+        m[-1, -1, nkb // 2] = 1.0
+    o = torch.full_like(q, float("nan"))
+    fvsr_lcsa.kernel_block_attention(q, k, v, m, heads, out=o)
+    torch.cuda.synchronize()
+    keep = m.bool().repeat_interleave(128, 1)[:, :lq].repeat_interleave(128, 2)[:, :, :lk]
+    bar = BF16_REL if dtype == torch.bfloat16 else FP32_REL
+    for h in range(heads):
+        c = slice(h * 128, (h + 1) * 128)
+        s = (q[:, c].double() @ k[:, c].double().t().contiguous() / 128 ** 0.5).masked_fill(~keep[h], -float("inf"))
+        ref = torch.softmax(s, -1).nan_to_num(0.0) @ v[:, c].double()
+        assert float((o[:, c].double() - ref).abs().max() / ref.abs().max()) <= bar, h
+
+
+@pytest.mark.parametrize("heads,lqb", [(2, 2), (8, 66)])
+def test_fp32_values_outside_the_split(dev, heads, lqb):
+    """fp32 operands that three bf16 parts cannot hold: an infinite V column stays infinite and leaves the others alone,
+    a NaN stays in its column, a -inf K row is masked out for the queries that score it -inf, and V near the smallest
+    normal number keeps its precision (split rows and one row per workgroup, 4 and 528 rows)."""
+    gen = torch.Generator(device=dev).manual_seed(heads)
+    lq, lk = lqb * 128, 512
+    q, k, v = (torch.randn((n, heads * 128), generator=gen, device=dev) for n in (lq, lk, lk))
+    m = torch.ones((heads, lqb, 4), device=dev)
+
+    def ref(q, k, v, h):
+        c = slice(h * 128, (h + 1) * 128)
+        s = q[:, c].double() @ k[:, c].double().t().contiguous() / 128 ** 0.5
+        return torch.softmax(s, -1) @ v[:, c].double()
+
+    v2 = v.clone()
+    v2[100, 5], v2[300, 200] = float("inf"), float("nan")
+    o = fvsr_lcsa.kernel_block_attention(q, k, v2, m, heads)
+    assert bool((o[:, 5] == float("inf")).all()) and bool(o[:, 200].isnan().all())
+    keep = [i for i in range(heads * 128) if i not in (5, 200)]
+    assert not o[:, keep].isnan().any() and not o[:, keep].isinf().any()
+    assert _rel(o[:, 6:128], ref(q, k, v, 0)[:, 6:].cpu().numpy()) <= FP32_REL
+
+    q2, k2 = q.clone(), k.clone()
+    q2[:, 0] = q2[:, 0].abs() + 0.5
+    k2[77, 0] = -float("inf")                  # scores -inf for every query of head 0: no weight
+    o = fvsr_lcsa.kernel_block_attention(q2, k2, v, m, heads)
+    assert _rel(o[:, :128], ref(q2, k2, v, 0).cpu().numpy()) <= FP32_REL
+
+    o = fvsr_lcsa.kernel_block_attention(q, k, v * 1e-36, m, heads)
+    r = ref(q, k, v * 1e-36, 1)
+    assert float((o[:, 128:256].double() - r).abs().max() / r.abs().max()) <= FP32_REL
