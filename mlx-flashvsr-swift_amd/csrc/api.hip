@@ -38,7 +38,6 @@ int launch_qkv_epilogue(int dtype, const void* q, const void* k, const void* v, 
                         void* v_out, int dst_slot0, int capacity, int slice_blocks, int64_t kv_head_stride,
                         hipStream_t stream);
 int launch_pool_mean(int dtype, PoolMean* jobs, int n, int C, unsigned* zero, int64_t nzero, hipStream_t stream);
-int launch_pool_finish(const PoolDst* dst, int n, int C, unsigned* zero, int64_t nzero, hipStream_t stream);
 int rope_table_floats();
 int blas_create(int device, void** out);
 void blas_destroy(void* p);
@@ -54,7 +53,7 @@ int noalloc_scratch(int device, int dtype, AttnArgs& a);
 void rope_tables_host(double theta, float* out);
 int launch_ring_append(int dtype, const void* k_new, const void* v_new, int n_blocks, int C, bool grid_layout,
                        int nbh, int nbw, int slot0, int capacity, void* ring_k, void* ring_v, int64_t head_stride,
-                       float* pooled, float* partial, hipStream_t stream);
+                       hipStream_t stream);
 int launch_ring_read(int dtype, const void* rk, const void* rv, void* ok, void* ov, int n_blocks, int C,
                      int64_t head_stride, KeyMap map, hipStream_t stream);
 int launch_window_layout(int dtype, const void* x, void* out, int f, int h, int w, int C, bool to_windows,
@@ -111,7 +110,6 @@ struct fvsr_kv_ring {
   void* k = nullptr;
   void* v = nullptr;
   float* pooled = nullptr;   // (layers, capacity * s, C)
-  float* partial = nullptr;  // (capacity * s * kPoolParts, C): pooled-key runs of one append
   size_t layer_tokens() const { return (size_t)capacity * s * kBlock; }
   char* layer_k(int l) const { return (char*)k + (size_t)l * layer_tokens() * C * esize(dtype); }
   char* layer_v(int l) const { return (char*)v + (size_t)l * layer_tokens() * C * esize(dtype); }
@@ -479,14 +477,11 @@ int fvsr_kv_ring_create(fvsr_ctx* ctx, int dtype, int layers, int heads, int bh,
     return set_error(FVSR_ERR_UNSUPPORTED, "a ring layer above 2 GiB is not supported (32-bit buffer offsets)");
   }
   const size_t pooled_bytes = (size_t)layers * capacity_slices * r->s * r->C * sizeof(float);
-  const size_t partial_bytes = (size_t)capacity_slices * r->s * kPoolParts * r->C * sizeof(float);
   if (hipSetDevice(ctx->device) != hipSuccess || hipMalloc(&r->k, kv_bytes) != hipSuccess ||
-      hipMalloc(&r->v, kv_bytes) != hipSuccess || hipMalloc((void**)&r->pooled, pooled_bytes) != hipSuccess ||
-      hipMalloc((void**)&r->partial, partial_bytes) != hipSuccess) {
+      hipMalloc(&r->v, kv_bytes) != hipSuccess || hipMalloc((void**)&r->pooled, pooled_bytes) != hipSuccess) {
     if (r->k) (void)hipFree(r->k);
     if (r->v) (void)hipFree(r->v);
     if (r->pooled) (void)hipFree(r->pooled);
-    if (r->partial) (void)hipFree(r->partial);
     delete r;
     return set_error(FVSR_ERR_OUT_OF_MEMORY, "ring allocation of 2 x " + std::to_string(kv_bytes) + " bytes failed");
   }
@@ -500,7 +495,6 @@ int fvsr_kv_ring_destroy(fvsr_kv_ring* r) {
   (void)hipFree(r->k);
   (void)hipFree(r->v);
   (void)hipFree(r->pooled);
-  (void)hipFree(r->partial);
   delete r;
   return FVSR_OK;
 }
@@ -530,8 +524,30 @@ static int check_layer(const fvsr_kv_ring* r, int layer) {
   return FVSR_OK;
 }
 
-int fvsr_kv_ring_append(fvsr_kv_ring* r, int layer, const void* k_new, const void* v_new, int n_slices, int layout,
-                        void* stream) {
+}  // extern "C"
+
+// Block means of the n_slices slices just written from slot0 on, as for plain buffers: over the slots up to the end of
+// the ring, then the wrapped remainder from slot 0, one launch. With q_pooled set (a layer call) the means of the queries
+// q (lq tokens, window order) and the selection histogram's reset (`hist`, nhist words) ride along. A slot's first token in
+// head 0's region of the (head-major) ring is s * 128 rows of 128 elements past the previous slot's.
+static int pool_new_slices(fvsr_kv_ring* r, int layer, int slot0, int n_slices, const void* q, int64_t lq,
+                           float* q_pooled, unsigned* hist, int64_t nhist, hipStream_t stream) {
+  const int first = std::min(n_slices, r->capacity - slot0);
+  const size_t slot_bytes = (size_t)r->s * kBlock * kHeadDim * esize(r->dtype);
+  PoolMean jobs[3];
+  int nj = 0;
+  jobs[nj++] = PoolMean{r->layer_k(layer) + slot0 * slot_bytes, (int64_t)first * r->s * kBlock,
+                        r->layer_pooled(layer), 0, slot0, r->capacity, r->s, r->head_stride()};
+  if (first < n_slices)
+    jobs[nj++] = PoolMean{r->layer_k(layer), (int64_t)(n_slices - first) * r->s * kBlock, r->layer_pooled(layer), 0,
+                          0, r->capacity, r->s, r->head_stride()};
+  if (q_pooled) jobs[nj++] = PoolMean{q, lq, q_pooled, 0, 0, 1, 1 << 30, 0};
+  return launch_pool_mean(r->dtype, jobs, nj, r->C, hist, nhist, stream);
+}
+
+static int append_impl(fvsr_kv_ring* r, int layer, const void* k_new, const void* v_new, int n_slices, int layout,
+                       hipStream_t stream, const void* q = nullptr, int64_t lq = 0, float* q_pooled = nullptr,
+                       unsigned* hist = nullptr, int64_t nhist = 0) {
   int rc = check_layer(r, layer);
   if (rc) return rc;
   FVSR_REQUIRE(k_new && v_new, FVSR_ERR_INVALID_ARG, "k_new and v_new must be non-NULL");
@@ -543,14 +559,12 @@ int fvsr_kv_ring_append(fvsr_kv_ring* r, int layer, const void* k_new, const voi
   FVSR_HIP_CHECK(hipSetDevice(r->ctx->device));
   const int slot0 = (r->head[layer] + r->count[layer]) % r->capacity;
   rc = launch_ring_append(r->dtype, k_new, v_new, n_slices * r->s, r->C, layout == FVSR_LAYOUT_GRID, r->bh, r->bw,
-                          slot0, r->capacity, r->layer_k(layer), r->layer_v(layer), r->head_stride(),
-                          r->layer_pooled(layer), r->partial, (hipStream_t)stream);
+                          slot0, r->capacity, r->layer_k(layer), r->layer_v(layer), r->head_stride(), stream);
   if (rc) return rc;
+  if ((rc = pool_new_slices(r, layer, slot0, n_slices, q, lq, q_pooled, hist, nhist, stream))) return rc;
   r->count[layer] += n_slices;
   return FVSR_OK;
 }
-
-}  // extern "C"
 
 // The ring append of fvsr_kv_ring_append_qkv. With q_pooled set (the layer call), the block means of the written
 // queries ride in the same pooling launch as the new keys' (to q_pooled), which also clears the selection
@@ -576,26 +590,18 @@ static int append_qkv_impl(fvsr_kv_ring* r, int layer, const void* q, const void
                            norm_k_weight, eps, rope_tables, q_out, r->layer_k(layer), r->layer_v(layer), slot0,
                            r->capacity, r->s, r->head_stride(), stream);
   if (rc) return rc;
-  // pooled keys of the new slots, as for plain buffers: block means over the slots up to the end of the ring, then
-  // the wrapped remainder from slot 0 (and the queries' means, and the histogram reset), one launch; a slot's first
-  // token in head 0's region of the (head-major) ring is s * 128 rows of 128 elements past the previous slot's
-  const int first = std::min(n_slices, r->capacity - slot0);
-  const size_t slot_bytes = (size_t)r->s * kBlock * kHeadDim * esize(r->dtype);
-  const int64_t lq = (int64_t)nb * kBlock;
-  PoolMean jobs[3];
-  int nj = 0;
-  jobs[nj++] = PoolMean{r->layer_k(layer) + slot0 * slot_bytes, (int64_t)first * r->s * kBlock,
-                        r->layer_pooled(layer), 0, slot0, r->capacity, r->s, r->head_stride()};
-  if (first < n_slices)
-    jobs[nj++] = PoolMean{r->layer_k(layer), (int64_t)(n_slices - first) * r->s * kBlock, r->layer_pooled(layer), 0,
-                          0, r->capacity, r->s, r->head_stride()};
-  if (q_pooled) jobs[nj++] = PoolMean{q_out, lq, q_pooled, 0, 0, 1, 1 << 30, 0};
-  if ((rc = launch_pool_mean(r->dtype, jobs, nj, r->C, hist, nhist, stream))) return rc;
+  if ((rc = pool_new_slices(r, layer, slot0, n_slices, q_out, (int64_t)nb * kBlock, q_pooled, hist, nhist, stream)))
+    return rc;
   r->count[layer] += n_slices;
   return FVSR_OK;
 }
 
 extern "C" {
+
+int fvsr_kv_ring_append(fvsr_kv_ring* r, int layer, const void* k_new, const void* v_new, int n_slices, int layout,
+                        void* stream) {
+  return append_impl(r, layer, k_new, v_new, n_slices, layout, (hipStream_t)stream);
+}
 
 int fvsr_kv_ring_append_qkv(fvsr_kv_ring* r, int layer, const void* q, const void* k, const void* v, int n_slices,
                             int t0, const void* norm_q_weight, const void* norm_k_weight, float eps,
@@ -716,14 +722,17 @@ int fvsr_lcsa_layer(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* qW, i
   const Carve cv = carve(r->heads, nq, nk_after, r->C);
   if ((rc = ensure_ws(ctx, cv.total))) return rc;
   const RingMark mark = ring_mark(r, layer);
-  if ((rc = fvsr_kv_ring_append(r, layer, k_new, v_new, n_new_slices, layout, stream))) return rc;
-  const int nk = r->count[layer] * r->s;
   char* ws = (char*)ctx->ws;
+  // the pooled queries and the histogram reset ride in the append's pooling launch
+  if ((rc = append_impl(r, layer, k_new, v_new, n_new_slices, layout, st, qW, lq, (float*)(ws + cv.pq),
+                        (unsigned*)(ws + cv.hist), (int64_t)(hist12_bytes(r->heads, q_slices) / sizeof(unsigned)))))
+    return rc;
+  const int nk = r->count[layer] * r->s;
   int32_t* kidx = (int32_t*)(ws + cv.kidx);
   int32_t* kcnt = (int32_t*)(ws + cv.kcnt);
   rc = select_impl(ctx, r->dtype, qW, lq, r->layer_pooled(layer), true, nullptr, (int64_t)nk * kBlock,
                    r->map(layer), nk, r->heads, q_slices, r->s, local_dev, topk, mask_out, probs_out, kidx, kcnt,
-                   st);
+                   st, true);
   if (rc) return ring_rewind(r, layer, mark, rc);
   rc = attention_ring_impl(ctx, r, layer, qW, lq, kidx, kcnt, nk, o, st);
   if (rc) return ring_rewind(r, layer, mark, rc);
@@ -754,7 +763,7 @@ int fvsr_lcsa_layer_qkv(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const void* q
   if ((rc = ensure_ws(ctx, cv.total))) return rc;
   char* ws = (char*)ctx->ws;
   const RingMark mark = ring_mark(r, layer);
-  // the pooled queries and the histogram reset ride in the append's pooling launches
+  // the pooled queries and the histogram reset ride in the append's pooling launch
   if ((rc = append_qkv_impl(r, layer, q, k, v, n_new_slices, t0, norm_q_weight, norm_k_weight, eps, rope_tables,
                             q_work, st, (float*)(ws + cv.pq), (unsigned*)(ws + cv.hist),
                             (int64_t)(hist12_bytes(r->heads, q_slices) / sizeof(unsigned)))))

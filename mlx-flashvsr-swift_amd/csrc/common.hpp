@@ -110,16 +110,6 @@ __host__ __device__ __forceinline__ int64_t kv_offset(int64_t t, int c, int C, i
   return head_stride == 0 ? t * C + c : (int64_t)(c / kHeadDim) * head_stride + t * kHeadDim + c % kHeadDim;
 }
 
-// One block-mean target of pool_finish_kernel (kv_ring.hip): nb blocks (L tokens) of run sums in partial; block b
-// is written to row ((slot0 + b / slice_blocks) % capacity) * slice_blocks + b % slice_blocks of out (a ring
-// slot mapping; slot0 0, capacity 1, slice_blocks >= nb for a plain buffer).
-struct PoolDst {
-  const float* partial;
-  float* out;
-  int64_t L;
-  int nb, slot0, capacity, slice_blocks;
-};
-
 constexpr int kPartialFloats = kBlock * kHeadDim + 2 * kBlock;   // one item's partial attention result
 
 // Arguments of the attention kernels (lcsa_attn.hip).

@@ -48,8 +48,7 @@ struct Vec16<bf16> {
 // Jobs j0, j1, j2 share one launch: grid (j0.nb + j1.nb + j2.nb, ceil(nvec / per)) with `per` threads per quarter,
 // block index b of the grid runs over j0's blocks, then j1's, then j2's. Quarter `part` of the workgroup sums the
 // rows [b*128 + 32*part, +32) that exist, in row order, for channel vectors y*per .. y*per + per - 1; the mean is
-// ((r0 + r1) + (r2 + r3)) / n, the order the ring append's runs are finished in (pool_finish_kernel), so pooled keys
-// are bit-identical whichever path wrote them. Every workgroup also clears its share of `zero` (nzero words).
+// ((r0 + r1) + (r2 + r3)) / n. Every workgroup also clears its share of `zero` (nzero words).
 constexpr int kPoolVecs = 64;   // channel vectors per workgroup quarter: a 1536-channel block takes 3 workgroups, so
                                 // even a one-slice append (135 blocks) spreads over every CU
 template <typename T>

@@ -85,6 +85,20 @@ def test_select_and_attention_over_ring_equal_plain(dev, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("channels", [8, 520, 1536, 1544, 3200, 4096])
+def test_window_layout_widths(dev, dtype, channels):
+    """Partition and reverse at token widths around the copy's 64-lane vectors and its six vectors a lane (1 to 1024
+    16-byte vectors a token)."""
+    f, h, w = 4, 16, 24
+    x = torch.arange(f * h * w * channels, dtype=torch.int64).reshape(f * h * w, channels)
+    x = (x % 251 - 125).to(dtype)
+    p = fvsr_lcsa.window_partition(x.to(dev), f, h, w)
+    want = x.reshape(f // 2, 2, h // 8, 8, w // 8, 8, channels).permute(0, 2, 4, 1, 3, 5, 6).reshape(f * h * w, channels)
+    assert torch.equal(p.cpu(), want)
+    assert torch.equal(fvsr_lcsa.window_reverse(p, f, h, w).cpu(), x)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads,bh,bw", [(1, 1, 1), (2, 2, 3), (2, 5, 7)])
 def test_dense_mode_takes_lists_as_a_set(dev, dtype, heads, bh, bw):
     """Mode DENSE reads caller-supplied lists as a mask: any order, repeats, indices outside the held range, a count
