@@ -8,7 +8,7 @@
 // queries, two waves per SIMD; K/V tiles of 32 keys reach LDS by direct buffer->LDS copies into 4-slot rings;
 // S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16_bf16 so each lane owns one query row; the softmax keeps a fixed
 // reference per row (see the kernel's comment). fp32 (the parity lane): 4 wave64s x 32 queries, every fp32 operand
-// split into three bf16 parts and multiplied on the same matrix instruction, with a lazy online-softmax rescale. In
+// split into two scaled fp16 parts and multiplied on the fp16 matrix cores, with a lazy online-softmax rescale. In
 // both, calls with few rows split the rows' key lists into pieces that a second kernel merges.
 #include <algorithm>
 #include <cstdlib>
@@ -900,73 +900,59 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 // ------------------------------------------------------------------------------------------------------------
 // fp32 (parity lane)
 // ------------------------------------------------------------------------------------------------------------
-// The products run on the bf16 matrix cores: every fp32 operand is the exact sum of three bf16 parts (24 significand
-// bits = 8 + 8 + 8, each part the rounded remainder of the ones before it), and a product takes the six partial
-// products above 2^-24 of it, hi*lo and lo*hi and mid*mid first, hi*hi last, accumulated in fp32. The three left out
-// (mid*lo, lo*mid, lo*lo) are at most 2^-23 of the product and lie below the rounding of the fp32 sum. Six k = 16
-// products cost 192 matrix-core cycles per 32 x 32 x 16 block of products, against 512 for the eight k = 2 fp32 ones.
+// The products run on the fp16 matrix cores: every fp32 operand, scaled by a power of two, is split into two fp16 parts
+// h + l (11 + 11 significand bits and l's sign; at most 2^-23 of the value is lost, 2^-25 typically), and a product takes
+// h h + h l + l h, accumulated in fp32. The l l left out is 2^-22 of the product at most, 2^-25 typically, below the rounding
+// of the fp32 sum. Three k = 16 products cost 96 matrix-core cycles per 32 x 32 x 16 block of products, against 512 for the eight
+// k = 2 fp32 ones and 192 for the six of three bf16 parts.
 //
-// A workgroup = 4 wave64s x 32 queries, two per CU (48 KB of tile LDS, at most 256 registers a wave), so that one
-// workgroup's staging, softmax and waits run under the other's products. Keys stream in tiles of 32: a tile's fp32
-// rows are loaded into registers half a step ahead (raw buffer loads, rows past the buffer read 0), split once per
-// workgroup and stored as three bf16 planes with the 16-byte chunk swizzles of the bf16 walk. K and V planes each have
-// one buffer: K(T+1) is stored while PV(T) runs, V(T+1) while QK(T+1) runs, with one barrier after each product.
-// S^T = K Q^T leaves each lane one query's scores; the lazy online softmax is in fp32, and P is split in registers.
+// fp16 holds 2^-24 .. 65504, so every operand is brought to a range where its parts keep their bits:
+//   Q  each row's largest element to 2^13 .. 2^14, exactly (the row's score factor takes the power back)
+//   K  the largest element of the item's first nonzero tile to 2^9 .. 2^10: 64 times as large a one still fits, and what l cannot
+//      hold is 2^-34 of the largest, an absolute error of the scores below their fp32 rounding
+//   V  likewise to 2^7 .. 2^8, 253 times as large a one still fits; l is kept as l 2^11 (multiplied by h 2^-11 of P), so that
+//      channels or tokens down to 2^-20 of the largest keep all their bits
+//   P  2^7 for the first tile's largest, at most 2^15 (the lazy rescale below)
+// An item that meets a larger element, an infinity, or operands outside 2^-60 .. 2^60 is redone on the fp32 matrix cores
+// (f32_exact_walk). NaNs propagate through the parts.
 //
-// The split cannot hold values past the largest bf16 (3.39e38, infinities), and the parts of values near the smallest
-// normal number are lost: a workgroup that met the one, or a thread that saw only such V, redoes its item on the fp32
-// matrix cores (f32_exact_walk). NaNs propagate through the parts.
+// A workgroup = 4 wave64s x 32 queries, two per CU (64 KB of tile LDS, at most 256 registers a wave), so that one
+// workgroup's softmax and waits run under the other's products. Keys stream in tiles of 32: a tile's fp32 rows are loaded into
+// registers two tiles ahead (raw buffer loads, rows past the buffer read 0), split once per workgroup between the products of the
+// tile before and stored as two fp16 planes with the 16-byte chunk swizzles of the bf16 walk. K and V planes are double
+// buffered, one barrier a tile. S^T = K Q^T leaves each lane one query's scores; the lazy online softmax is in fp32, and P is
+// split in registers.
 //
-// Bound by the matrix cores (58 % busy) with the split's and the softmax's VALU work and the two barriers a tile.
-// 504 rows x 32 blocks: 705 us, 192 TFLOP/s of fp32 products, past the 157 of the fp32 matrix instructions, on which the
-// former kernel reached 90 to 120; 512 x 512 two-chunk clip 2813 -> 1528 us. Its error against 64 bits is the smaller one:
-// 1.4e-6 against 1.9e-6 on that clip, 5.3e-7 against 8.1e-7 on a sparse 512 x 512 layer.
-constexpr int kF32Plane = kTileBytes;              // one bf16 plane of a 32-key tile
-constexpr float kSplitMax = 3.3895314e38f;         // the largest finite bf16
-constexpr float kSplitMin = 1.2621775e-29f;        // 2^-96: the parts of smaller values near the normal range's end
+// Bound by the matrix cores together with the splits', the softmax's and the operand reads' issue slots (48 MFMAs = 1536
+// cycles, about 240 VALU and 60 LDS instructions a wave and tile). 512 x 512, 12 heads: 192 rows x 32 of 48 blocks (layer call
+// of 2 latent frames over 6) 316 us on the fp32 instructions, 178 with three bf16 parts, 121 now; two-chunk clip 3834, 1458
+// and 918 us. Its error against 64 bits is the smallest of the three: 8.1e-7, 5.3e-7, 4.2e-7 and 1.9e-6, 1.4e-6, 1.1e-6.
+constexpr int kF32Plane = kTileBytes;              // one fp16 plane of a 32-key tile
+constexpr int kF32Buf = 4 * kF32Plane;             // K planes h, l, then V planes h, l 2^11
+constexpr float kSplitMax = 65000.f;               // the largest scaled element the parts may hold
+constexpr float kRangeMin = 8.6736174e-19f, kRangeMax = 1.1529215e18f;   // 2^-60, 2^60: operands the scaling serves
+constexpr float kPRef = 7.f, kPGrow = 15.f;        // P is 2^7 at the reference's score; the reference follows past 2^15
 constexpr int kExactLd = 132;                      // padded fp32 row of the exact walk's tiles (floats)
 
-// two values as their packed parts h + m + l
-__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  auto pack = [](float x, float y) -> unsigned {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
-  };
-  auto lo = [](unsigned u) { return __uint_as_float(u << 16); };
-  auto hi = [](unsigned u) { return __uint_as_float(u & 0xffff0000u); };
-  h = pack(a, b);
-  const float ra = a - lo(h), rb = b - hi(h);
-  m = pack(ra, rb);
-  l = pack(ra - lo(m), rb - hi(m));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+
+// two values (x 2^S, and x 2^S 2^L in a2, b2) as packed fp16 parts h and l 2^L
+template <int L>
+__device__ __forceinline__ void split_pair(float a, float b, float a2, float b2, unsigned& h, unsigned& l) {
+  const f16x2 hv = __builtin_convertvector(f32x2{a, b}, f16x2);
+  constexpr float kNeg = -(float)(1 << L);
+  const float ra = fmaf((float)hv[0], kNeg, a2), rb = fmaf((float)hv[1], kNeg, b2);
+  h = __builtin_bit_cast(unsigned, hv);
+  l = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{ra, rb}, f16x2));
 }
 
-struct Planes8 {   // eight values as three bf16 parts
-  u32x4 h, m, l;
-};
-__device__ __forceinline__ Planes8 split8(const f32x4& x, const f32x4& y, float& mag) {
-  Planes8 p;
-  unsigned h, m, l;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = i < 2 ? x[2 * i] : y[2 * i - 4], b = i < 2 ? x[2 * i + 1] : y[2 * i - 3];
-    split_pair(a, b, h, m, l);
-    p.h[i] = h;
-    p.m[i] = m;
-    p.l[i] = l;
-    mag = fmaxf(mag, fmaxf(fabsf(a), fabsf(b)));
-  }
-  return p;
-}
-
-// The six partial products of one k = 16 step, smallest first.
-__device__ __forceinline__ void mfma_split(f32x16& acc, const bf16x8& ah, const bf16x8& am, const bf16x8& al,
-                                           const bf16x8& bh, const bf16x8& bm, const bf16x8& bl) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bm, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bh, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bm, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc, 0, 0, 0);
+// the power of two that brings a magnitude mx (0, or within kRangeMin .. kRangeMax) to 2^(target - 1) .. 2^target; 1 for 0
+__device__ __forceinline__ float scale_to(float mx, int target) {
+  const int e = (int)((__float_as_uint(mx) >> 23) & 255u);   // 2^(e - 127) <= mx < 2^(e - 126)
+  return mx >= kRangeMin && mx <= kRangeMax ? __uint_as_float((unsigned)(target - 1 - (e - 127) + 127) << 23) : 1.f;
 }
 
 // One item on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), for operands the split cannot hold. Every wave of the
@@ -1036,9 +1022,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
                      const float* __restrict__ Q, float* __restrict__ O, const int32_t* __restrict__ order,
                      int32_t* __restrict__ counter) {
-  __shared__ __attribute__((aligned(1024))) char smem[6 * kF32Plane];   // K planes h, m, l, then V planes h, m, l
-  static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 6 * kF32Plane, "the exact walk's tiles fit");
+  __shared__ __attribute__((aligned(1024))) char smem[2 * kF32Buf];
+  static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 2 * kF32Buf, "the exact walk's tiles fit");
   __shared__ int item_s;
+  __shared__ unsigned tile_max[2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
@@ -1054,14 +1041,14 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
   const int st_v[2] = {r_ld * kRowBytes + ((c_ld ^ swz_v(r_ld)) << 4),
                        (r_ld + 16) * kRowBytes + ((c_ld ^ swz_v(r_ld + 16)) << 4)};
   // operand reads, as in the bf16 walk
-  const int kb = l32 * kRowBytes, kx = swz_k(l32);
+  int k_off[8], v_off[4];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) k_off[t] = l32 * kRowBytes + (((2 * t + g) ^ swz_k(l32)) << 4);
   const int G = lane >> 4, mm = lane & 15, vr = 4 * (G >> 1) + (mm >> 2);
-  int v_off[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
     v_off[dt] = vr * kRowBytes + (((4 * dt + 2 * (G & 1) + ((mm & 3) >> 1)) ^ swz_v(vr)) << 4) + (mm & 1) * 8;
   lds_char* const lds = (lds_char*)(uintptr_t)lds_addr(smem);
-  lds_char* const ldsv = lds + 3 * kF32Plane;
 
   for (bool first = true;; first = false) {
     int item;
@@ -1074,35 +1061,19 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     const int32_t* __restrict__ klist = kidx + (int64_t)it.row * a.nk_stride + it.b0;
     const int nblocks = it.nblocks;
     const int64_t qrow = (int64_t)it.qb * kBlock + wave * 32 + l32;
-    float mag = 0.f, mag_v = 0.f;   // largest magnitude this thread split: Q and K, V
-    bf16x8 qh[8], qm[8], ql[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      f32x4 x = f32x4{0, 0, 0, 0}, y = f32x4{0, 0, 0, 0};
-      if (qrow < a.lq) {
-        const float* p = Q + qrow * a.ld + it.h * kHeadDim + 16 * t + 8 * g;
-        x = *(const f32x4*)p;
-        y = *(const f32x4*)(p + 4);
-      }
-      const Planes8 p = split8(x, y, mag);
-      qh[t] = __builtin_bit_cast(bf16x8, p.h);
-      qm[t] = __builtin_bit_cast(bf16x8, p.m);
-      ql[t] = __builtin_bit_cast(bf16x8, p.l);
-    }
+
+    // walked block b: byte offset of its first row (past the buffer for an index outside [0, nk) and past the walk's end)
+    // and its keys taking part
+    auto walk_entry = [&](int b) -> int { return b < nblocks ? klist[b] : -1; };
+    auto entry_off = [&](int j) -> uint32_t {
+      return (unsigned)j < (unsigned)a.nk ? (uint32_t)a.map.row(j) * row_bytes : range;
+    };
+    auto entry_keys = [&](int j) -> int {
+      return (unsigned)j < (unsigned)a.nk ? (int)min<int64_t>(kBlock, a.lk - (int64_t)j * kBlock) : 0;
+    };
+    const uint32_t sub_bytes = kTileKeys * row_bytes;
     const uint32_t ld_off = r_ld * row_bytes + (uint32_t)(it.h * a.kv_head_stride * 4) + c_ld * 32;
-    // tile T = quarter T % 4 of the T / 4-th listed block: byte offset of its first row (past the buffer for a block
-    // outside [0, nk) and past the walk's end) and its keys taking part
-    auto tile_off = [&](int T) -> uint32_t {
-      if ((T >> 2) >= nblocks) return range;
-      const int j = klist[T >> 2];
-      return (unsigned)j < (unsigned)a.nk ? (uint32_t)(a.map.row(j) + (T & 3) * kTileKeys) * row_bytes : range;
-    };
-    auto tile_valid = [&](int T) -> int {
-      const int j = klist[T >> 2];
-      if ((unsigned)j >= (unsigned)a.nk) return 0;
-      return (int)min<int64_t>(kTileKeys, a.lk - ((int64_t)j * kBlock + (T & 3) * kTileKeys));
-    };
-    f32x4 raw[4];
+    f32x4 raw[4];   // this thread's part of the K or V tile to be split next
     auto load_raw = [&](__amdgpu_buffer_rsrc_t rs, uint32_t off) {
       const uint32_t o0 = ld_off + off, o1 = o0 + 16 * row_bytes;   // < 2^31 + 2^18: no wrap
       raw[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0, 0, 0));
@@ -1110,42 +1081,150 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
       raw[2] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1, 0, 0));
       raw[3] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1 + 16, 0, 0));
     };
-    auto store_planes = [&](lds_char* base, const int (&at)[2], float& largest) {
+    auto largest = [&]() -> float {
+      float m = 0.f;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const Planes8 p = split8(raw[2 * i], raw[2 * i + 1], largest);
-        *(lds_u32x4*)(base + at[i]) = p.h;
-        *(lds_u32x4*)(base + kF32Plane + at[i]) = p.m;
-        *(lds_u32x4*)(base + 2 * kF32Plane + at[i]) = p.l;
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(raw[i][e]));
+      return m;
+    };
+
+    // K and V scales from the item's first tile with a nonzero element of theirs: the first tile, but for leading zeros
+    float kmax = 0.f, vmax = 0.f;
+    for (int T = 0; T < 4 * nblocks && (kmax == 0.f || vmax == 0.f); ++T) {
+      const uint32_t off = entry_off(klist[T >> 2]);
+      const uint32_t at = off == range ? range : off + (T & 3) * sub_bytes;
+      if (tid < 2) tile_max[tid] = 0u;
+      __syncthreads();
+      load_raw(krs, at);
+      atomicMax(&tile_max[0], __float_as_uint(largest()));   // magnitudes: bit order is value order
+      load_raw(vrs, at);
+      atomicMax(&tile_max[1], __float_as_uint(largest()));
+      __syncthreads();
+      if (kmax == 0.f) kmax = __uint_as_float(tile_max[0]);
+      if (vmax == 0.f) vmax = __uint_as_float(tile_max[1]);
+      __syncthreads();   // tile_max has been read
+    }
+    auto in_range = [](float m) { return m == 0.f || (m >= kRangeMin && m <= kRangeMax); };
+    bool exact = !in_range(kmax) || !in_range(vmax);
+    const float sk = scale_to(kmax, 10), sv = scale_to(vmax, 8), sv2 = sv * 2048.f;
+    float mag_k = 0.f, mag_v = 0.f;   // largest scaled magnitude this thread split
+
+    // Q as the B operand of S^T = K Q^T, scaled by its row's power of two
+    f16x8 qh[8], ql[8];
+    float c_row;
+    {
+      f32x4 x[16];
+      float m = 0.f;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        x[2 * t] = x[2 * t + 1] = f32x4{0, 0, 0, 0};
+        if (qrow < a.lq) {
+          const float* p = Q + qrow * a.ld + it.h * kHeadDim + 16 * t + 8 * g;
+          x[2 * t] = *(const f32x4*)p;
+          x[2 * t + 1] = *(const f32x4*)(p + 4);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(x[2 * t][e]), fabsf(x[2 * t + 1][e])));
+      }
+      m = pair_max(m);
+      exact |= !in_range(m);
+      const float sq = scale_to(m, 14);
+      c_row = a.c / (sq * sk);   // powers of two: exact
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        u32x4 h, l;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = x[2 * t + (i >> 1)][2 * (i & 1)] * sq, r = x[2 * t + (i >> 1)][2 * (i & 1) + 1] * sq;
+          unsigned hw, lw;
+          split_pair<0>(p, r, p, r, hw, lw);
+          h[i] = hw;
+          l[i] = lw;
+        }
+        qh[t] = __builtin_bit_cast(f16x8, h);
+        ql[t] = __builtin_bit_cast(f16x8, l);
+      }
+    }
+
+    // pair I (elements 2 I, 2 I + 1 of this thread's 16) of the raw tile; after pairs 3 and 7 a chunk of 8 is stored
+    u32x4 wh, wl;
+    auto split_k = [&](auto i_c, lds_char* planes) {
+      constexpr int I = decltype(i_c)::value;
+      const float p = raw[I >> 1][2 * (I & 1)] * sk, r = raw[I >> 1][2 * (I & 1) + 1] * sk;
+      unsigned hw, lw;
+      split_pair<0>(p, r, p, r, hw, lw);
+      mag_k = fmaxf(mag_k, fmaxf(fabsf(p), fabsf(r)));
+      asm volatile("" : "+v"(mag_k));   // here: the compiler would keep the elements of a whole block for one late maximum
+      wh[I & 3] = hw;
+      wl[I & 3] = lw;
+      if constexpr ((I & 3) == 3) {
+        *(lds_u32x4*)(planes + st_k[I >> 2]) = wh;
+        *(lds_u32x4*)(planes + kF32Plane + st_k[I >> 2]) = wl;
       }
     };
+    auto split_v = [&](auto i_c, lds_char* planes) {
+      constexpr int I = decltype(i_c)::value;
+      const float x = raw[I >> 1][2 * (I & 1)], y = raw[I >> 1][2 * (I & 1) + 1];
+      const float p = x * sv, r = y * sv;
+      unsigned hw, lw;
+      split_pair<11>(p, r, x * sv2, y * sv2, hw, lw);
+      mag_v = fmaxf(mag_v, fmaxf(fabsf(p), fabsf(r)));
+      asm volatile("" : "+v"(mag_v));   // here: the compiler would keep the elements of a whole block for one late maximum
+      wh[I & 3] = hw;
+      wl[I & 3] = lw;
+      if constexpr ((I & 3) == 3) {
+        *(lds_u32x4*)(planes + 2 * kF32Plane + st_v[I >> 2]) = wh;
+        *(lds_u32x4*)(planes + 3 * kF32Plane + st_v[I >> 2]) = wl;
+      }
+    };
+
     f32x16 acc[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) acc[d] = f32x16{};
-    float m_run = -INFINITY, l_run = 0.f;
-    const int ntiles = 4 * nblocks;
+    float m_ref = -INFINITY, l_run = 0.f;   // P = exp2(c S - m_ref); the row's largest score so far is about m_ref + 7 .. + 15
 
-    load_raw(krs, tile_off(0));
-    store_planes(lds, st_k, mag);
-    load_raw(vrs, tile_off(0));
-    __syncthreads();   // K(0) stored
-    for (int T = 0; T < ntiles; ++T) {
-      // V(T) goes to LDS (PV(T-1) is done) while this tile's scores are formed; then K(T+1) is requested
-      store_planes(ldsv, st_v, mag_v);
-      const uint32_t off_next = tile_off(T + 1);
-      load_raw(krs, off_next);
+    // one tile, in buffer SUB % 2: its products, while the next tile (byte offset off1; its K in raw) is split into the other
+    // buffer: K in the second half of the scores' products, V in the first half of the output's, so that each one's loads have
+    // half a tile to arrive in one set of registers
+    auto step = [&](auto sub_c, int valid, uint32_t off1, uint32_t off2) {
+      constexpr int SUB = decltype(sub_c)::value;
+      lds_char* const buf = lds + (SUB & 1) * kF32Buf;
+      lds_char* const nxt = lds + ((SUB & 1) ^ 1) * kF32Buf;
+      f16x8 kh[8], kl[8];
+      auto read_k = [&](int t) {
+        kh[t] = *(const lds_f16x8*)(buf + k_off[t]);
+        kl[t] = *(const lds_f16x8*)(buf + kF32Plane + k_off[t]);
+      };
+      read_k(0);
+      read_k(1);
       f32x16 s = f32x16{};
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        lds_char* const p = lds + kb + (((2 * t + g) ^ kx) << 4);
-        const bf16x8 kh = *(const lds_bf16x8*)p, km = *(const lds_bf16x8*)(p + kF32Plane);
-        const bf16x8 kl = *(const lds_bf16x8*)(p + 2 * kF32Plane);
-        mfma_split(s, kh, km, kl, qh[t], qm[t], ql[t]);
-      }
-      __syncthreads();   // K(T) has been read, V(T) is stored
-      store_planes(lds, st_k, mag);
-      load_raw(vrs, off_next);
-      const int valid = tile_valid(T);
+      static_for<0, 8>([&](auto t_c) {
+        constexpr int t = decltype(t_c)::value;
+        if constexpr (t + 2 < 8) read_k(t + 2);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[t], qh[t], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], ql[t], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], qh[t], s, 0, 0, 0);
+        if constexpr (t >= 4) {
+          split_k(std::integral_constant<int, 2 * t - 8>{}, nxt);
+          split_k(std::integral_constant<int, 2 * t - 7>{}, nxt);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      load_raw(vrs, off1);
+      f16x8 vh[8], vl[8];
+      auto read_v = [&](int i) {   // pair i = (u, dt): V^T operands of keys 16 u .., dims 32 dt ..
+        lds_char* const pa = buf + 2 * kF32Plane + v_off[i & 3] + 16 * (i >> 2) * kRowBytes;
+        const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)pa);
+        const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + 8 * kRowBytes));
+        vh[i] = __builtin_bit_cast(f16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+        const i16x4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + kF32Plane));
+        const i16x4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + kF32Plane + 8 * kRowBytes));
+        vl[i] = __builtin_bit_cast(f16x8, __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7));
+      };
+      read_v(0);
+      read_v(1);
       if (valid < kTileKeys) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -1154,49 +1233,93 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
       float mx = fmaxf(s[0], s[1]);
 #pragma unroll
       for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
-      const float m_use = rescale_if_grown<4>(pair_max(mx) * a.c, m_run, l_run, acc);
+      const float mxc = pair_max(mx) * c_row;
+      // the lazy rescale: the reference follows only when P would pass 2^15, a wave-uniform branch
+      const bool grow = mxc > m_ref + kPGrow;
+      if (__ballot(grow) != 0) {
+        const float m_new = grow ? mxc - kPRef : m_ref;
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;   // m_ref = -inf: 0
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[d][r] *= alpha;
+        m_ref = m_new;
+      }
+      const float negm = m_ref == -INFINITY ? 0.f : -m_ref;
       float sum[2] = {0.f, 0.f};
-      bf16x8 ph[2], pm[2], pl[2];
+      f16x8 ph[2], pl[2], ps[2];   // h, l and h 2^-11 of P
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        u32x4 wh, wm, wl;
+        u32x4 h, l, hs;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i], a.c, -m_use));
-          const float y = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i + 1], a.c, -m_use));
+          const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i], c_row, negm));
+          const float y = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i + 1], c_row, negm));
           sum[0] += x;
           sum[1] += y;
-          unsigned h, m, l;
-          split_pair(x, y, h, m, l);
-          wh[i] = h;
-          wm[i] = m;
-          wl[i] = l;
+          unsigned hw, lw;
+          split_pair<0>(x, y, x, y, hw, lw);
+          h[i] = hw;
+          l[i] = lw;
+          hs[i] = __builtin_bit_cast(
+              unsigned, __builtin_bit_cast(f16x2, hw) * f16x2{(_Float16)4.8828125e-4f, (_Float16)4.8828125e-4f});
         }
-        ph[u] = __builtin_bit_cast(bf16x8, wh);
-        pm[u] = __builtin_bit_cast(bf16x8, wm);
-        pl[u] = __builtin_bit_cast(bf16x8, wl);
+        ph[u] = __builtin_bit_cast(f16x8, h);
+        pl[u] = __builtin_bit_cast(f16x8, l);
+        ps[u] = __builtin_bit_cast(f16x8, hs);
       }
       l_run += sum[0] + sum[1];
+      __builtin_amdgcn_sched_barrier(0);
       // O^T += V^T P^T
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          bf16x8 vv[3];
-#pragma unroll
-          for (int p = 0; p < 3; ++p) {
-            lds_char* const pa = ldsv + p * kF32Plane + v_off[dt] + 16 * u * kRowBytes;
-            const i16x4 va = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)pa);
-            const i16x4 vb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + 8 * kRowBytes));
-            vv[p] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7));
-          }
-          mfma_split(acc[dt], vv[0], vv[1], vv[2], ph[u], pm[u], pl[u]);
+      static_for<0, 8>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value, u = i >> 2, dt = i & 3;
+        if constexpr (i + 2 < 8) read_v(i + 2);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i], ps[u], acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], pl[u], acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], ph[u], acc[dt], 0, 0, 0);
+        if constexpr (i < 4) {
+          split_v(std::integral_constant<int, 2 * i>{}, nxt);
+          split_v(std::integral_constant<int, 2 * i + 1>{}, nxt);
         }
-      __syncthreads();   // V(T) has been read, K(T+1) is stored
+        if constexpr (i == 3) load_raw(krs, off2);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      __syncthreads();   // this tile has been read, the next one is stored
+    };
+
+    int e0 = walk_entry(0), e1 = walk_entry(1);
+    uint32_t o0 = entry_off(e0);
+    auto sub_off = [&](uint32_t o, int sub) -> uint32_t { return o == range ? range : o + sub * sub_bytes; };
+    load_raw(krs, sub_off(o0, 0));
+    static_for<0, 8>([&](auto i_c) { split_k(i_c, lds); });
+    load_raw(vrs, sub_off(o0, 0));
+    static_for<0, 8>([&](auto i_c) { split_v(i_c, lds); });
+    load_raw(krs, sub_off(o0, 1));
+    __syncthreads();
+    for (int b = 0; b < nblocks; ++b) {
+      const int n0 = entry_keys(e0);
+      const uint32_t o1 = entry_off(e1);
+      e0 = e1;
+      e1 = walk_entry(b + 2);
+      static_for<0, 4>([&](auto sub_c) {
+        constexpr int SUB = decltype(sub_c)::value;
+        step(sub_c, n0 - SUB * kTileKeys, sub_off(SUB < 3 ? o0 : o1, (SUB + 1) & 3),
+             sub_off(SUB < 2 ? o0 : o1, (SUB + 2) & 3));
+      });
+      o0 = o1;
     }
-    if (__syncthreads_or(!(fmaxf(mag, mag_v) <= kSplitMax) || (mag_v > 0.f && mag_v < kSplitMin)))
-      f32_exact_walk(a, it.h, qrow, klist, nblocks, (float*)smem, acc, m_run, l_run);
-    attn_store<DIRECT, float>(a, it, item, wave, acc, m_run == -INFINITY ? 0.f : m_run, pair_sum(l_run), O);
+    exact |= !(fmaxf(mag_k, mag_v) <= kSplitMax);
+    if (__syncthreads_or(exact)) {
+      f32_exact_walk(a, it.h, qrow, klist, nblocks, (float*)smem, acc, m_ref, l_run);
+    } else {
+      const float inv = 1.f / sv;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[d][r] *= inv;
+    }
+    attn_store<DIRECT, float>(a, it, item, wave, acc, m_ref == -INFINITY ? 0.f : m_ref, pair_sum(l_run), O);
     __syncthreads();   // smem and item_s are free for the next item
   }
 }

@@ -514,7 +514,7 @@ def test_split_key_lists(dev, dtype, heads, lqb, nkb):
 
 @pytest.mark.parametrize("heads,lqb", [(2, 2), (8, 66)])
 def test_fp32_values_outside_the_split(dev, heads, lqb):
-    """fp32 operands that three bf16 parts cannot hold: an infinite V column stays infinite and leaves the others alone,
+    """fp32 operands that the split into 16-bit parts cannot hold: an infinite V column stays infinite and leaves the others alone,
     a NaN stays in its column, a -inf K row is masked out for the queries that score it -inf, and V near the smallest
     normal number keeps its precision (split rows and one row per workgroup, 4 and 528 rows)."""
     gen = torch.Generator(device=dev).manual_seed(heads)
@@ -544,3 +544,46 @@ def test_fp32_values_outside_the_split(dev, heads, lqb):
     o = fvsr_lcsa.kernel_block_attention(q, k, v * 1e-36, m, heads)
     r = ref(q, k, v * 1e-36, 1)
     assert float((o[:, 128:256].double() - r).abs().max() / r.abs().max()) <= FP32_REL
+
+
+@pytest.mark.parametrize("what", ["plain", "tiny", "huge", "zero start", "K grows", "V grows", "V outlier first",
+                                  "V channels", "Q rows"])
+def test_fp32_operand_scales(dev, what):
+    """The fp32 lane scales K and V by the first nonzero tile of a list and Q by row before it splits them: operands far from
+    1, lists that begin with zeros, magnitudes that grow along the list past what the scale leaves room for (redone on the fp32
+    instructions), a first tile far above the rest, channels and query rows six decades apart. Split rows and whole ones; the
+    error of each output channel relative to its own size, at the lane's bar."""
+    heads, lqb, nkb = 2, 3, 7
+    gen = torch.Generator(device=dev).manual_seed(len(what))
+    lq, lk = lqb * 128 - 9, nkb * 128 - 37
+    q, k, v = (torch.randn((n, heads * 128), generator=gen, device=dev) for n in (lq, lk, lk))
+    if what == "tiny":
+        q, k, v = q * 1e9, k * 1e-9, v * 1e-12
+    elif what == "huge":
+        q, k, v = q * 1e-7, k * 1e7, v * 1e12
+    elif what == "zero start":
+        k[:160], v[:200] = 0.0, 0.0
+    elif what == "K grows":
+        k[:128] *= 1e-4
+    elif what == "V grows":
+        v[:128] *= 1e-5
+    elif what == "V outlier first":
+        v[:32] *= 1e4
+    elif what == "V channels":
+        v = v * (10.0 ** -(torch.arange(heads * 128, device=dev) % 7).float())
+    elif what == "Q rows":
+        q = q * (10.0 ** -(torch.arange(lq, device=dev) % 7).float())[:, None]
+    for heads_rep in (1, 128):   # 6 rows (split) and 768 (whole rows, persistent walk)
+        qq, kk, vv = (x.repeat(1, heads_rep) if heads_rep == 1 else x[:, :128].repeat(1, 256).contiguous()
+                      for x in (q, k, v))
+        n = heads if heads_rep == 1 else 256
+        m = torch.ones((n, lqb, nkb), device=dev)
+        m[:, 1, 2] = 0.0
+        o = fvsr_lcsa.kernel_block_attention(qq, kk, vv, m, n)
+        keep = m[0].bool().repeat_interleave(128, 0)[:lq].repeat_interleave(128, 1)[:, :lk]
+        for h in (0, n - 1):
+            c = slice(h * 128, (h + 1) * 128)
+            s = (qq[:, c].double() @ kk[:, c].double().t().contiguous() / 128 ** 0.5).masked_fill(~keep, -float("inf"))
+            ref = torch.softmax(s, -1) @ vv[:, c].double()
+            err = (o[:, c].double() - ref).abs().amax(0) / ref.abs().amax(0)
+            assert float(err.max()) <= FP32_REL, (h, float(err.max()))
