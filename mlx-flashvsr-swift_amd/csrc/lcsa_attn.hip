@@ -1041,13 +1041,10 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
   const int st_v[2] = {r_ld * kRowBytes + ((c_ld ^ swz_v(r_ld)) << 4),
                        (r_ld + 16) * kRowBytes + ((c_ld ^ swz_v(r_ld + 16)) << 4)};
   // operand reads, as in the bf16 walk
-  int k_off[8], v_off[4];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) k_off[t] = l32 * kRowBytes + (((2 * t + g) ^ swz_k(l32)) << 4);
+  // (chunk 2 t + g of a K row is 32 t xor chunk g's offset, V columns 32 dt .. are 64 dt xor columns 0 ..'s)
+  const int k_off = l32 * kRowBytes + ((g ^ swz_k(l32)) << 4);
   const int G = lane >> 4, mm = lane & 15, vr = 4 * (G >> 1) + (mm >> 2);
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
-    v_off[dt] = vr * kRowBytes + (((4 * dt + 2 * (G & 1) + ((mm & 3) >> 1)) ^ swz_v(vr)) << 4) + (mm & 1) * 8;
+  const int v_off = vr * kRowBytes + (((2 * (G & 1) + ((mm & 3) >> 1)) ^ swz_v(vr)) << 4) + (mm & 1) * 8;
   lds_char* const lds = (lds_char*)(uintptr_t)lds_addr(smem);
 
   for (bool first = true;; first = false) {
@@ -1073,15 +1070,15 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     };
     const uint32_t sub_bytes = kTileKeys * row_bytes;
     const uint32_t ld_off = r_ld * row_bytes + (uint32_t)(it.h * a.kv_head_stride * 4) + c_ld * 32;
-    f32x4 raw[4];   // this thread's part of the K or V tile to be split next
-    auto load_raw = [&](__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    f32x4 rk[4], rv[4];   // this thread's part of the K and V tiles to be split next
+    auto load_raw = [&](__amdgpu_buffer_rsrc_t rs, f32x4 (&raw)[4], uint32_t off) {
       const uint32_t o0 = ld_off + off, o1 = o0 + 16 * row_bytes;   // < 2^31 + 2^18: no wrap
       raw[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0, 0, 0));
       raw[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0 + 16, 0, 0));
       raw[2] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1, 0, 0));
       raw[3] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1 + 16, 0, 0));
     };
-    auto largest = [&]() -> float {
+    auto largest = [](const f32x4 (&raw)[4]) -> float {
       float m = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -1097,10 +1094,10 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
       const uint32_t at = off == range ? range : off + (T & 3) * sub_bytes;
       if (tid < 2) tile_max[tid] = 0u;
       __syncthreads();
-      load_raw(krs, at);
-      atomicMax(&tile_max[0], __float_as_uint(largest()));   // magnitudes: bit order is value order
-      load_raw(vrs, at);
-      atomicMax(&tile_max[1], __float_as_uint(largest()));
+      load_raw(krs, rk, at);
+      load_raw(vrs, rv, at);
+      atomicMax(&tile_max[0], __float_as_uint(largest(rk)));   // magnitudes: bit order is value order
+      atomicMax(&tile_max[1], __float_as_uint(largest(rv)));
       __syncthreads();
       if (kmax == 0.f) kmax = __uint_as_float(tile_max[0]);
       if (vmax == 0.f) vmax = __uint_as_float(tile_max[1]);
@@ -1152,7 +1149,7 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     u32x4 wh, wl;
     auto split_k = [&](auto i_c, lds_char* planes) {
       constexpr int I = decltype(i_c)::value;
-      const float p = raw[I >> 1][2 * (I & 1)] * sk, r = raw[I >> 1][2 * (I & 1) + 1] * sk;
+      const float p = rk[I >> 1][2 * (I & 1)] * sk, r = rk[I >> 1][2 * (I & 1) + 1] * sk;
       unsigned hw, lw;
       split_pair<0>(p, r, p, r, hw, lw);
       mag_k = fmaxf(mag_k, fmaxf(fabsf(p), fabsf(r)));
@@ -1166,7 +1163,7 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     };
     auto split_v = [&](auto i_c, lds_char* planes) {
       constexpr int I = decltype(i_c)::value;
-      const float x = raw[I >> 1][2 * (I & 1)], y = raw[I >> 1][2 * (I & 1) + 1];
+      const float x = rv[I >> 1][2 * (I & 1)], y = rv[I >> 1][2 * (I & 1) + 1];
       const float p = x * sv, r = y * sv;
       unsigned hw, lw;
       split_pair<11>(p, r, x * sv2, y * sv2, hw, lw);
@@ -1185,46 +1182,46 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     for (int d = 0; d < 4; ++d) acc[d] = f32x16{};
     float m_ref = -INFINITY, l_run = 0.f;   // P = exp2(c S - m_ref); the row's largest score so far is about m_ref + 7 .. + 15
 
-    // one tile, in buffer SUB % 2: its products, while the next tile (byte offset off1; its K in raw) is split into the other
-    // buffer: K in the second half of the scores' products, V in the first half of the output's, so that each one's loads have
-    // half a tile to arrive in one set of registers
+    // One tile, in buffer SUB % 2, while the next tile (byte offset off1; its K in rk) is split into the other buffer. 24
+    // rounds of one MFMA each for the scores, then 24 for the output, fenced so that the order below is the issue order: a
+    // wave issues in order and an MFMA holds the matrix core for 32 cycles, so a slice of the other work follows each. K is
+    // split under the last 16 rounds of the scores, the exponentials and the split of P for keys 16 .. 31 run under the first 12
+    // rounds of the output (those of keys 0 .. 15), V is split under the last 12. K of the tile after the next (off2) is
+    // requested half way through the output, V of the next at the start.
     auto step = [&](auto sub_c, int valid, uint32_t off1, uint32_t off2) {
       constexpr int SUB = decltype(sub_c)::value;
       lds_char* const buf = lds + (SUB & 1) * kF32Buf;
       lds_char* const nxt = lds + ((SUB & 1) ^ 1) * kF32Buf;
       f16x8 kh[8], kl[8];
       auto read_k = [&](int t) {
-        kh[t] = *(const lds_f16x8*)(buf + k_off[t]);
-        kl[t] = *(const lds_f16x8*)(buf + kF32Plane + k_off[t]);
+        lds_char* const p = buf + (k_off ^ (t << 5));
+        kh[t] = *(const lds_f16x8*)p;
+        kl[t] = *(const lds_f16x8*)(p + kF32Plane);
       };
       read_k(0);
       read_k(1);
+      load_raw(vrs, rv, off1);
       f32x16 s = f32x16{};
-      static_for<0, 8>([&](auto t_c) {
-        constexpr int t = decltype(t_c)::value;
-        if constexpr (t + 2 < 8) read_k(t + 2);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[t], qh[t], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], ql[t], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], qh[t], s, 0, 0, 0);
-        if constexpr (t >= 4) {
-          split_k(std::integral_constant<int, 2 * t - 8>{}, nxt);
-          split_k(std::integral_constant<int, 2 * t - 7>{}, nxt);
-        }
+      static_for<0, 24>([&](auto r_c) {
+        constexpr int r = decltype(r_c)::value, t = r / 3;
+        if constexpr (r % 3 == 0 && t + 2 < 8) read_k(t + 2);
+        if constexpr (r % 3 == 0) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[t], qh[t], s, 0, 0, 0);
+        if constexpr (r % 3 == 1) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], ql[t], s, 0, 0, 0);
+        if constexpr (r % 3 == 2) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], qh[t], s, 0, 0, 0);
+        if constexpr (r >= 8 && r % 2 == 0) split_k(std::integral_constant<int, (r - 8) / 2>{}, nxt);
         __builtin_amdgcn_sched_barrier(0);
       });
-      load_raw(vrs, off1);
       f16x8 vh[8], vl[8];
-      auto read_v = [&](int i) {   // pair i = (u, dt): V^T operands of keys 16 u .., dims 32 dt ..
-        lds_char* const pa = buf + 2 * kF32Plane + v_off[i & 3] + 16 * (i >> 2) * kRowBytes;
+      auto read_v = [&](int plane, int i) -> f16x8 {   // i = 4 u + dt: V^T operand of keys 16 u .., dims 32 dt ..
+        lds_char* const pa = buf + (2 + plane) * kF32Plane + (v_off ^ ((i & 3) << 6)) + 16 * (i >> 2) * kRowBytes;
         const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)pa);
         const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + 8 * kRowBytes));
-        vh[i] = __builtin_bit_cast(f16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
-        const i16x4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + kF32Plane));
-        const i16x4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + kF32Plane + 8 * kRowBytes));
-        vl[i] = __builtin_bit_cast(f16x8, __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7));
+        return __builtin_bit_cast(f16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
       };
-      read_v(0);
-      read_v(1);
+      vl[0] = read_v(1, 0);
+      vl[1] = read_v(1, 1);
+      vh[0] = read_v(0, 0);
+      vh[1] = read_v(0, 1);
       if (valid < kTileKeys) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -1247,55 +1244,70 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
         m_ref = m_new;
       }
       const float negm = m_ref == -INFINITY ? 0.f : -m_ref;
-      float sum[2] = {0.f, 0.f};
-      f16x8 ph[2], pl[2], ps[2];   // h, l and h 2^-11 of P
+      u32x4 ph[2], pl[2], ps[2];   // h, l and h 2^-11 of P
+      float px, py, sum[2] = {0.f, 0.f};
+      auto exp_x = [&](int j) { px = __builtin_amdgcn_exp2f(fmaf(s[2 * j], c_row, negm)); };
+      auto exp_y = [&](int j) { py = __builtin_amdgcn_exp2f(fmaf(s[2 * j + 1], c_row, negm)); };
+      auto split_p = [&](int j) {   // keys 2 j, 2 j + 1 of this lane's 16
+        sum[0] += px;
+        sum[1] += py;
+        asm volatile("" : "+v"(sum[0]), "+v"(sum[1]));   // here: summed later, all 16 would stay in registers
+        unsigned hw, lw;
+        split_pair<0>(px, py, px, py, hw, lw);
+        ph[j >> 2][j & 3] = hw;
+        pl[j >> 2][j & 3] = lw;
+        ps[j >> 2][j & 3] = __builtin_bit_cast(
+            unsigned, __builtin_bit_cast(f16x2, hw) * f16x2{(_Float16)4.8828125e-4f, (_Float16)4.8828125e-4f});
+      };
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        u32x4 h, l, hs;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i], c_row, negm));
-          const float y = __builtin_amdgcn_exp2f(fmaf(s[8 * u + 2 * i + 1], c_row, negm));
-          sum[0] += x;
-          sum[1] += y;
-          unsigned hw, lw;
-          split_pair<0>(x, y, x, y, hw, lw);
-          h[i] = hw;
-          l[i] = lw;
-          hs[i] = __builtin_bit_cast(
-              unsigned, __builtin_bit_cast(f16x2, hw) * f16x2{(_Float16)4.8828125e-4f, (_Float16)4.8828125e-4f});
-        }
-        ph[u] = __builtin_bit_cast(f16x8, h);
-        pl[u] = __builtin_bit_cast(f16x8, l);
-        ps[u] = __builtin_bit_cast(f16x8, hs);
+      for (int j = 0; j < 4; ++j) {
+        exp_x(j);
+        exp_y(j);
+        split_p(j);
       }
-      l_run += sum[0] + sum[1];
       __builtin_amdgcn_sched_barrier(0);
-      // O^T += V^T P^T
-      static_for<0, 8>([&](auto i_c) {
-        constexpr int i = decltype(i_c)::value, u = i >> 2, dt = i & 3;
-        if constexpr (i + 2 < 8) read_v(i + 2);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i], ps[u], acc[dt], 0, 0, 0);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], pl[u], acc[dt], 0, 0, 0);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], ph[u], acc[dt], 0, 0, 0);
-        if constexpr (i < 4) {
-          split_v(std::integral_constant<int, 2 * i>{}, nxt);
-          split_v(std::integral_constant<int, 2 * i + 1>{}, nxt);
+      // O^T += V^T P^T: keys 16 u .., two blocks of 32 dims in turn, so that successive sums into one are two rounds apart
+      static_for<0, 24>([&](auto r_c) {
+        constexpr int r = decltype(r_c)::value, u = r / 12, k = r % 12, n = k % 6, dt = 2 * (k / 6) + n % 2, i = 4 * u + dt;
+        if constexpr (n / 2 == 0)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i], __builtin_bit_cast(f16x8, ps[u]), acc[dt], 0, 0, 0);
+        if constexpr (n / 2 == 1)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], __builtin_bit_cast(f16x8, pl[u]), acc[dt], 0, 0, 0);
+        if constexpr (n / 2 == 2)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], __builtin_bit_cast(f16x8, ph[u]), acc[dt], 0, 0, 0);
+        // the next two blocks' operands, each plane into the registers that its last use freed
+        if constexpr ((n == 1 || n == 4) && 4 * u + 2 * (k / 6) + 2 < 8) {
+          constexpr int j = 4 * u + 2 * (k / 6) + 2;
+          if constexpr (n == 1) {
+            vl[j] = read_v(1, j);
+            vl[j + 1] = read_v(1, j + 1);
+          } else {
+            vh[j] = read_v(0, j);
+            vh[j + 1] = read_v(0, j + 1);
+          }
         }
-        if constexpr (i == 3) load_raw(krs, off2);
+        if constexpr (u == 0) {
+          if constexpr (k % 3 == 0) exp_x(4 + k / 3);
+          if constexpr (k % 3 == 1) exp_y(4 + k / 3);
+          if constexpr (k % 3 == 2) split_p(4 + k / 3);
+        } else {
+          if constexpr (k % 3 < 2) split_v(std::integral_constant<int, 2 * (k / 3) + k % 3>{}, nxt);
+        }
+        if constexpr (r == 12) load_raw(krs, rk, off2);
         __builtin_amdgcn_sched_barrier(0);
       });
+      l_run += sum[0] + sum[1];
       __syncthreads();   // this tile has been read, the next one is stored
     };
 
     int e0 = walk_entry(0), e1 = walk_entry(1);
     uint32_t o0 = entry_off(e0);
     auto sub_off = [&](uint32_t o, int sub) -> uint32_t { return o == range ? range : o + sub * sub_bytes; };
-    load_raw(krs, sub_off(o0, 0));
+    load_raw(krs, rk, sub_off(o0, 0));
+    load_raw(vrs, rv, sub_off(o0, 0));
     static_for<0, 8>([&](auto i_c) { split_k(i_c, lds); });
-    load_raw(vrs, sub_off(o0, 0));
     static_for<0, 8>([&](auto i_c) { split_v(i_c, lds); });
-    load_raw(krs, sub_off(o0, 1));
+    load_raw(krs, rk, sub_off(o0, 1));
     __syncthreads();
     for (int b = 0; b < nblocks; ++b) {
       const int n0 = entry_keys(e0);
