@@ -67,6 +67,18 @@ __device__ __forceinline__ unsigned wave_incl_scan(unsigned x) {
   return x;
 }
 
+// inclusive scan over the 64 lanes of a wave of integers, on the DPP moves (no LDS round trips): rows of 16 lanes by shifts
+// of 1, 2, 4 and 8, then lane 15 of each row into the next and lane 31 into the upper half. Every lane active.
+__device__ __forceinline__ int wave_scan_dpp(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 // Logical key block j of the key range -> first token row of that block in the K/V buffer.
 // Plain buffers: plain_key_map() (slot_head 0, capacity 1, slice_blocks 65536 >= Nk) gives row j*128.
 // Ring: block j lives in slot (head + j / s) % capacity at block j % s of that slot.
@@ -133,10 +145,12 @@ struct AttnArgs {
   int kv_ld;                // elements between consecutive K/V token rows: heads * 128 or 128
   int64_t kv_bytes;         // bytes of each of the k and v buffers (the buffer-load range), < 2 GiB
   float c;               // softmax scale * log2(e)
-  int32_t* order;        // (H * nq) rows, longest key list first (bf16 persistent walk; workspace)
+  int32_t* order;        // (H * nq) rows, longest key list first (persistent walk), or the rows' pieces (split rows)
   int32_t* counter;      // per-XCD queue counters of the walk, counter[8 x] for XCD x (workspace, 256 bytes; set by
                          // the order kernel)
-  int pieces;            // > 1: each row's key list is split into that many items (set by launch_attention)
+  int pieces;                   // > 1: each row's key list is split into that many items, in a workgroup each
+  int split_items, split_min;   // split_items > 0: the rows' key lists are split into at most that many items of at least
+                                // split_min blocks, in a workgroup each (set by launch_attention)
   float* part_o;         // workspace of part_items partial results (kPartialFloats each): the accumulators of the items
   float* part_ml;        // (128 x 128 floats each), then their references and sums (2 x 128 floats each)
   int64_t part_items;

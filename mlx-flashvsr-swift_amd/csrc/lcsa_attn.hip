@@ -163,55 +163,164 @@ __device__ __forceinline__ int next_dealt_item(int32_t* counters, int rows) {
   return rows;
 }
 
-// The next item of this workgroup. DIRECT (every item has a workgroup of its own): one item, the XCD-remapped workgroup
-// index. Else the row at its position of the order's first wave, then of its XCD's queue. Called by the whole workgroup;
-// false when nothing is left.
-template <bool DIRECT>
-__device__ __forceinline__ bool next_item(const int32_t* __restrict__ order, int32_t* __restrict__ counter, int rows,
-                                          bool first, int tid, int* item_s, int& item) {
-  if constexpr (DIRECT) {
-    item = xcd_remap(blockIdx.x, gridDim.x);
-    return first;
+constexpr int kMaxSplitItems = 512;   // the partial results of a call: at most 34 MB
+constexpr int kMaxSplitRows = 256;    // rows whose lists are split: a row or two a thread in split_item
+constexpr int kMaxPieces = 32;        // the merge walks a row's pieces one after another
+
+// An item: a row (head-major, 128 queries), or one of the `pieces` pieces of a row's key list: entries [b0, b0 + nblocks).
+struct AttnItem {
+  int row, h, qb, b0, nblocks;
+  int slot, pieces;   // pieces > 1: the item's partial result
+};
+
+// Splits the rows' key lists into at most G pieces of about the same length: T, the most blocks of a piece, is the smallest
+// of 64 candidates from max(min_blocks, longest / kMaxPieces, blocks / G) up to the longest list with sum max(1, ceil(len / T)) <= G
+// (rows <= G, so the last always fits), and a row of n = ceil(len / T) pieces is cut at len p / n. The pieces number the
+// rows in order. Every workgroup finds the same T and then its own piece; a row's first piece leaves (n << 16 | number) in
+// plan[row] for the merge. `sm` is LDS for kMaxSplitRows + 4 x 64 + 8 ints. Called by the whole workgroup of THREADS; false for a
+// workgroup without an item. Costs about a microsecond: one round trip for the lengths and four barriers.
+template <int THREADS>
+__device__ __forceinline__ bool split_item(const AttnArgs& a, const int32_t* __restrict__ kcnt, int rows, int32_t* plan,
+                                           int* sm, AttnItem& it) {
+  constexpr int kWaves = THREADS / 64, kPer = kMaxSplitRows / THREADS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int* const lens = sm;                          // [kMaxSplitRows]
+  int* const cand = sm + kMaxSplitRows;          // [kWaves][64]
+  int* const tot = cand + kWaves * 64;           // [2 kWaves]
+  // thread tid holds rows kPer tid .. kPer tid + kPer - 1 (length 0 past the last row)
+  int len[kPer], sum = 0, mx = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int r = kPer * tid + i;
+    len[i] = r < rows ? max(0, min(kcnt[r], a.nk_stride)) : 0;
+    lens[r] = len[i];
+    sum += len[i];
+    mx = max(mx, len[i]);
   }
-  int p = blockIdx.x;
-  if (!first) {
-    if (tid == 0) *item_s = next_dealt_item(counter, rows);
-    __syncthreads();
-    p = *item_s;
-    __syncthreads();
+  sum = wave_scan_dpp(sum);
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
+  if (lane == 63) {
+    tot[wave] = sum;
+    tot[kWaves + wave] = mx;
   }
-  if (p >= rows) return false;
-  item = order[p];
+  __syncthreads();
+  sum = mx = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    sum += tot[w];
+    mx = max(mx, tot[kWaves + w]);
+  }
+  const int G = a.split_items;
+  const int t0 = max(max(a.split_min, (mx + kMaxPieces - 1) / kMaxPieces), (sum + G - 1) / G);
+  const int dt = max(1, (mx - t0 + 62) / 63);   // t0 + 63 dt >= mx
+  // ceil(len / T) in fp32: floor((len + T - 1/2) / T) is at least 1 / (2 T) from an integer, and len + T < 2^18
+  auto pieces_of = [](int len, float t, float inv) -> int { return max(1, (int)((len + t - 0.5f) * inv)); };
+  const float tc = (float)(t0 + lane * dt), ic = 1.f / tc;
+  // lane l tries T = t0 + l dt; each wave counts the pieces of its own rows
+  int n = 0;
+  const int r_end = min(rows, (wave + 1) * kPer * 64);
+  for (int r = wave * kPer * 64; r < r_end; r += 8) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const i32x4 x = *(const i32x4*)(lens + r), y = *(const i32x4*)(lens + r + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      n += r + e < r_end ? pieces_of(x[e], tc, ic) : 0;
+      n += r + 4 + e < r_end ? pieces_of(y[e], tc, ic) : 0;
+    }
+  }
+  cand[wave * 64 + lane] = n;
+  __syncthreads();
+  n = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) n += cand[w * 64 + lane];
+  const int best = __ffsll((unsigned long long)__ballot(n <= G)) - 1;   // lane 63 fits
+  const int items = __builtin_amdgcn_readlane(n, best);
+  const float T = (float)(t0 + best * dt), iT = 1.f / T;
+  // XCD x (workgroups b with b % 8 = x) takes a contiguous range of the pieces, whose key blocks overlap
+  const int xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
+  const int q = items / kXcds, rem = items % kXcds;
+  const int mine = idx < q + (xcd < rem ? 1 : 0) ? xcd * q + min(xcd, rem) + idx : -1;
+  // the row that holds piece `mine`
+  int c[kPer], csum = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    c[i] = kPer * tid + i < rows ? pieces_of(len[i], T, iT) : 0;
+    csum += c[i];
+  }
+  int at = wave_scan_dpp(csum) - csum;
+  // pieces of the waves before: their candidates' counts
+  for (int w = 0; w < wave; ++w) at += __builtin_amdgcn_readfirstlane(cand[w * 64 + best]);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (mine >= at && mine < at + c[i]) {
+      tot[0] = kPer * tid + i;
+      tot[1] = mine - at;
+      tot[2] = c[i];
+    }
+    at += c[i];
+  }
+  __syncthreads();
+  if (mine < 0) return false;
+  const int row = __builtin_amdgcn_readfirstlane(tot[0]), piece = __builtin_amdgcn_readfirstlane(tot[1]);
+  it.pieces = __builtin_amdgcn_readfirstlane(tot[2]);
+  const int n_row = __builtin_amdgcn_readfirstlane(lens[row]);
+  it.slot = mine;
+  it.row = row;
+  it.h = row / a.nq;
+  it.qb = row - it.h * a.nq;
+  it.b0 = (int)((int64_t)n_row * piece / it.pieces);
+  it.nblocks = (int)((int64_t)n_row * (piece + 1) / it.pieces) - it.b0;
+  if (piece == 0 && tid == 0) plan[row] = it.pieces << 16 | mine;
+  __syncthreads();   // the LDS is free
   return true;
 }
 
-// An item: a row (head-major, 128 queries), or with a.pieces > 1 (DIRECT only) piece `item / rows` of row
-// `item % rows`: entries [b0, b0 + nblocks) of the row's list. Neighbouring items are neighbouring rows' same pieces,
-// whose key blocks overlap.
-struct AttnItem {
-  int row, h, qb, b0, nblocks;
-};
-template <bool DIRECT>
-__device__ __forceinline__ AttnItem attn_item(const AttnArgs& a, const int32_t* __restrict__ kcnt, int rows, int item) {
-  AttnItem it;
-  const int piece = DIRECT ? item / rows : 0;
-  it.row = item - piece * rows;
+// The next item of this workgroup. DIRECT (every item has a workgroup of its own): one item, a piece of the split or the
+// XCD-remapped workgroup index as piece (index / rows of a.pieces) of row (index % rows). Else the row at its position of the order's first wave, then of its XCD's
+// queue. Called by the whole workgroup; false when nothing is left.
+template <bool DIRECT, int THREADS>
+__device__ __forceinline__ bool next_item(const AttnArgs& a, const int32_t* __restrict__ kcnt,
+                                          int32_t* __restrict__ order, int32_t* __restrict__ counter, int rows,
+                                          bool first, int tid, int* item_s, int* sm, AttnItem& it) {
+  if constexpr (DIRECT) {
+    if (a.split_items > 0) return split_item<THREADS>(a, kcnt, rows, order, sm, it);
+    it.slot = xcd_remap(blockIdx.x, gridDim.x);   // neighbouring items: neighbouring rows' same pieces
+    const int piece = it.slot / rows;
+    it.row = it.slot - piece * rows;
+    it.h = it.row / a.nq;
+    it.qb = it.row - it.h * a.nq;
+    it.pieces = a.pieces;
+    const int n = max(0, min(kcnt[it.row], a.nk_stride));
+    it.b0 = (int)((int64_t)n * piece / a.pieces);
+    it.nblocks = (int)((int64_t)n * (piece + 1) / a.pieces) - it.b0;
+    return true;
+  } else {
+    int p = blockIdx.x;
+    if (!first) {
+      if (tid == 0) *item_s = next_dealt_item(counter, rows);
+      __syncthreads();
+      p = *item_s;
+      __syncthreads();
+    }
+    if (p >= rows) return false;
+    it.row = order[p];
+  }
   it.h = it.row / a.nq;
   it.qb = it.row - it.h * a.nq;
-  const int n = max(0, min(kcnt[it.row], a.nk_stride));
-  it.b0 = DIRECT ? (int)((int64_t)n * piece / a.pieces) : 0;
-  it.nblocks = (DIRECT ? (int)((int64_t)n * (piece + 1) / a.pieces) : n) - it.b0;
-  return it;
+  it.b0 = 0;
+  it.nblocks = max(0, min(kcnt[it.row], a.nk_stride));
+  it.pieces = 1;
+  return true;
 }
 
-// An item that lists no block: an unsplit row is zeros (SparseAttention.swift:47-53; DiT.swift:300-304), a piece is a
-// partial result of weight 0.
-template <bool DIRECT, typename T>
-__device__ __forceinline__ void attn_empty_item(const AttnArgs& a, const AttnItem& it, int item, T* __restrict__ O,
-                                                int tid, int threads) {
+// An item that lists no block: a whole row is zeros (SparseAttention.swift:47-53; DiT.swift:300-304), a piece is a partial
+// result of weight 0.
+template <typename T>
+__device__ __forceinline__ void attn_empty_item(const AttnArgs& a, const AttnItem& it, T* __restrict__ O, int tid,
+                                                int threads) {
   constexpr int VN = 16 / sizeof(T), kVecs = kHeadDim / VN;
-  if (DIRECT && a.pieces > 1) {
-    if (tid < kBlock) a.part_ml[(int64_t)item * 2 * kBlock + kBlock + tid] = 0.f;
+  if (it.pieces > 1) {
+    for (int e = tid; e < kBlock; e += threads) a.part_ml[(int64_t)it.slot * 2 * kBlock + kBlock + e] = 0.f;
     return;
   }
   for (int e = tid; e < kBlock * kVecs; e += threads) {
@@ -224,12 +333,12 @@ __device__ __forceinline__ void attn_empty_item(const AttnArgs& a, const AttnIte
 // at acc[dt][4 r4 + e]) from the unnormalised accumulator, the softmax sum l and the reference m (log2 units): the output
 // row, or the piece's partial result in register order (1 KB per store instruction).
 template <bool DIRECT, typename T>
-__device__ __forceinline__ void attn_store(const AttnArgs& a, const AttnItem& it, int item, int group,
+__device__ __forceinline__ void attn_store(const AttnArgs& a, const AttnItem& it, int group,
                                            const f32x16 (&acc)[4], float m, float l, T* __restrict__ O) {
   typedef T Tx4 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
-  if (DIRECT && a.pieces > 1) {
-    float* const po = a.part_o + ((int64_t)item * 4 + group) * (32 * kHeadDim) + 4 * lane;
+  if (DIRECT && it.pieces > 1) {
+    float* const po = a.part_o + ((int64_t)it.slot * 4 + group) * (32 * kHeadDim) + 4 * lane;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       f32x4 v;
@@ -238,7 +347,7 @@ __device__ __forceinline__ void attn_store(const AttnArgs& a, const AttnItem& it
       *(f32x4*)(po + i * 256) = v;
     }
     if (g == 0) {
-      float* const ml = a.part_ml + (int64_t)item * 2 * kBlock + group * 32 + l32;
+      float* const ml = a.part_ml + (int64_t)it.slot * 2 * kBlock + group * 32 + l32;
       ml[0] = m;
       ml[kBlock] = l;
     }
@@ -269,7 +378,7 @@ template <int QG, bool DIRECT>
 __global__ __attribute__((amdgpu_flat_work_group_size(256 / QG, 256 / QG), amdgpu_waves_per_eu(3 - QG, 3 - QG)))
 void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
                       const bf16* __restrict__ Q, bf16* __restrict__ O,
-                      const int32_t* __restrict__ order, int32_t* __restrict__ counter) {
+                      int32_t* __restrict__ order, int32_t* __restrict__ counter) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * kVRing];
   __shared__ int item_s;
 
@@ -287,12 +396,12 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
   // of the second, ...) and, once that queue is empty, of the other XCDs' queues in turn. So the long rows start
   // early, the rows running together on one XCD share key blocks in its L2, and the short ones balance the tail.
   for (bool first = true;; first = false) {
-  int item;
-  if (!next_item<DIRECT>(order, counter, rows, first, tid, &item_s, item)) break;
-  const AttnItem it = attn_item<DIRECT>(a, kcnt, rows, item);
+  AttnItem it;
+  if (!next_item<DIRECT, kThreads>(a, kcnt, order, counter, rows, first, tid, &item_s, (int*)smem, it)) break;
   if (it.nblocks <= 0) {
-    attn_empty_item<DIRECT, bf16>(a, it, item, O, tid, kThreads);
-    continue;
+    attn_empty_item<bf16>(a, it, O, tid, kThreads);
+    if constexpr (DIRECT) break;
+    else continue;
   }
   const int h = it.h, qb = it.qb, nblocks = it.nblocks;
   const int hc = h * kHeadDim;
@@ -708,7 +817,8 @@ void attn_bf16_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_
   }
 
 #pragma unroll
-  for (int q = 0; q < QG; ++q) attn_store<DIRECT, bf16>(a, it, item, wave * QG + q, acc[q], m_ref[q], pair_sum(l_run[q]), O);
+  for (int q = 0; q < QG; ++q) attn_store<DIRECT, bf16>(a, it, wave * QG + q, acc[q], m_ref[q], pair_sum(l_run[q]), O);
+  if constexpr (DIRECT) break;
   }   // next item
 }
 
@@ -925,8 +1035,8 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 //
 // Bound by the matrix cores together with the splits', the softmax's and the operand reads' issue slots (48 MFMAs = 1536
 // cycles, about 240 VALU and 60 LDS instructions a wave and tile). 512 x 512, 12 heads: 192 rows x 32 of 48 blocks (layer call
-// of 2 latent frames over 6) 316 us on the fp32 instructions, 178 with three bf16 parts, 121 now; two-chunk clip 3834, 1458
-// and 918 us. Its error against 64 bits is the smallest of the three: 8.1e-7, 5.3e-7, 4.2e-7 and 1.9e-6, 1.4e-6, 1.1e-6.
+// of 2 latent frames over 6) 316 us on the fp32 instructions, 178 with three bf16 parts, 106 now; two-chunk clip 3834, 1458
+// and 854 us. Its error against 64 bits is the smallest of the three: 8.1e-7, 5.3e-7, 3.8e-7 and 1.9e-6, 1.4e-6, 1.1e-6.
 constexpr int kF32Plane = kTileBytes;              // one fp16 plane of a 32-key tile
 constexpr int kF32Buf = 4 * kF32Plane;             // K planes h, l, then V planes h, l 2^11
 constexpr float kSplitMax = 65000.f;               // the largest scaled element the parts may hold
@@ -1020,7 +1130,7 @@ __device__ __forceinline__ void f32_exact_walk(const AttnArgs& a, int h, int64_t
 template <bool DIRECT>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
 void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
-                     const float* __restrict__ Q, float* __restrict__ O, const int32_t* __restrict__ order,
+                     const float* __restrict__ Q, float* __restrict__ O, int32_t* __restrict__ order,
                      int32_t* __restrict__ counter) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * kF32Buf];
   static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 2 * kF32Buf, "the exact walk's tiles fit");
@@ -1048,12 +1158,12 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
   lds_char* const lds = (lds_char*)(uintptr_t)lds_addr(smem);
 
   for (bool first = true;; first = false) {
-    int item;
-    if (!next_item<DIRECT>(order, counter, rows, first, tid, &item_s, item)) break;
-    const AttnItem it = attn_item<DIRECT>(a, kcnt, rows, item);
+    AttnItem it;
+    if (!next_item<DIRECT, 256>(a, kcnt, order, counter, rows, first, tid, &item_s, (int*)smem, it)) break;
     if (it.nblocks <= 0) {
-      attn_empty_item<DIRECT, float>(a, it, item, O, tid, 256);
-      continue;
+      attn_empty_item<float>(a, it, O, tid, 256);
+      if constexpr (DIRECT) break;
+      else continue;
     }
     const int32_t* __restrict__ klist = kidx + (int64_t)it.row * a.nk_stride + it.b0;
     const int nblocks = it.nblocks;
@@ -1331,7 +1441,8 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[d][r] *= inv;
     }
-    attn_store<DIRECT, float>(a, it, item, wave, acc, m_ref == -INFINITY ? 0.f : m_ref, pair_sum(l_run), O);
+    attn_store<DIRECT, float>(a, it, wave, acc, m_ref == -INFINITY ? 0.f : m_ref, pair_sum(l_run), O);
+    if constexpr (DIRECT) break;
     __syncthreads();   // smem and item_s are free for the next item
   }
 }
@@ -1340,34 +1451,40 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
 // merge of split rows
 // ------------------------------------------------------------------------------------------------------------
 // O of a row split into pieces: sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p, M the largest reference of the pieces
-// that listed a block. One workgroup per 32 queries of a row, one wave per 32 dims; reads 64 KB a piece and row in
-// register order, so it runs at the rate the partial results come out of the caches.
+// with a weight. Pieces of one count have their results `rows` apart, those of split_item one after another (plan: n << 16 |
+// the first piece's number; rows of one piece are written already). One workgroup per 32
+// queries of a row, one wave per 32 dims; reads 64 KB a piece and row in register order, so it runs at the rate the
+// partial results come out of the caches.
 template <typename T>
-__global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, T* __restrict__ O) {
+__global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, const int32_t* __restrict__ plan, T* __restrict__ O) {
   typedef T Tx4 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31, dt = threadIdx.x >> 6;
   const int row = blockIdx.x >> 2, group = blockIdx.x & 3;
   const int rows = a.heads * a.nq;
+  const bool planned = a.split_items > 0;
+  const int pieces = planned ? plan[row] >> 16 : a.pieces, first = planned ? plan[row] & 0xffff : row;
+  if (pieces <= 1) return;
   const int h = row / a.nq, qb = row - h * a.nq;
-  const float* const ml = a.part_ml + (int64_t)row * 2 * kBlock + group * 32 + l32;
-  const float* const po = a.part_o + ((int64_t)row * 4 + group) * (32 * kHeadDim) + 1024 * dt + 4 * lane;
-  const int64_t sml = (int64_t)rows * 2 * kBlock, so = (int64_t)rows * kBlock * kHeadDim;   // piece to piece
+  const float* const ml = a.part_ml + (int64_t)first * 2 * kBlock + group * 32 + l32;
+  const float* const po = a.part_o + ((int64_t)first * 4 + group) * (32 * kHeadDim) + 1024 * dt + 4 * lane;
+  const int64_t ml_step = (int64_t)(planned ? 1 : rows) * 2 * kBlock;   // piece to piece
+  const int64_t o_step = (int64_t)(planned ? 1 : rows) * kBlock * kHeadDim;
   float M = -INFINITY;
 #pragma unroll 4
-  for (int p = 0; p < a.pieces; ++p) {
-    const float m = ml[p * sml];
-    M = fmaxf(M, ml[p * sml + kBlock] != 0.f ? m : -INFINITY);
+  for (int p = 0; p < pieces; ++p) {
+    const float m = ml[p * ml_step];
+    M = fmaxf(M, ml[p * ml_step + kBlock] != 0.f ? m : -INFINITY);
   }
   f32x4 acc[4] = {};
   float l = 0.f;
 #pragma unroll 4
-  for (int p = 0; p < a.pieces; ++p) {
-    const float lp = ml[p * sml + kBlock], sc = __builtin_amdgcn_exp2f(ml[p * sml] - M);
+  for (int p = 0; p < pieces; ++p) {
+    const float lp = ml[p * ml_step + kBlock], sc = __builtin_amdgcn_exp2f(ml[p * ml_step] - M);
     const bool in = lp != 0.f;   // a piece of weight 0 may hold anything
     l += in ? sc * lp : 0.f;
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) {
-      const f32x4 x = *(const f32x4*)(po + p * so + 256 * r4);
+      const f32x4 x = *(const f32x4*)(po + p * o_step + 256 * r4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[r4][e] += in ? sc * x[e] : 0.f;
     }
@@ -1474,23 +1591,29 @@ static int attn_query_groups() {
   return qg;
 }
 
-// Pieces per row. Few rows leave workgroup slots idle and make each row's key list one serial chain, so their lists are
-// split; a piece costs 65 KB of partial result written and read again, and the merge a launch. Measured (12 heads unless
-// said; us a call, unsplit against the pieces chosen):
-//   bf16: one workgroup per CU already runs at 70 % of what two reach together, so the split stops at one item per CU, and
-//   at 4 key blocks an item: 48 rows x 16 blocks 34.4 -> 24.3, 72 x 24 47.9 -> 30.8, 8 (2 heads) x 200 179 -> 30; 108 x 19
-//   31.9 -> 28.0; splitting on to two items per CU is slower (72 x 24 in 7: 34.6, 216 x 18 in 2: 43.1 -> 49.1) until an item
-//   holds about 24 blocks (192 x 64 in 2: 81.2 -> 75.8).
-//   fp32: a block costs 3 times as much, so every slot is filled, down to one block an item: 48 x 16 198 -> 60, 72 x 24
-//   294 -> 101, 216 x 18 226 -> 197, 192 x 64 505 -> 361.
-constexpr int kMaxSplitItems = 512;   // the partial results of a call: at most 34 MB
-constexpr int kMaxPieces = 32;        // the merge walks a row's pieces one after another
-static int split_pieces(int dtype, int64_t rows, int nk, int cus, int64_t max_items) {
-  auto fit = [&](int64_t items, int blocks) -> int64_t {   // pieces of at least `blocks` key blocks within `items`
-    return std::min(std::min(items, max_items) / rows, (int64_t)(nk / blocks));
-  };
-  const int64_t n = dtype == FVSR_DTYPE_BF16 ? std::max(fit(cus, 4), fit(2 * cus, 24)) : fit(2 * cus, 1);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(n, kMaxPieces));
+// How a call's rows are split. Few rows leave workgroup slots idle and make each row's key list one serial chain, so their
+// lists are split into pieces; a piece costs 65 KB of partial result written and read again, and the merge a launch. Measured (12
+// heads, us a call with its merge; whole rows, the rows halved .. in equal pieces, pieces of one length):
+//   bf16, up to half a row per CU: one workgroup per CU already runs at 70 % of what two reach together, so one item per CU of
+//   at least 4 blocks, in equal pieces: planning costs about a microsecond and gains nothing there (48 rows x 16 of 16 blocks
+//   31.4, 21.3, 23.0; 72 x 19 of 24 42.3, 26.4, 28.1; 108 x 9 of 19 31.3, 25.6, 26.9).
+//   bf16, up to a row per CU: two items per CU where lists are long, in pieces of one length of at least 8 blocks (192 rows x
+//   32 of 64 78.8, 72.7, 67.9; x 29 of 48 64.3, 63.5, 64.7); short lists stay whole (216 x 16 of 18 37.3, 44.4).
+//   fp32, where a block costs three times as much: every slot is filled, pieces of one length, down to a block (48 x 16 of 16
+//   100, 44.9, 44.9; 72 x 19 of 24 137, 63.5, 60.1; 108 x 9 of 19 99, 62.1, 55.1; 192 x 29 of 48 208, 186.6, 174.5; 192 x 32 of
+//   64 258, 218.9, 187.6).
+struct SplitRule {
+  int pieces;              // equal pieces of every row (1: whole rows)
+  int items, min_blocks;   // or, if items > 0, pieces of one length (split_item)
+};
+static SplitRule split_rule(int dtype, int64_t rows, int nk, int cus, int64_t max_items) {
+  const int64_t one = std::min<int64_t>(cus, max_items), two = std::min<int64_t>(2 * cus, max_items);
+  if (rows > kMaxSplitRows) return SplitRule{1, 0, 0};
+  if (dtype != FVSR_DTYPE_BF16) return 2 * rows <= two && nk >= 2 ? SplitRule{1, (int)two, 1} : SplitRule{1, 0, 0};
+  if (2 * rows <= one && nk >= 8)
+    return SplitRule{(int)std::min<int64_t>(std::min<int64_t>(one / rows, nk / 4), kMaxPieces), 0, 0};
+  if (2 * rows <= two && nk >= 48) return SplitRule{1, (int)two, 8};
+  return SplitRule{1, 0, 0};
 }
 
 // the most items that attentions over up to `rows` rows and nk key blocks split into
@@ -1504,10 +1627,13 @@ int launch_attention(int dtype, AttnArgs a, hipStream_t stream) {
   const bool half = dtype == FVSR_DTYPE_BF16;
   // two workgroups are resident per CU (64 KB of LDS each in the bf16 walk, 48 KB in the fp32 one)
   const int slots = std::min(2 * device_cus(), kMaxPersistentWgs);
-  a.pieces = split_pieces(dtype, rows, a.nk, device_cus(), a.part_items);
-  a.part_ml = a.part_o + (int64_t)rows * a.pieces * kBlock * kHeadDim;
+  const SplitRule rule = a.order ? split_rule(dtype, rows, a.nk, device_cus(), a.part_items) : SplitRule{1, 0, 0};
+  a.pieces = rule.pieces;
+  a.split_items = rule.items;
+  a.split_min = rule.min_blocks;
+  a.part_ml = a.part_o + a.part_items * kBlock * kHeadDim;
   const bool direct = rows * a.pieces <= slots || !a.order;   // a workgroup per item
-  const dim3 grid(direct ? rows * a.pieces : slots);
+  const dim3 grid(a.split_items > 0 ? a.split_items : direct ? rows * a.pieces : slots);
   if (!direct)
     hipLaunchKernelGGL(attn_order_kernel, dim3(1), dim3(1024), 0, stream, a.kcnt, rows, a.nk_stride, slots, a.order,
                        a.counter);
@@ -1515,22 +1641,22 @@ int launch_attention(int dtype, AttnArgs a, hipStream_t stream) {
     constexpr bool DIRECT = decltype(direct_c)::value;
     if (!half)
       hipLaunchKernelGGL(attn_f32_kernel<DIRECT>, grid, dim3(256), 0, stream, a, a.kidx, a.kcnt, (const float*)a.q,
-                         (float*)a.o, (const int32_t*)a.order, a.counter);
+                         (float*)a.o, a.order, a.counter);
     else if (attn_query_groups() == 2)
       hipLaunchKernelGGL((attn_bf16_kernel<2, DIRECT>), grid, dim3(128), 0, stream, a, a.kidx, a.kcnt,
-                         (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
+                         (const bf16*)a.q, (bf16*)a.o, a.order, a.counter);
     else
       hipLaunchKernelGGL((attn_bf16_kernel<1, DIRECT>), grid, dim3(256), 0, stream, a, a.kidx, a.kcnt,
-                         (const bf16*)a.q, (bf16*)a.o, (const int32_t*)a.order, a.counter);
+                         (const bf16*)a.q, (bf16*)a.o, a.order, a.counter);
   };
   if (direct) walk(std::true_type{});
   else walk(std::false_type{});
   FVSR_HIP_CHECK(hipGetLastError());
-  if (a.pieces > 1) {
+  if (a.split_items > 0 || a.pieces > 1) {
     if (half)
-      hipLaunchKernelGGL(attn_merge_kernel<bf16>, dim3(4 * rows), dim3(256), 0, stream, a, (bf16*)a.o);
+      hipLaunchKernelGGL(attn_merge_kernel<bf16>, dim3(4 * rows), dim3(256), 0, stream, a, a.order, (bf16*)a.o);
     else
-      hipLaunchKernelGGL(attn_merge_kernel<float>, dim3(4 * rows), dim3(256), 0, stream, a, (float*)a.o);
+      hipLaunchKernelGGL(attn_merge_kernel<float>, dim3(4 * rows), dim3(256), 0, stream, a, a.order, (float*)a.o);
     FVSR_HIP_CHECK(hipGetLastError());
   }
   return FVSR_OK;

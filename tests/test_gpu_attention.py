@@ -481,8 +481,8 @@ def test_row_counts_beyond_the_order_kernels_lds(dev, heads, lqb, uniform):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("heads,lqb,nkb", [(1, 1, 3), (1, 1, 130), (3, 5, 8), (2, 9, 50), (12, 16, 26), (16, 16, 25),
-                                           (12, 42, 9)])
+@pytest.mark.parametrize("heads,lqb,nkb", [(1, 1, 3), (1, 1, 130), (3, 5, 8), (2, 9, 50), (12, 16, 26), (12, 16, 50),
+                                           (16, 16, 25), (16, 16, 48), (12, 42, 9)])
 def test_split_key_lists(dev, dtype, heads, lqb, nkb):
     """Rows whose key lists are split over workgroups and merged: one row and 3 or 130 key blocks (the most pieces),
     rows that leave slots over, 256 rows (the last that fp32 splits) and 504 (unsplit). Lists of every length from empty
