@@ -29,6 +29,10 @@ int launch_set_lists(const int32_t* kidx, const int32_t* kcnt, int rows, int nk_
                      int32_t* kcnt_out, hipStream_t stream);
 int launch_scores_softmax(const float* pq, const float* pk, KeyMap kmap, int heads, int C, int nq, int nk, int s,
                           const uint8_t* local, float* probs, unsigned* hist, int q_slices, hipStream_t stream);
+bool select_is_small(int s, int nk);
+int launch_select_small(const float* pq, const float* pk, KeyMap kmap, int heads, int C, int nq, int nk, int s,
+                        const uint8_t* local, int q_slices, int topk, float* probs, float* mask_out, int32_t* kidx,
+                        int32_t* kcnt, hipStream_t stream);
 size_t hist12_bytes(int heads, int q_slices);
 size_t topk_cand_bytes(int heads, int64_t nq);
 int launch_topk_emit(const float* probs, int heads, int nq, int nk, int q_slices, int topk, unsigned* hist,
@@ -263,6 +267,9 @@ static int select_impl(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, con
                                (int64_t)(hist12_bytes(heads, q_slices) / sizeof(unsigned)), stream)))
       return rc;
   }
+  if (select_is_small(s, nk))
+    return launch_select_small(pq, pk, kmap, heads, C, (int)nq, nk, s, local, q_slices, topk, probs_out, mask_out, kidx,
+                               kcnt, stream);
   if ((rc = launch_scores_softmax(pq, pk, kmap, heads, C, (int)nq, nk, s, local, probs, hist, q_slices, stream)))
     return rc;
   return launch_topk_emit(probs, heads, (int)nq, nk, q_slices, topk, hist, (unsigned*)(ws + cv.cand),

@@ -23,6 +23,7 @@
 //                         bin, each workgroup gathers the bin's elements of its share of the row (held in
 //                         registers), and the last to arrive finishes the low 19 bits by three radix passes in LDS
 //                         (full-row 4-pass radix select when the bin is too large)
+//   select_small_kernel  scores, threshold and lists in one launch for rows of up to kSmallProbs probabilities
 //   topk_emit_kernel     one wave per query row: mask and compacted key lists (ballot + popcount),
 //                        the row's probs loaded into registers at once
 #include "common.hpp"
@@ -332,15 +333,15 @@ __device__ __forceinline__ unsigned* thr_ctl(unsigned* hist12, int rows, int row
   return hist12 + (int64_t)rows * kHistBins + 2 * row;
 }
 
-// One radix digit over `count(visit)` of a workgroup of kThrThreads: every (masked) element visited is histogrammed
+// One radix digit over `count(visit)` of a workgroup of THREADS (>= 256, a digit each): every (masked) element visited is histogrammed
 // by its digit (u >> shift) & dmask; the digit holding ascending rank `rank` extends `prefix`, `rank` becomes the
 // rank inside it. Zeros matching the prefix are counted by ballot (they all fall in digit 0).
-template <class Visit>
-__device__ __forceinline__ void radix_digit(unsigned (&hist)[kThrThreads / 64][256], unsigned* tot,
+template <int THREADS, class Visit>
+__device__ __forceinline__ void radix_digit(unsigned (&hist)[THREADS / 64][256], unsigned* tot,
                                             unsigned& prefix, unsigned& rank, unsigned pmask, int shift,
                                             unsigned dmask, Visit&& visit, unsigned* s_prefix, unsigned* s_rank) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  for (int e = tid; e < (kThrThreads / 64) * 256; e += kThrThreads) (&hist[0][0])[e] = 0;
+  for (int e = tid; e < (THREADS / 64) * 256; e += THREADS) (&hist[0][0])[e] = 0;
   __syncthreads();
   unsigned zeros = 0;
   visit([&](unsigned u) {   // called by every lane of the wave together
@@ -351,10 +352,10 @@ __device__ __forceinline__ void radix_digit(unsigned (&hist)[kThrThreads / 64][2
   });
   if (lane == 0 && zeros) atomicAdd(&hist[wave][0], zeros);
   __syncthreads();
-  {
+  if (tid < 256) {
     unsigned c = 0;
 #pragma unroll
-    for (int w = 0; w < kThrThreads / 64; ++w) c += hist[w][tid];
+    for (int w = 0; w < THREADS / 64; ++w) c += hist[w][tid];
     tot[tid] = c;
   }
   __syncthreads();
@@ -390,7 +391,6 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
                                                                      unsigned* __restrict__ hist12,
                                                                      unsigned* __restrict__ cand_ws,
                                                                      float* __restrict__ thr_out) {
-  static_assert(kThrThreads == 256, "the digit scan gives each thread of a 256-thread workgroup one digit");
   __shared__ unsigned hist[kThrThreads / 64][256];
   __shared__ unsigned tot[256];
   __shared__ unsigned wsum[kThrThreads / 64];
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
     const int shifts[3] = {11, 3, 0};
     const unsigned dmasks[3] = {255u, 255u, 7u};
     for (int pass = 0; pass < 3; ++pass) {
-      radix_digit(hist, tot, prefix, rk, pmask, shifts[pass], dmasks[pass], [&](auto&& f) {
+      radix_digit<kThrThreads>(hist, tot, prefix, rk, pmask, shifts[pass], dmasks[pass], [&](auto&& f) {
         for (unsigned b0 = 0; b0 < ncand; b0 += kThrThreads) {
           const unsigned e = b0 + tid;
           f(e < ncand ? cand[e] : 0xffffffffu);
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
     const int shifts[4] = {23, 15, 7, 0};
     for (int pass = 0; pass < 4; ++pass) {
       const unsigned dmask = pass == 3 ? 127u : 255u;
-      radix_digit(hist, tot, prefix, rk, pmask, shifts[pass], dmask, [&](auto&& f) {
+      radix_digit<kThrThreads>(hist, tot, prefix, rk, pmask, shifts[pass], dmask, [&](auto&& f) {
         for (int64_t b0 = 0; b0 < n; b0 += kThrThreads) {
           const int64_t e = b0 + tid;
           f(e < n ? bits[e] : 0xffffffffu);
@@ -625,6 +625,150 @@ __global__ __launch_bounds__(256) void topk_emit_kernel(const float* __restrict_
 }
 
 // ------------------------------------------------------------------------------------------------------------
+// small selections in one launch
+// ------------------------------------------------------------------------------------------------------------
+// Scores, softmax, threshold and lists of one (head, query slice) of up to kSmallProbs probabilities in one workgroup, with
+// the bits of the three kernels above (the same product, sum and divide orders; an exact threshold). Those are latency-bound at
+// these sizes, each a launch and a chain of round trips through the caches; here the only round trip is that of the pooled rows.
+// Bound by that round trip and by barriers; one workgroup a row leaves most of the chip idle, so the rule stops where the
+// general kernels' spread work wins. Selection calls of 12 heads, us (query blocks a slice x key blocks, slices; one launch,
+// three): 16 x 64 17.5, 22.4; 16 x 48, 3 slices 17.3, 31.5; 24 x 96 27.6, 28.5; 2 x 512 54.9, 59.6; 30 x 120 33.9, 30.5; 45 x 90
+// 36.3, 34.8. A 384 x 256 clip of five chunks 328 -> 283.
+constexpr int kSmallProbs = 2048;
+constexpr int kSmallKeys = 512;
+constexpr int kSmallThreads = 512;
+__global__ __launch_bounds__(kSmallThreads) void select_small_kernel(const float* __restrict__ pq,
+                                                                     const float* __restrict__ pk, KeyMap kmap, int C,
+                                                                     int nq, int nk, int s,
+                                                                     const uint8_t* __restrict__ local, int q_slices,
+                                                                     int topk, float* __restrict__ probs,
+                                                                     float* __restrict__ mask_out,
+                                                                     int32_t* __restrict__ kidx,
+                                                                     int32_t* __restrict__ kcnt) {
+  constexpr int kWaves = kSmallThreads / 64;
+  __shared__ float ss[kSmallProbs];   // [s][nk]: scores, then probabilities
+  __shared__ unsigned hist[kWaves][256];
+  __shared__ unsigned tot[256];
+  __shared__ unsigned s_prefix, s_rank;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int li = lane & 15, lg = lane >> 4;
+  const int h = blockIdx.x / q_slices, t = blockIdx.x - h * q_slices;
+  const int n = s * nk;
+  const float sqrt_d = sqrtf((float)kHeadDim);
+  // 16 x 16 tiles of scores over the waves, operands straight from memory, every load of a tile in flight: lane l holds
+  // rows l % 16 of both, dims 32 (l / 16) .. + 31 (rows past the end read the last one and are not stored)
+  const int kt_n = (nk + 15) / 16, tiles = (s + 15) / 16 * kt_n;
+  for (int tile = wave; tile < tiles; tile += kWaves) {
+    const int qt = tile / kt_n, kt = tile - qt * kt_n;
+    const int j = 16 * kt + li;
+    const float* qrow = pq + ((int64_t)t * s + min(16 * qt + li, s - 1)) * C + h * kHeadDim + 32 * lg;
+    const float* krow = pk + (kmap.row(min(j, nk - 1)) / kBlock) * C + h * kHeadDim + 32 * lg;
+    f32x4 qv[8], kv[8];
+    bool see[4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      qv[i] = *(const f32x4*)(qrow + 4 * i);
+      kv[i] = *(const f32x4*)(krow + 4 * i);
+    }
+    const int ksp = min(j, nk - 1) % s;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) see[v] = local[(int64_t)min(16 * qt + 4 * lg + v, s - 1) * s + ksp] != 0;
+    __builtin_amdgcn_sched_barrier(0);   // every load first
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i][e], kv[i][e], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = 16 * qt + 4 * lg + v;
+      if (r < s && j < nk) ss[r * nk + j] = see[v] ? acc[v] / sqrt_d : -INFINITY;
+    }
+  }
+  __syncthreads();
+  // softmax, two rows of a wave side by side
+  for (int r0 = wave; r0 < s; r0 += 2 * kWaves) {
+    float mx[2] = {-INFINITY, -INFINITY}, sum[2] = {0.f, 0.f};
+    float* const row[2] = {ss + r0 * nk, ss + min(r0 + kWaves, s - 1) * nk};
+    const bool two = r0 + kWaves < s;
+    for (int j = lane; j < nk; j += 64) {
+      mx[0] = fmaxf(mx[0], row[0][j]);
+      if (two) mx[1] = fmaxf(mx[1], row[1][j]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      mx[0] = fmaxf(mx[0], __shfl_xor(mx[0], o));
+      mx[1] = fmaxf(mx[1], __shfl_xor(mx[1], o));
+    }
+    for (int j = lane; j < nk; j += 64) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (u == 1 && !two) break;
+        const float ex = expf(row[u][j] - mx[u]);
+        row[u][j] = ex;
+        sum[u] += ex;
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      sum[0] += __shfl_xor(sum[0], o);
+      sum[1] += __shfl_xor(sum[1], o);
+    }
+    for (int j = lane; j < nk; j += 64) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (u == 1 && !two) break;
+        const float p = row[u][j] / sum[u];
+        row[u][j] = p;
+        if (probs) probs[((int64_t)h * nq + (int64_t)t * s + r0 + u * kWaves) * nk + j] = p;
+      }
+    }
+  }
+  // the (k+1)-th largest: four radix digits over the bit patterns
+  const int k = min(n - 1, topk);
+  if (tid == 0) {
+    s_prefix = 0u;
+    s_rank = 0u;
+  }
+  __syncthreads();
+  unsigned prefix = 0u, rk = (unsigned)(n - 1 - k), pmask = 0x80000000u;
+  const int shifts[4] = {23, 15, 7, 0};
+#pragma unroll
+  for (int pass = 0; pass < 4; ++pass) {
+    const unsigned dmask = pass == 3 ? 127u : 255u;
+    radix_digit<kSmallThreads>(hist, tot, prefix, rk, pmask, shifts[pass], dmask, [&](auto&& f) {
+      for (int b0 = 0; b0 < n; b0 += kSmallThreads) {
+        const int e = b0 + tid;
+        f(e < n ? __float_as_uint(ss[e]) & 0x7fffffffu : 0xffffffffu);   // the mask: NaN inputs
+      }
+    }, &s_prefix, &s_rank);
+    pmask |= dmask << shifts[pass];
+  }
+  const float th = __uint_as_float(prefix);
+  // mask and lists, as topk_emit_kernel
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (int r = wave; r < s; r += kWaves) {
+    const int64_t row = (int64_t)h * nq + (int64_t)t * s + r, roff = row * nk;
+    int n_sel = 0;
+    for (int j0 = 0; j0 < nk; j0 += 64) {
+      const int j = j0 + lane;
+      const bool sel = j < nk && ss[r * nk + min(j, nk - 1)] > th;
+      const uint64_t b = __ballot(sel);
+      if (sel) kidx[roff + n_sel + __popcll(b & lt)] = j;
+      if (j < nk && mask_out) mask_out[roff + j] = sel ? 1.f : 0.f;
+      n_sel += __popcll(b);
+    }
+    int n_un = n_sel;
+    for (int j0 = 0; j0 < nk; j0 += 64) {
+      const int j = j0 + lane;
+      const bool un = j < nk && !(ss[r * nk + min(j, nk - 1)] > th);
+      const uint64_t b = __ballot(un);
+      if (un) kidx[roff + n_un + __popcll(b & lt)] = j;
+      n_un += __popcll(b);
+    }
+    if (lane == 0) kcnt[row] = n_sel;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
 // launch
 // ------------------------------------------------------------------------------------------------------------
 // the block means of n (1..3) jobs in one launch (each job's nb is set here from its L); it also clears
@@ -650,6 +794,19 @@ int launch_pool_mean(int dtype, PoolMean* jobs, int n, int C, unsigned* zero, in
   else
     hipLaunchKernelGGL(pool_mean_kernel<float>, grid, dim3(kPoolParts * per), 0, stream, j[0], j[1], j[2], C, zero,
                        nzero);
+  FVSR_HIP_CHECK(hipGetLastError());
+  return FVSR_OK;
+}
+
+// whether a selection of `s` query blocks a slice over nk key blocks runs as one launch (launch_select_small)
+bool select_is_small(int s, int nk) { return nk <= kSmallKeys && (int64_t)s * nk <= kSmallProbs; }
+
+// probs and mask_out may be null; every list entry is written
+int launch_select_small(const float* pq, const float* pk, KeyMap kmap, int heads, int C, int nq, int nk, int s,
+                        const uint8_t* local, int q_slices, int topk, float* probs, float* mask_out, int32_t* kidx,
+                        int32_t* kcnt, hipStream_t stream) {
+  hipLaunchKernelGGL(select_small_kernel, dim3(heads * q_slices), dim3(kSmallThreads), 0, stream, pq, pk, kmap, C, nq,
+                     nk, s, local, q_slices, topk, probs, mask_out, kidx, kcnt);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }

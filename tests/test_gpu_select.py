@@ -243,3 +243,34 @@ def test_threshold_on_exact_ties_in_a_large_bin(dev):
     check_mask(mask, ref_mask, ref_probs, 1, topk)
     check_lists(mask, kidx, kcnt)
     assert int(mask.sum()) == int((ref_probs > tie).sum())
+
+
+@pytest.mark.parametrize("s,nk", [(32, 64), (31, 66), (16, 128), (17, 120), (4, 512), (3, 512), (2, 512), (256, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_small_selection_equals_the_general_one(dev, s, nk, dtype):
+    """Rows of up to 2048 probabilities and 512 key blocks are selected in one launch, with the bits of the three kernels that
+    serve larger ones: the same call with one more key block, of the one window column that the local mask hides, takes the
+    general path. Tail blocks cut short, two query slices; top-k from none through a share to every pair."""
+    gen = torch.Generator(device=dev).manual_seed(s * 1000 + nk)
+    heads, q_slices = 3, 2
+    q = torch.randn((q_slices * s * 128 - 50, heads * 128), generator=gen, device=dev)
+    k = torch.randn(((nk + 1) * 128, heads * 128), generator=gen, device=dev)
+    q += torch.randn((q_slices * s, heads * 128), generator=gen, device=dev).repeat_interleave(128, 0)[:q.shape[0]]
+    k += torch.randn((nk + 1, heads * 128), generator=gen, device=dev).repeat_interleave(128, 0)
+    q, k = q.to(dtype), k.to(dtype)
+    local = np.random.default_rng(nk).random((s, s)) < 0.8
+    local[:, nk % s] = False
+    local[:, (nk + 1) % s] = True      # no row without a visible block: its probabilities are NaN, which equal nothing
+    lk = nk * 128
+    for topk in (0, 1, s * nk // 3, s * nk - 1, s * (nk + 1) + 3):
+        small = fvsr_lcsa.draft_block_mask_and_probs(q, k[:lk], heads, q_slices, s, local, topk)
+        large = fvsr_lcsa.draft_block_mask_and_probs(q, k, heads, q_slices, s, local, topk)
+        assert torch.equal(small[1], large[1][..., :nk]) and bool((large[1][..., nk] == 0).all()), topk
+        if topk != s * nk - 1:   # the zeros of the hidden column are the smallest: the rank counts them only there
+            assert torch.equal(small[0], large[0][..., :nk]), topk
+        check_lists(small[0], small[2], small[3])
+        if topk == s * nk // 3:
+            ref_mask, ref_probs = O.draft_block_mask_and_probs(q.float().cpu().numpy(), k[:lk].float().cpu().numpy(), heads,
+                                                               q_slices, s, local, topk, lq=q.shape[0], lk=lk)
+            assert O.compare(small[1].cpu().numpy(), ref_probs)["rel"] <= 1e-5
+            check_mask(small[0], ref_mask, ref_probs, q_slices, topk)
