@@ -47,11 +47,11 @@ int blas_create(int device, void** out);
 void blas_destroy(void* p);
 int linear_bf16(void* state, const void* x, int64_t L, int K, const void* w, int N, const void* bias, int epilogue,
                 void* y, hipStream_t stream);
-int launch_residual_norm(void* x, const void* y, int gate, int64_t L, int C, float eps, const void* w,
-                         const void* bias, int scale, int shift, const void* mod, const void* t_mod, void* out,
-                         hipStream_t stream);
-int launch_rms_norm(const void* x, int64_t L, int C, float eps, const void* w, void* out, hipStream_t stream,
-                    int list_rows = 0, int nkc = 0, int32_t* kidx = nullptr, int32_t* kcnt = nullptr);
+int launch_modulation(const void* m, const void* t, void* out, int C, hipStream_t stream);
+int launch_residual_norm(void* x, const void* y, const void* gate, int64_t L, int C, float eps, const void* w,
+                         const void* bias, const void* scale, const void* shift, void* out, hipStream_t stream);
+int launch_rms_norm(const void* x, int64_t L, int C, float eps, const void* w, void* out, hipStream_t stream);
+int launch_full_lists(int rows, int nkc, int32_t* kidx, int32_t* kcnt, hipStream_t stream);
 int noalloc_scratch_init(int device);
 int noalloc_scratch(int device, int dtype, AttnArgs& a);
 void rope_tables_host(double theta, float* out);
@@ -814,12 +814,13 @@ static int ensure_block_ws(fvsr_ctx* ctx, size_t bytes) {
 
 // activations of one block call: L tokens of C channels, FFN width F, cross-attention lists for nq query blocks
 struct BlockCarve {
-  size_t in, q, k, v, qw, attn, tmp, ffn, kidx, kcnt, total;
+  size_t mod, in, q, k, v, qw, attn, tmp, ffn, kidx, kcnt, total;
 };
 static BlockCarve block_carve(int64_t L, int C, int F, int64_t nq, int nkc) {
   BlockCarve c;
   size_t off = 0;
   const size_t tok = align256((size_t)L * C * 2);
+  c.mod = off; off += align256((size_t)6 * C * 2);
   c.in = off; off += tok;
   c.q = off; off += tok;
   c.k = off; off += tok;
@@ -920,15 +921,16 @@ int fvsr_dit_block(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const fvsr_dit_blo
   const BlockCarve bc = block_carve(L, C, F, (int64_t)r->heads * nq, nkc);
   if ((rc = ensure_block_ws(ctx, bc.total))) return rc;
   char* ws = (char*)ctx->block_ws;
+  bf16* mod = (bf16*)(ws + bc.mod);
   void *in = ws + bc.in, *q = ws + bc.q, *k = ws + bc.k, *v = ws + bc.v, *qw = ws + bc.qw, *attn = ws + bc.attn;
   void *tmp = ws + bc.tmp, *ffn = ws + bc.ffn;
   int32_t* kidx = (int32_t*)(ws + bc.kidx);
   int32_t* kcnt = (int32_t*)(ws + bc.kcnt);
-  // rows of mod = modulation + t_mod (DiT.swift:495): shift, scale, gate of the self-attention (0..2) and of the FFN (3..5)
-  const void* const m = w->modulation;
+  auto row = [&](int i) -> const void* { return mod + (size_t)i * C; };   // shift/scale/gate MSA, shift/scale/gate MLP
   void* blas = ctx->blas;
-  // inX = norm1(x) * (1 + scaleMSA) + shiftMSA (DiT.swift:496-498)
-  if ((rc = launch_residual_norm(x, nullptr, -1, L, C, eps, nullptr, nullptr, 1, 0, m, t_mod, in, st))) return rc;
+  // mod = modulation + t_mod; inX = norm1(x) * (1 + scaleMSA) + shiftMSA (DiT.swift:495-498)
+  if ((rc = launch_modulation(w->modulation, t_mod, mod, C, st))) return rc;
+  if ((rc = launch_residual_norm(x, nullptr, nullptr, L, C, eps, nullptr, nullptr, row(1), row(0), in, st))) return rc;
   // self-attention: projections, the LCSA layer call (norm + RoPE + partition + ring + select + attend + evict,
   // output in natural order), o projection (DiT.swift:500-539)
   if ((rc = linear_bf16(blas, in, L, C, w->q_weight, C, w->q_bias, 0, q, st))) return rc;
@@ -939,22 +941,23 @@ int fvsr_dit_block(fvsr_ctx* ctx, fvsr_kv_ring* r, int layer, const fvsr_dit_blo
     return rc;
   if ((rc = linear_bf16(blas, attn, L, C, w->o_weight, C, w->o_bias, 0, tmp, st))) return rc;
   // x = x + gateMSA * o; caIn = norm3(x) (affine) (DiT.swift:541-542)
-  if ((rc = launch_residual_norm(x, tmp, 2, L, C, eps, w->norm3_weight, w->norm3_bias, -1, -1, m, t_mod, in, st)))
+  if ((rc = launch_residual_norm(x, tmp, row(2), L, C, eps, w->norm3_weight, w->norm3_bias, nullptr, nullptr, in, st)))
     return rc;
   // cross-attention: q = normQ(q(caIn)); SDPA over the cached context K/V (every context block listed, scale
   // 1/sqrt(128)); o projection (DiT.swift:352-361)
   if ((rc = linear_bf16(blas, in, L, C, w->cross_q_weight, C, w->cross_q_bias, 0, q, st))) return rc;
-  if ((rc = launch_rms_norm(q, L, C, eps, w->cross_norm_q_weight, q, st, (int)(r->heads * nq), nkc, kidx, kcnt))) return rc;
+  if ((rc = launch_rms_norm(q, L, C, eps, w->cross_norm_q_weight, q, st))) return rc;
+  if ((rc = launch_full_lists((int)(r->heads * nq), nkc, kidx, kcnt, st))) return rc;
   if ((rc = fvsr_lcsa_attention(ctx, FVSR_DTYPE_BF16, q, L, w->cross_k, w->cross_v, w->ctx_len, r->heads, kidx, kcnt,
                                 nkc, attn, stream)))
     return rc;
   if ((rc = linear_bf16(blas, attn, L, C, w->cross_o_weight, C, w->cross_o_bias, 0, tmp, st))) return rc;
   // x = x + caOut; inF = norm2(x) * (1 + scaleMLP) + shiftMLP (DiT.swift:545-546)
-  if ((rc = launch_residual_norm(x, tmp, -1, L, C, eps, nullptr, nullptr, 4, 3, m, t_mod, in, st))) return rc;
+  if ((rc = launch_residual_norm(x, tmp, nullptr, L, C, eps, nullptr, nullptr, row(4), row(3), in, st))) return rc;
   // FFN: Linear(C, F) + GELU(tanh) fused, Linear(F, C); x = x + gateMLP * ffn (DiT.swift:547)
   if ((rc = linear_bf16(blas, in, L, C, w->ffn1_weight, F, w->ffn1_bias, 1, ffn, st))) return rc;
   if ((rc = linear_bf16(blas, ffn, L, F, w->ffn2_weight, C, w->ffn2_bias, 0, tmp, st))) return rc;
-  return launch_residual_norm(x, tmp, 5, L, C, eps, nullptr, nullptr, -1, -1, m, t_mod, nullptr, st);
+  return launch_residual_norm(x, tmp, row(5), L, C, eps, nullptr, nullptr, nullptr, nullptr, nullptr, st);
 }
 
 }  // extern "C"

@@ -155,18 +155,12 @@ constexpr int kMaxVecs = 6;   // C <= 64 * 6 * 8 = 3072 channels
 
 __device__ __forceinline__ float rb(float x) { return (float)(bf16)x; }
 
-// Modulation rows (shift / scale / gate): bf16(modulation + t_mod) (DiT.swift:495), formed where they are used: a launch of
-// its own for the six rows took 2.6 us and the gap before it on a 512-token call, the second 16-byte load is hidden here.
-struct ModRow {
-  const bf16 *m, *t;   // C channels each; m null: none
-  __device__ __forceinline__ bf16x8 load(int c) const {
-    const bf16x8 a = *(const bf16x8*)(m + c), b = *(const bf16x8*)(t + c);
-    bf16x8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)a[e] + (float)b[e]);
-    return o;
-  }
-};
+// mod[r * C + c] = bf16(modulation[r * C + c] + t_mod[r * C + c]), 6 rows (DiT.swift:495)
+__global__ void modulation_kernel(const bf16* __restrict__ m, const bf16* __restrict__ t, bf16* __restrict__ out,
+                                  int n) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n) out[e] = (bf16)((float)m[e] + (float)t[e]);
+}
 
 // Per token (row of x, C channels), in this order:
 //   1. residual (y != null): x = bf16(x + bf16(gate * y)) (gate null: x = bf16(x + y)), written back to x
@@ -176,10 +170,11 @@ struct ModRow {
 //        neither: out = bf16(n)
 // The same pass serves x + gate * attn -> norm3, x + ca -> norm2 + modulation, and the final x + gate * ffn.
 __global__ __launch_bounds__(256) void residual_norm_kernel(bf16* __restrict__ x, const bf16* __restrict__ y,
-                                                            ModRow gate, int64_t L, int C, float eps,
-                                                            const bf16* __restrict__ w,
-                                                            const bf16* __restrict__ bias, ModRow scale, ModRow shift,
-                                                            bf16* __restrict__ out) {
+                                                            const bf16* __restrict__ gate, int64_t L, int C,
+                                                            float eps, const bf16* __restrict__ w,
+                                                            const bf16* __restrict__ bias,
+                                                            const bf16* __restrict__ scale,
+                                                            const bf16* __restrict__ shift, bf16* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (n >= L) return;
@@ -193,13 +188,14 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(bf16* __restrict__ x
     u4 v = *(const u4*)(x + n * C + cv * 8);
     if (y) {
       const u4 yv = *(const u4*)(y + n * C + cv * 8);
-      bf16x8 gg = {};
-      if (gate.m) gg = gate.load(cv * 8);
+      u4 gv = u4{0, 0, 0, 0};
+      if (gate) gv = *(const u4*)(gate + cv * 8);
       bf16* a = (bf16*)&v;
       const bf16* yy = (const bf16*)&yv;
+      const bf16* gg = (const bf16*)&gv;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float add = gate.m ? rb((float)gg[e] * (float)yy[e]) : (float)yy[e];
+        const float add = gate ? rb((float)gg[e] * (float)yy[e]) : (float)yy[e];
         a[e] = (bf16)((float)a[e] + add);
       }
       *(u4*)(x + n * C + cv * 8) = v;
@@ -241,8 +237,10 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(bf16* __restrict__ x
       const bf16* bb = (const bf16*)&bv;
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = (bf16)(((float)a[e] - mean) * inv * (float)ww[e] + (float)bb[e]);
-    } else if (scale.m) {
-      const bf16x8 ss = scale.load(cv * 8), hh = shift.load(cv * 8);
+    } else if (scale) {
+      const u4 sv = *(const u4*)(scale + cv * 8), hv = *(const u4*)(shift + cv * 8);
+      const bf16* ss = (const bf16*)&sv;
+      const bf16* hh = (const bf16*)&hv;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float nn = rb(((float)a[e] - mean) * inv);
@@ -256,25 +254,9 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(bf16* __restrict__ x
   }
 }
 
-// Key lists that name every one of nkc context blocks: kcnt[r] = nkc, kidx[r * nkc + j] = j (rows 0: none)
-struct FullLists {
-  int rows, nkc;
-  int32_t *kidx, *kcnt;
-};
-
-// WanRMSNorm over the full width (DiT.swift:34-47), natural order: out = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * w). The
-// launch also writes the lists that the cross-attention over these queries walks (a launch of their own took 1.4 us and the gap
-// before it; a token has 64 threads, its rows * nkc / L list entries are fewer than that for nkc * heads < 8192).
+// WanRMSNorm over the full width (DiT.swift:34-47), natural order: out = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * w)
 __global__ __launch_bounds__(256) void rms_norm_kernel(const bf16* __restrict__ x, int64_t L, int C, float eps,
-                                                       const bf16* __restrict__ w, bf16* __restrict__ out,
-                                                       FullLists lists) {
-  const int64_t entries = (int64_t)lists.rows * lists.nkc;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < entries; e += (int64_t)gridDim.x * 256) {
-    const int64_t row = e / lists.nkc;
-    const int j = (int)(e - row * lists.nkc);
-    lists.kidx[e] = j;
-    if (j == 0) lists.kcnt[row] = lists.nkc;
-  }
+                                                       const bf16* __restrict__ w, bf16* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (n >= L) return;
@@ -307,30 +289,46 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const bf16* __restrict__ 
   }
 }
 
-// gate, scale, shift: rows of `mod` and `t_mod` (C channels each, of the same index), or -1 for none
-int launch_residual_norm(void* x, const void* y, int gate, int64_t L, int C, float eps, const void* w,
-                         const void* bias, int scale, int shift, const void* mod, const void* t_mod, void* out,
-                         hipStream_t stream) {
-  if (L <= 0) return FVSR_OK;
-  if (C % 8 || C / 8 > 64 * kMaxVecs) return set_error(FVSR_ERR_UNSUPPORTED, "norm: channels must be a multiple of 8, <= 3072");
-  auto row = [&](int i) {
-    return i < 0 ? ModRow{nullptr, nullptr}
-                 : ModRow{(const bf16*)mod + (size_t)i * C, (const bf16*)t_mod + (size_t)i * C};
-  };
-  hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)ceil_div(L, 4)), dim3(256), 0, stream, (bf16*)x,
-                     (const bf16*)y, row(gate), L, C, eps, (const bf16*)w, (const bf16*)bias, row(scale), row(shift),
-                     (bf16*)out);
+// every query block lists every context block: kcnt[r] = nkc, kidx[r * nkc + j] = j
+__global__ void full_lists_kernel(int rows, int nkc, int32_t* __restrict__ kidx, int32_t* __restrict__ kcnt) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * nkc) return;
+  kidx[e] = e % nkc;
+  if (e % nkc == 0) kcnt[e / nkc] = nkc;
+}
+
+int launch_modulation(const void* m, const void* t, void* out, int C, hipStream_t stream) {
+  const int n = 6 * C;
+  hipLaunchKernelGGL(modulation_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, (const bf16*)m, (const bf16*)t,
+                     (bf16*)out, n);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }
 
-// list_rows > 0: also kidx / kcnt of list_rows rows that list all of nkc blocks
-int launch_rms_norm(const void* x, int64_t L, int C, float eps, const void* w, void* out, hipStream_t stream,
-                    int list_rows, int nkc, int32_t* kidx, int32_t* kcnt) {
+int launch_residual_norm(void* x, const void* y, const void* gate, int64_t L, int C, float eps, const void* w,
+                         const void* bias, const void* scale, const void* shift, void* out, hipStream_t stream) {
+  if (L <= 0) return FVSR_OK;
+  if (C % 8 || C / 8 > 64 * kMaxVecs) return set_error(FVSR_ERR_UNSUPPORTED, "norm: channels must be a multiple of 8, <= 3072");
+  hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)ceil_div(L, 4)), dim3(256), 0, stream, (bf16*)x,
+                     (const bf16*)y, (const bf16*)gate, L, C, eps, (const bf16*)w, (const bf16*)bias,
+                     (const bf16*)scale, (const bf16*)shift, (bf16*)out);
+  FVSR_HIP_CHECK(hipGetLastError());
+  return FVSR_OK;
+}
+
+int launch_rms_norm(const void* x, int64_t L, int C, float eps, const void* w, void* out, hipStream_t stream) {
   if (L <= 0) return FVSR_OK;
   if (C % 8 || C / 8 > 64 * kMaxVecs) return set_error(FVSR_ERR_UNSUPPORTED, "norm: channels must be a multiple of 8, <= 3072");
   hipLaunchKernelGGL(rms_norm_kernel, dim3((unsigned)ceil_div(L, 4)), dim3(256), 0, stream, (const bf16*)x, L, C, eps,
-                     (const bf16*)w, (bf16*)out, FullLists{list_rows, nkc, kidx, kcnt});
+                     (const bf16*)w, (bf16*)out);
+  FVSR_HIP_CHECK(hipGetLastError());
+  return FVSR_OK;
+}
+
+int launch_full_lists(int rows, int nkc, int32_t* kidx, int32_t* kcnt, hipStream_t stream) {
+  const int n = rows * nkc;
+  if (n <= 0) return FVSR_OK;
+  hipLaunchKernelGGL(full_lists_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, rows, nkc, kidx, kcnt);
   FVSR_HIP_CHECK(hipGetLastError());
   return FVSR_OK;
 }
