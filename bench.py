@@ -29,7 +29,7 @@ for p in (PKG, ROOT):
 METRIC = "block-sparse attn ms/layer-call + effective TFLOP/s (% MFMA peak), 1920×1152"
 HEADLINE = "sparse_1920x1152_bf16"   # the workload METRIC is quoted on; its PMC summary holds the traffic figure
 PEAK_BF16_TFLOPS = 2500.0            # MI355X dense bf16 MFMA
-PEAK_FP32_TFLOPS = 157.3             # MI355X dense fp32 MFMA (the fp32 lane, split on the fp16 matrix cores, can pass it)
+PEAK_FP32_TFLOPS = 157.3             # MI355X dense fp32 MFMA (the fp32 lane, split on the bf16 matrix cores, can pass it)
 PROFILE_PMC = os.path.join(ROOT, "profiles", "lcsa_attn_bf16_1920x1152_pmc.txt")
 
 

@@ -8,7 +8,7 @@
 // queries, two waves per SIMD; K/V tiles of 32 keys reach LDS by direct buffer->LDS copies into 4-slot rings;
 // S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16_bf16 so each lane owns one query row; the softmax keeps a fixed
 // reference per row (see the kernel's comment). fp32 (the parity lane): 4 wave64s x 32 queries, every fp32 operand
-// split into two scaled fp16 parts and multiplied on the fp16 matrix cores, with a lazy online-softmax rescale. In
+// split into three bf16 parts and multiplied on the bf16 matrix cores, with a lazy online-softmax rescale. In
 // both, calls with few rows split the rows' key lists into pieces that a second kernel merges.
 #include <algorithm>
 #include <cstdlib>
@@ -1010,59 +1010,65 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 // ------------------------------------------------------------------------------------------------------------
 // fp32 (parity lane)
 // ------------------------------------------------------------------------------------------------------------
-// The products run on the fp16 matrix cores: every fp32 operand, scaled by a power of two, is split into two fp16 parts
-// h + l (11 + 11 significand bits and l's sign; at most 2^-23 of the value is lost, 2^-25 typically), and a product takes
-// h h + h l + l h, accumulated in fp32. The l l left out is 2^-22 of the product at most, 2^-25 typically, below the rounding
-// of the fp32 sum. Three k = 16 products cost 96 matrix-core cycles per 32 x 32 x 16 block of products, against 512 for the eight
-// k = 2 fp32 ones and 192 for the six of three bf16 parts.
+// The products run on the bf16 matrix cores: every fp32 operand is the exact sum of three bf16 parts (24 significand
+// bits = 8 + 8 + 8, each part the rounded remainder of the ones before it), and a product takes the six partial
+// products above 2^-24 of it, smallest first, accumulated in fp32. The three left out (m l, l m, l l) are 2^-26 of the
+// product at most, below the rounding of the fp32 sum. bf16 has fp32's exponents, so no operand is scaled by its
+// neighbours and the error of a product is relative to that product, whatever else the list holds. Six k = 16 products
+// cost 192 matrix-core cycles per 32 x 32 x 16 block of products, against 512 for the eight k = 2 fp32 ones. (Two fp16 parts
+// and three products would cost 96, but fp16 holds 2^-24 .. 65504 only: under any scale shared by a row, a tile or a
+// list, elements far below the largest lose their bits, also where the largest has no weight in the result.)
 //
-// fp16 holds 2^-24 .. 65504, so every operand is brought to a range where its parts keep their bits:
-//   Q  each row's largest element to 2^13 .. 2^14, exactly (the row's score factor takes the power back)
-//   K  the largest element of the item's first nonzero tile to 2^9 .. 2^10: 64 times as large a one still fits, and what l cannot
-//      hold is 2^-34 of the largest, an absolute error of the scores below their fp32 rounding
-//   V  likewise to 2^7 .. 2^8, 253 times as large a one still fits; l is kept as l 2^11 (multiplied by h 2^-11 of P), so that
-//      channels or tokens down to 2^-20 of the largest keep all their bits
-//   P  2^7 for the first tile's largest, at most 2^15 (the lazy rescale below)
-// An item that meets a larger element, an infinity, or operands outside 2^-60 .. 2^60 is redone on the fp32 matrix cores
-// (f32_exact_walk). NaNs propagate through the parts.
+// At the ends of the range:
+//   magnitudes above 2^59 (infinities among them): the item is redone on the fp32 matrix instructions (f32_exact_walk). Up
+//      to there no partial product or sum of a score that fp32 holds overflows.
+//   V is multiplied by 2^24 before the split, so that every part of the smallest fp32 number is a normal bf16; the
+//      output takes the power back, exactly. Parts of Q and K below 2^-126 may be lost: at most 2^-126 2^59 128 = 2^-60 of a
+//      score, an absolute error that the exponential does not see.
+// NaNs propagate through the parts.
 //
-// A workgroup = 4 wave64s x 32 queries, two per CU (64 KB of tile LDS, at most 256 registers a wave), so that one
-// workgroup's softmax and waits run under the other's products. Keys stream in tiles of 32: a tile's fp32 rows are loaded into
-// registers two tiles ahead (raw buffer loads, rows past the buffer read 0), split once per workgroup between the products of the
-// tile before and stored as two fp16 planes with the 16-byte chunk swizzles of the bf16 walk. K and V planes are double
-// buffered, one barrier a tile. S^T = K Q^T leaves each lane one query's scores; the lazy online softmax is in fp32, and P is
-// split in registers.
+// A workgroup = 4 wave64s x 32 queries, two per CU (48 KB of tile LDS, at most 256 registers a wave), so that one
+// workgroup's softmax and waits run under the other's products. Keys stream in tiles of 32: a tile's fp32 rows are
+// loaded into registers a phase ahead (raw buffer loads, rows past the buffer read 0), split once per workgroup and
+// stored as three bf16 planes with the 16-byte chunk swizzles of the bf16 walk. K and V planes have one buffer each (two
+// would leave one workgroup a CU): V(T) is split and stored between the products of the scores of tile T, K(T+1) between
+// those of its output, with a barrier after each. S^T = K Q^T leaves each lane one query's scores; the lazy online softmax
+// is in fp32, and P is split in registers.
 //
-// Bound by the matrix cores together with the splits', the softmax's and the operand reads' issue slots (48 MFMAs = 1536
-// cycles, about 240 VALU and 60 LDS instructions a wave and tile). 512 x 512, 12 heads: 192 rows x 32 of 48 blocks (layer call
-// of 2 latent frames over 6) 316 us on the fp32 instructions, 178 with three bf16 parts, 106 now; two-chunk clip 3834, 1458
-// and 854 us. Its error against 64 bits is the smallest of the three: 8.1e-7, 5.3e-7, 3.8e-7 and 1.9e-6, 1.4e-6, 1.1e-6.
-constexpr int kF32Plane = kTileBytes;              // one fp16 plane of a 32-key tile
-constexpr int kF32Buf = 4 * kF32Plane;             // K planes h, l, then V planes h, l 2^11
-constexpr float kSplitMax = 65000.f;               // the largest scaled element the parts may hold
-constexpr float kRangeMin = 8.6736174e-19f, kRangeMax = 1.1529215e18f;   // 2^-60, 2^60: operands the scaling serves
-constexpr float kPRef = 7.f, kPGrow = 15.f;        // P is 2^7 at the reference's score; the reference follows past 2^15
+// Bound by the matrix cores: 504 rows x 32 blocks 651 us, 208 TFLOP/s of fp32 products, where six bf16 products at the
+// rate of a large bf16 GEMM would give 228; the splits, the softmax and the operand reads (about 500 VALU and 96 LDS
+// instructions a wave and tile) run under the 96 MFMAs (3072 cycles). 512 x 512, 12 heads, us on the fp32 instructions
+// and now: layer call of 2 latent frames over 6 311, 130; two-chunk clip 3841, 1270 (two scaled fp16 parts: 101 and 838, wrong
+// for the unequal operands named above). Its error against 64 bits is the smallest of the three: 8.1e-7, 3.8e-7 (fp16
+// parts 3.8e-7) and 1.9e-6, 8.7e-7 (1.1e-6).
+constexpr int kF32Plane = kTileBytes;              // one bf16 plane of a 32-key tile
+constexpr float kSplitMax = 5.7646075e17f;         // 2^59: the largest magnitude the split serves
+constexpr float kSplitV = 16777216.f;              // 2^24: V's factor before the split
 constexpr int kExactLd = 132;                      // padded fp32 row of the exact walk's tiles (floats)
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 
-// two values (x 2^S, and x 2^S 2^L in a2, b2) as packed fp16 parts h and l 2^L
-template <int L>
-__device__ __forceinline__ void split_pair(float a, float b, float a2, float b2, unsigned& h, unsigned& l) {
-  const f16x2 hv = __builtin_convertvector(f32x2{a, b}, f16x2);
-  constexpr float kNeg = -(float)(1 << L);
-  const float ra = fmaf((float)hv[0], kNeg, a2), rb = fmaf((float)hv[1], kNeg, b2);
-  h = __builtin_bit_cast(unsigned, hv);
-  l = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{ra, rb}, f16x2));
+// two values as their packed bf16 parts h + m + l
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  auto pack = [](float x, float y) -> unsigned {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
+  };
+  auto lo = [](unsigned u) { return __uint_as_float(u << 16); };
+  auto hi = [](unsigned u) { return __uint_as_float(u & 0xffff0000u); };
+  h = pack(a, b);
+  const float ra = a - lo(h), rb = b - hi(h);
+  m = pack(ra, rb);
+  l = pack(ra - lo(m), rb - hi(m));
 }
 
-// the power of two that brings a magnitude mx (0, or within kRangeMin .. kRangeMax) to 2^(target - 1) .. 2^target; 1 for 0
-__device__ __forceinline__ float scale_to(float mx, int target) {
-  const int e = (int)((__float_as_uint(mx) >> 23) & 255u);   // 2^(e - 127) <= mx < 2^(e - 126)
-  return mx >= kRangeMin && mx <= kRangeMax ? __uint_as_float((unsigned)(target - 1 - (e - 127) + 127) << 23) : 1.f;
+// partial product N (0 .. 5, smallest first) of a k = 16 step: A's parts ah, am, al by B's bh, bm, bl
+template <int N>
+__device__ __forceinline__ void mfma_part(f32x16& acc, const bf16x8& ah, const bf16x8& am, const bf16x8& al,
+                                          const bf16x8& bh, const bf16x8& bm, const bf16x8& bl) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(N == 0 ? al : N == 2 || N == 3 ? am : ah,
+                                                N == 1 ? bl : N == 2 || N == 4 ? bm : bh, acc, 0, 0, 0);
 }
 
 // One item on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), for operands the split cannot hold. Every wave of the
@@ -1132,10 +1138,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t* __restrict__ kcnt,
                      const float* __restrict__ Q, float* __restrict__ O, int32_t* __restrict__ order,
                      int32_t* __restrict__ counter) {
-  __shared__ __attribute__((aligned(1024))) char smem[2 * kF32Buf];
-  static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 2 * kF32Buf, "the exact walk's tiles fit");
+  __shared__ __attribute__((aligned(1024))) char smem[6 * kF32Plane];   // K planes h, m, l, then V planes h, m, l
+  static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 6 * kF32Plane, "the exact walk's tiles fit");
   __shared__ int item_s;
-  __shared__ unsigned tile_max[2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
@@ -1156,6 +1161,7 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
   const int G = lane >> 4, mm = lane & 15, vr = 4 * (G >> 1) + (mm >> 2);
   const int v_off = vr * kRowBytes + (((2 * (G & 1) + ((mm & 3) >> 1)) ^ swz_v(vr)) << 4) + (mm & 1) * 8;
   lds_char* const lds = (lds_char*)(uintptr_t)lds_addr(smem);
+  lds_char* const ldsv = lds + 3 * kF32Plane;
 
   for (bool first = true;; first = false) {
     AttnItem it;
@@ -1180,158 +1186,113 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     };
     const uint32_t sub_bytes = kTileKeys * row_bytes;
     const uint32_t ld_off = r_ld * row_bytes + (uint32_t)(it.h * a.kv_head_stride * 4) + c_ld * 32;
-    f32x4 rk[4], rv[4];   // this thread's part of the K and V tiles to be split next
-    auto load_raw = [&](__amdgpu_buffer_rsrc_t rs, f32x4 (&raw)[4], uint32_t off) {
-      const uint32_t o0 = ld_off + off, o1 = o0 + 16 * row_bytes;   // < 2^31 + 2^18: no wrap
-      raw[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0, 0, 0));
-      raw[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o0 + 16, 0, 0));
-      raw[2] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1, 0, 0));
-      raw[3] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o1 + 16, 0, 0));
+    f32x4 raw[4];   // this thread's part of the K or V tile to be split next
+    // half I: the 8 floats of row r_ld + 16 I. The sum stays below 2^32: a listed block's offset and the head's lie inside
+    // the buffer (< 2^31 bytes), the offset past it is the buffer's size.
+    auto load_half = [&](__amdgpu_buffer_rsrc_t rs, auto i_c, uint32_t off) {
+      constexpr int I = decltype(i_c)::value;
+      const uint32_t o = ld_off + off + I * 16 * row_bytes;
+      raw[2 * I] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0));
+      raw[2 * I + 1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16, 0, 0));
     };
-    auto largest = [](const f32x4 (&raw)[4]) -> float {
-      float m = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(raw[i][e]));
-      return m;
-    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
 
-    // K and V scales from the item's first tile with a nonzero element of theirs: the first tile, but for leading zeros
-    float kmax = 0.f, vmax = 0.f;
-    for (int T = 0; T < 4 * nblocks && (kmax == 0.f || vmax == 0.f); ++T) {
-      const uint32_t off = entry_off(klist[T >> 2]);
-      const uint32_t at = off == range ? range : off + (T & 3) * sub_bytes;
-      if (tid < 2) tile_max[tid] = 0u;
-      __syncthreads();
-      load_raw(krs, rk, at);
-      load_raw(vrs, rv, at);
-      atomicMax(&tile_max[0], __float_as_uint(largest(rk)));   // magnitudes: bit order is value order
-      atomicMax(&tile_max[1], __float_as_uint(largest(rv)));
-      __syncthreads();
-      if (kmax == 0.f) kmax = __uint_as_float(tile_max[0]);
-      if (vmax == 0.f) vmax = __uint_as_float(tile_max[1]);
-      __syncthreads();   // tile_max has been read
-    }
-    auto in_range = [](float m) { return m == 0.f || (m >= kRangeMin && m <= kRangeMax); };
-    bool exact = !in_range(kmax) || !in_range(vmax);
-    const float sk = scale_to(kmax, 10), sv = scale_to(vmax, 8), sv2 = sv * 2048.f;
-    float mag_k = 0.f, mag_v = 0.f;   // largest scaled magnitude this thread split
-
-    // Q as the B operand of S^T = K Q^T, scaled by its row's power of two
-    f16x8 qh[8], ql[8];
-    float c_row;
-    {
-      f32x4 x[16];
-      float m = 0.f;
+    float mag = 0.f;   // largest magnitude this thread split
+    // Q as the B operand of S^T = K Q^T
+    bf16x8 qh[8], qm[8], ql[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        x[2 * t] = x[2 * t + 1] = f32x4{0, 0, 0, 0};
-        if (qrow < a.lq) {
-          const float* p = Q + qrow * a.ld + it.h * kHeadDim + 16 * t + 8 * g;
-          x[2 * t] = *(const f32x4*)p;
-          x[2 * t + 1] = *(const f32x4*)(p + 4);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(x[2 * t][e]), fabsf(x[2 * t + 1][e])));
+    for (int t = 0; t < 8; ++t) {
+      f32x4 x[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+      if (qrow < a.lq) {
+        const float* p = Q + qrow * a.ld + it.h * kHeadDim + 16 * t + 8 * g;
+        x[0] = *(const f32x4*)p;
+        x[1] = *(const f32x4*)(p + 4);
       }
-      m = pair_max(m);
-      exact |= !in_range(m);
-      const float sq = scale_to(m, 14);
-      c_row = a.c / (sq * sk);   // powers of two: exact
+      u32x4 h, m, l;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        u32x4 h, l;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = x[2 * t + (i >> 1)][2 * (i & 1)] * sq, r = x[2 * t + (i >> 1)][2 * (i & 1) + 1] * sq;
-          unsigned hw, lw;
-          split_pair<0>(p, r, p, r, hw, lw);
-          h[i] = hw;
-          l[i] = lw;
-        }
-        qh[t] = __builtin_bit_cast(f16x8, h);
-        ql[t] = __builtin_bit_cast(f16x8, l);
+      for (int i = 0; i < 4; ++i) {
+        const float p = x[i >> 1][2 * (i & 1)], r = x[i >> 1][2 * (i & 1) + 1];
+        unsigned hw, mw, lw;
+        split_pair(p, r, hw, mw, lw);
+        mag = fmaxf(mag, fmaxf(fabsf(p), fabsf(r)));
+        h[i] = hw;
+        m[i] = mw;
+        l[i] = lw;
       }
+      qh[t] = __builtin_bit_cast(bf16x8, h);
+      qm[t] = __builtin_bit_cast(bf16x8, m);
+      ql[t] = __builtin_bit_cast(bf16x8, l);
     }
 
-    // pair I (elements 2 I, 2 I + 1 of this thread's 16) of the raw tile; after pairs 3 and 7 a chunk of 8 is stored
-    u32x4 wh, wl;
-    auto split_k = [&](auto i_c, lds_char* planes) {
+    // pair I (elements 2 I, 2 I + 1 of this thread's 16) of the raw tile, times `scale`; after every other pair half a chunk
+    // is stored at its place of the planes (chunks of rows r_ld and r_ld + 16 at at[0] and at[1])
+    u32x2 wh, wm, wl;
+    auto split_raw = [&](auto i_c, float scale, lds_char* planes, const int (&at)[2]) {
       constexpr int I = decltype(i_c)::value;
-      const float p = rk[I >> 1][2 * (I & 1)] * sk, r = rk[I >> 1][2 * (I & 1) + 1] * sk;
-      unsigned hw, lw;
-      split_pair<0>(p, r, p, r, hw, lw);
-      mag_k = fmaxf(mag_k, fmaxf(fabsf(p), fabsf(r)));
-      asm volatile("" : "+v"(mag_k));   // here: the compiler would keep the elements of a whole block for one late maximum
-      wh[I & 3] = hw;
-      wl[I & 3] = lw;
-      if constexpr ((I & 3) == 3) {
-        *(lds_u32x4*)(planes + st_k[I >> 2]) = wh;
-        *(lds_u32x4*)(planes + kF32Plane + st_k[I >> 2]) = wl;
-      }
-    };
-    auto split_v = [&](auto i_c, lds_char* planes) {
-      constexpr int I = decltype(i_c)::value;
-      const float x = rv[I >> 1][2 * (I & 1)], y = rv[I >> 1][2 * (I & 1) + 1];
-      const float p = x * sv, r = y * sv;
-      unsigned hw, lw;
-      split_pair<11>(p, r, x * sv2, y * sv2, hw, lw);
-      mag_v = fmaxf(mag_v, fmaxf(fabsf(p), fabsf(r)));
-      asm volatile("" : "+v"(mag_v));   // here: the compiler would keep the elements of a whole block for one late maximum
-      wh[I & 3] = hw;
-      wl[I & 3] = lw;
-      if constexpr ((I & 3) == 3) {
-        *(lds_u32x4*)(planes + 2 * kF32Plane + st_v[I >> 2]) = wh;
-        *(lds_u32x4*)(planes + 3 * kF32Plane + st_v[I >> 2]) = wl;
+      const float x = raw[I >> 1][2 * (I & 1)], y = raw[I >> 1][2 * (I & 1) + 1];
+      unsigned hw, mw, lw;
+      split_pair(x * scale, y * scale, hw, mw, lw);
+      mag = fmaxf(mag, fmaxf(fabsf(x), fabsf(y)));
+      asm volatile("" : "+v"(mag));   // here: the compiler would keep the elements of a whole block for one late maximum
+      wh[I & 1] = hw;
+      wm[I & 1] = mw;
+      wl[I & 1] = lw;
+      if constexpr ((I & 1) == 1) {
+        lds_char* const to = planes + at[I >> 2] + (I & 2) * 4;
+        *(lds_u32x2*)to = wh;
+        *(lds_u32x2*)(to + kF32Plane) = wm;
+        *(lds_u32x2*)(to + 2 * kF32Plane) = wl;
       }
     };
 
     f32x16 acc[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) acc[d] = f32x16{};
-    float m_ref = -INFINITY, l_run = 0.f;   // P = exp2(c S - m_ref); the row's largest score so far is about m_ref + 7 .. + 15
+    float m_run = -INFINITY, l_run = 0.f;
 
-    // One tile, in buffer SUB % 2, while the next tile (byte offset off1; its K in rk) is split into the other buffer. 24
-    // rounds of one MFMA each for the scores, then 24 for the output, fenced so that the order below is the issue order: a
-    // wave issues in order and an MFMA holds the matrix core for 32 cycles, so a slice of the other work follows each. K is
-    // split under the last 16 rounds of the scores, the exponentials and the split of P for keys 16 .. 31 run under the first 12
-    // rounds of the output (those of keys 0 .. 15), V is split under the last 12. K of the tile after the next (off2) is
-    // requested half way through the output, V of the next at the start.
-    auto step = [&](auto sub_c, int valid, uint32_t off1, uint32_t off2) {
-      constexpr int SUB = decltype(sub_c)::value;
-      lds_char* const buf = lds + (SUB & 1) * kF32Buf;
-      lds_char* const nxt = lds + ((SUB & 1) ^ 1) * kF32Buf;
-      f16x8 kh[8], kl[8];
-      auto read_k = [&](int t) {
-        lds_char* const p = buf + (k_off ^ (t << 5));
-        kh[t] = *(const lds_f16x8*)p;
-        kl[t] = *(const lds_f16x8*)(p + kF32Plane);
+    // One tile: K is stored, V waits in raw; the next tile is at byte offset off1. 48 rounds of one MFMA each for the
+    // scores, then 48 for the output, fenced so that the order below is the issue order: a wave issues in order and an MFMA
+    // holds the matrix core for 32 cycles, so a slice of the other work follows each. V is split under the scores, K of the
+    // next tile and the second half of P under the output; raw's halves are requested anew as they are split.
+    auto step = [&](int valid, uint32_t off1) {
+      bf16x8 kh[8], km[8], kl[8];
+      auto read_k = [&](int plane, int t) -> bf16x8 {
+        return *(const lds_bf16x8*)(lds + plane * kF32Plane + (k_off ^ (t << 5)));
       };
-      read_k(0);
-      read_k(1);
-      load_raw(vrs, rv, off1);
+      kl[0] = read_k(2, 0);
+      kh[0] = read_k(0, 0);
+      km[0] = read_k(1, 0);
       f32x16 s = f32x16{};
-      static_for<0, 24>([&](auto r_c) {
-        constexpr int r = decltype(r_c)::value, t = r / 3;
-        if constexpr (r % 3 == 0 && t + 2 < 8) read_k(t + 2);
-        if constexpr (r % 3 == 0) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[t], qh[t], s, 0, 0, 0);
-        if constexpr (r % 3 == 1) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], ql[t], s, 0, 0, 0);
-        if constexpr (r % 3 == 2) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[t], qh[t], s, 0, 0, 0);
-        if constexpr (r >= 8 && r % 2 == 0) split_k(std::integral_constant<int, (r - 8) / 2>{}, nxt);
+      // the five small products of every chunk first, then the large ones: only these round at the score's own size
+      static_for<0, 48>([&](auto r_c) {
+        constexpr int r = decltype(r_c)::value, t = r < 40 ? r / 5 : r - 40, n = r < 40 ? r % 5 : 5;
+        // the next chunk's parts, each as late as its latency allows: l and m into the registers that their last use freed
+        if constexpr (r < 40) {
+          if constexpr (n == 1 && t + 1 < 8) kl[t + 1] = read_k(2, t + 1);
+          if constexpr (n == 2) kh[(t + 1) & 7] = read_k(0, (t + 1) & 7);
+          if constexpr (n == 3 && t + 1 < 8) km[t + 1] = read_k(1, t + 1);
+          if constexpr (n == 4 && t == 7) kh[1] = read_k(0, 1);
+        } else if constexpr (t + 2 < 8) {
+          kh[t + 2] = read_k(0, t + 2);
+        }
+        mfma_part<n>(s, kh[t], km[t], kl[t], qh[t], qm[t], ql[t]);
+        if constexpr (r % 6 == 3) split_raw(std::integral_constant<int, r / 6>{}, kSplitV, ldsv, st_v);
+        if constexpr (r == 22) load_half(krs, I0{}, off1);
+        if constexpr (r == 46) load_half(krs, I1{}, off1);
         __builtin_amdgcn_sched_barrier(0);
       });
-      f16x8 vh[8], vl[8];
-      auto read_v = [&](int plane, int i) -> f16x8 {   // i = 4 u + dt: V^T operand of keys 16 u .., dims 32 dt ..
-        lds_char* const pa = buf + (2 + plane) * kF32Plane + (v_off ^ ((i & 3) << 6)) + 16 * (i >> 2) * kRowBytes;
+      __syncthreads();   // K has been read, V is stored
+      bf16x8 vh[8], vm[8], vl[8];
+      auto read_v = [&](int plane, int i) -> bf16x8 {   // i = 4 u + dt: V^T operand of keys 16 u .., dims 32 dt ..
+        lds_char* const pa = ldsv + plane * kF32Plane + (v_off ^ ((i & 3) << 6)) + 16 * (i >> 2) * kRowBytes;
         const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)pa);
         const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pa + 8 * kRowBytes));
-        return __builtin_bit_cast(f16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
       };
-      vl[0] = read_v(1, 0);
-      vl[1] = read_v(1, 1);
+      vl[0] = read_v(2, 0);
       vh[0] = read_v(0, 0);
-      vh[1] = read_v(0, 1);
+      vm[0] = read_v(1, 0);
       if (valid < kTileKeys) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -1340,34 +1301,20 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
       float mx = fmaxf(s[0], s[1]);
 #pragma unroll
       for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
-      const float mxc = pair_max(mx) * c_row;
-      // the lazy rescale: the reference follows only when P would pass 2^15, a wave-uniform branch
-      const bool grow = mxc > m_ref + kPGrow;
-      if (__ballot(grow) != 0) {
-        const float m_new = grow ? mxc - kPRef : m_ref;
-        const float alpha = grow ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;   // m_ref = -inf: 0
-        l_run *= alpha;
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[d][r] *= alpha;
-        m_ref = m_new;
-      }
-      const float negm = m_ref == -INFINITY ? 0.f : -m_ref;
-      u32x4 ph[2], pl[2], ps[2];   // h, l and h 2^-11 of P
+      const float m_use = rescale_if_grown<4>(pair_max(mx) * a.c, m_run, l_run, acc);
+      u32x4 ph[2], pm[2], pl[2];
       float px, py, sum[2] = {0.f, 0.f};
-      auto exp_x = [&](int j) { px = __builtin_amdgcn_exp2f(fmaf(s[2 * j], c_row, negm)); };
-      auto exp_y = [&](int j) { py = __builtin_amdgcn_exp2f(fmaf(s[2 * j + 1], c_row, negm)); };
+      auto exp_x = [&](int j) { px = __builtin_amdgcn_exp2f(fmaf(s[2 * j], a.c, -m_use)); };
+      auto exp_y = [&](int j) { py = __builtin_amdgcn_exp2f(fmaf(s[2 * j + 1], a.c, -m_use)); };
       auto split_p = [&](int j) {   // keys 2 j, 2 j + 1 of this lane's 16
         sum[0] += px;
         sum[1] += py;
         asm volatile("" : "+v"(sum[0]), "+v"(sum[1]));   // here: summed later, all 16 would stay in registers
-        unsigned hw, lw;
-        split_pair<0>(px, py, px, py, hw, lw);
+        unsigned hw, mw, lw;
+        split_pair(px, py, hw, mw, lw);
         ph[j >> 2][j & 3] = hw;
+        pm[j >> 2][j & 3] = mw;
         pl[j >> 2][j & 3] = lw;
-        ps[j >> 2][j & 3] = __builtin_bit_cast(
-            unsigned, __builtin_bit_cast(f16x2, hw) * f16x2{(_Float16)4.8828125e-4f, (_Float16)4.8828125e-4f});
       };
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1376,72 +1323,58 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
         split_p(j);
       }
       __builtin_amdgcn_sched_barrier(0);
-      // O^T += V^T P^T: keys 16 u .., two blocks of 32 dims in turn, so that successive sums into one are two rounds apart
-      static_for<0, 24>([&](auto r_c) {
-        constexpr int r = decltype(r_c)::value, u = r / 12, k = r % 12, n = k % 6, dt = 2 * (k / 6) + n % 2, i = 4 * u + dt;
-        if constexpr (n / 2 == 0)
-          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i], __builtin_bit_cast(f16x8, ps[u]), acc[dt], 0, 0, 0);
-        if constexpr (n / 2 == 1)
-          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], __builtin_bit_cast(f16x8, pl[u]), acc[dt], 0, 0, 0);
-        if constexpr (n / 2 == 2)
-          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i], __builtin_bit_cast(f16x8, ph[u]), acc[dt], 0, 0, 0);
-        // the next two blocks' operands, each plane into the registers that its last use freed
-        if constexpr ((n == 1 || n == 4) && 4 * u + 2 * (k / 6) + 2 < 8) {
-          constexpr int j = 4 * u + 2 * (k / 6) + 2;
-          if constexpr (n == 1) {
-            vl[j] = read_v(1, j);
-            vl[j + 1] = read_v(1, j + 1);
-          } else {
-            vh[j] = read_v(0, j);
-            vh[j + 1] = read_v(0, j + 1);
-          }
+      // O^T += V^T P^T
+      static_for<0, 48>([&](auto r_c) {
+        constexpr int r = decltype(r_c)::value, i = r / 6, u = i / 4, n = r % 6;
+        if constexpr (i + 1 < 8) {
+          if constexpr (n == 1) vl[i + 1] = read_v(2, i + 1);
+          if constexpr (n == 2) vh[i + 1] = read_v(0, i + 1);
+          if constexpr (n == 4) vm[i + 1] = read_v(1, i + 1);
         }
+        mfma_part<n>(acc[i & 3], vh[i], vm[i], vl[i], __builtin_bit_cast(bf16x8, ph[u]),
+                     __builtin_bit_cast(bf16x8, pm[u]), __builtin_bit_cast(bf16x8, pl[u]));
         if constexpr (u == 0) {
-          if constexpr (k % 3 == 0) exp_x(4 + k / 3);
-          if constexpr (k % 3 == 1) exp_y(4 + k / 3);
-          if constexpr (k % 3 == 2) split_p(4 + k / 3);
-        } else {
-          if constexpr (k % 3 < 2) split_v(std::integral_constant<int, 2 * (k / 3) + k % 3>{}, nxt);
+          if constexpr (n == 1) exp_x(4 + i);
+          if constexpr (n == 2) exp_y(4 + i);
+          if constexpr (n == 4) split_p(4 + i);
         }
-        if constexpr (r == 12) load_raw(krs, rk, off2);
+        if constexpr (n == 3) split_raw(std::integral_constant<int, i>{}, 1.f, lds, st_k);
+        if constexpr (r == 22) load_half(vrs, I0{}, off1);
+        if constexpr (r == 46) load_half(vrs, I1{}, off1);
         __builtin_amdgcn_sched_barrier(0);
       });
       l_run += sum[0] + sum[1];
-      __syncthreads();   // this tile has been read, the next one is stored
+      __syncthreads();   // V has been read, K of the next tile is stored
     };
 
     int e0 = walk_entry(0), e1 = walk_entry(1);
     uint32_t o0 = entry_off(e0);
     auto sub_off = [&](uint32_t o, int sub) -> uint32_t { return o == range ? range : o + sub * sub_bytes; };
-    load_raw(krs, rk, sub_off(o0, 0));
-    load_raw(vrs, rv, sub_off(o0, 0));
-    static_for<0, 8>([&](auto i_c) { split_k(i_c, lds); });
-    static_for<0, 8>([&](auto i_c) { split_v(i_c, lds); });
-    load_raw(krs, rk, sub_off(o0, 1));
-    __syncthreads();
+    load_half(krs, I0{}, o0);
+    load_half(krs, I1{}, o0);
+    static_for<0, 8>([&](auto i_c) { split_raw(i_c, 1.f, lds, st_k); });
+    load_half(vrs, I0{}, o0);
+    load_half(vrs, I1{}, o0);
+    __syncthreads();   // K is stored
     for (int b = 0; b < nblocks; ++b) {
       const int n0 = entry_keys(e0);
       const uint32_t o1 = entry_off(e1);
       e0 = e1;
       e1 = walk_entry(b + 2);
-      static_for<0, 4>([&](auto sub_c) {
-        constexpr int SUB = decltype(sub_c)::value;
-        step(sub_c, n0 - SUB * kTileKeys, sub_off(SUB < 3 ? o0 : o1, (SUB + 1) & 3),
-             sub_off(SUB < 2 ? o0 : o1, (SUB + 2) & 3));
-      });
+#pragma nounroll   // one copy of the step: it fills the instruction cache
+      for (int sub = 0; sub < 4; ++sub)
+        step(n0 - sub * kTileKeys, sub_off(sub < 3 ? o0 : o1, (sub + 1) & 3));
       o0 = o1;
     }
-    exact |= !(fmaxf(mag_k, mag_v) <= kSplitMax);
-    if (__syncthreads_or(exact)) {
-      f32_exact_walk(a, it.h, qrow, klist, nblocks, (float*)smem, acc, m_ref, l_run);
+    if (__syncthreads_or(!(mag <= kSplitMax))) {
+      f32_exact_walk(a, it.h, qrow, klist, nblocks, (float*)smem, acc, m_run, l_run);
     } else {
-      const float inv = 1.f / sv;
 #pragma unroll
       for (int d = 0; d < 4; ++d)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[d][r] *= inv;
+        for (int r = 0; r < 16; ++r) acc[d][r] *= 1.f / kSplitV;
     }
-    attn_store<DIRECT, float>(a, it, wave, acc, m_ref == -INFINITY ? 0.f : m_ref, pair_sum(l_run), O);
+    attn_store<DIRECT, float>(a, it, wave, acc, m_run == -INFINITY ? 0.f : m_run, pair_sum(l_run), O);
     if constexpr (DIRECT) break;
     __syncthreads();   // smem and item_s are free for the next item
   }
@@ -1599,9 +1532,9 @@ static int attn_query_groups() {
 //   31.4, 21.3, 23.0; 72 x 19 of 24 42.3, 26.4, 28.1; 108 x 9 of 19 31.3, 25.6, 26.9).
 //   bf16, up to a row per CU: two items per CU where lists are long, in pieces of one length of at least 8 blocks (192 rows x
 //   32 of 64 78.8, 72.7, 67.9; x 29 of 48 64.3, 63.5, 64.7); short lists stay whole (216 x 16 of 18 37.3, 44.4).
-//   fp32, where a block costs three times as much: every slot is filled, pieces of one length, down to a block (48 x 16 of 16
-//   100, 44.9, 44.9; 72 x 19 of 24 137, 63.5, 60.1; 108 x 9 of 19 99, 62.1, 55.1; 192 x 29 of 48 208, 186.6, 174.5; 192 x 32 of
-//   64 258, 218.9, 187.6).
+//   fp32, where a block costs five times as much: every slot is filled, pieces of one length, down to a block (48 x 16 of 16
+//   157, 53, 55; 72 x 19 of 24 212, 92, 77; 108 x 9 of 19 153, 79, 69; 192 x 29 of 48 340, 301, 272; 192 x 32 of 64 423, 356,
+//   300).
 struct SplitRule {
   int pieces;              // equal pieces of every row (1: whole rows)
   int items, min_blocks;   // or, if items > 0, pieces of one length (split_item)

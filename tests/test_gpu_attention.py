@@ -549,10 +549,9 @@ def test_fp32_values_outside_the_split(dev, heads, lqb):
 @pytest.mark.parametrize("what", ["plain", "tiny", "huge", "zero start", "K grows", "V grows", "V outlier first",
                                   "V channels", "Q rows"])
 def test_fp32_operand_scales(dev, what):
-    """The fp32 lane scales K and V by the first nonzero tile of a list and Q by row before it splits them: operands far from
-    1, lists that begin with zeros, magnitudes that grow along the list past what the scale leaves room for (redone on the fp32
-    instructions), a first tile far above the rest, channels and query rows six decades apart. Split rows and whole ones; the
-    error of each output channel relative to its own size, at the lane's bar."""
+    """fp32 operands far from 1, lists that begin with zeros, magnitudes that grow along the list, a first tile far above the
+    rest, channels and query rows six decades apart. Split rows and whole ones; the error of each output channel relative to
+    its own size, at the lane's bar."""
     heads, lqb, nkb = 2, 3, 7
     gen = torch.Generator(device=dev).manual_seed(len(what))
     lq, lk = lqb * 128 - 9, nkb * 128 - 37
@@ -587,3 +586,51 @@ def test_fp32_operand_scales(dev, what):
             ref = torch.softmax(s, -1) @ vv[:, c].double()
             err = (o[:, c].double() - ref).abs().amax(0) / ref.abs().amax(0)
             assert float(err.max()) <= FP32_REL, (h, float(err.max()))
+
+
+@pytest.mark.parametrize("what,size", [("K outlier", 1e6), ("K outlier", 1e9), ("K outlier", 1e12), ("K outlier", 1e17),
+                                       ("K outlier", 1e30), ("K channels", 1e6), ("K channels", 1e12),
+                                       ("V outlier", 1e8), ("V outlier", 1e16), ("V outlier", 1e30),
+                                       ("V channels", 1e5), ("tiny Q and K", 1e-17), ("tiny Q and K", 1e-30),
+                                       ("tiny start", 1e-20), ("subnormal V", 1e-38)])
+def test_fp32_error_is_relative_to_what_counts(dev, what, size):
+    """fp32 operands of very unequal size keep fp32's bits wherever the large ones sit: a key or a V token without weight
+    (every query scores the key about -size / 25) ahead of ordinary ones, q and k channels of opposite size (the same scores),
+    V channels 35 decades apart, q and k whose scores vanish under a ragged last block, a list that begins with near zeros,
+    V at the end of the normal range. Split rows and whole ones; every output channel relative to its own size, at the lane's
+    bar, which leaves an order of magnitude over fp32's own rounding."""
+    heads, lqb, nkb = 2, 3, 7
+    gen = torch.Generator(device=dev).manual_seed(len(what))
+    lq, lk = lqb * 128 - 9, nkb * 128 - 37
+    q, k, v = (torch.randn((n, heads * 128), generator=gen, device=dev) for n in (lq, lk, lk))
+    if what in ("K outlier", "V outlier"):
+        q[:, ::128] = q[:, ::128].abs() + 0.5
+        k[5, ::128] = -(size if what == "K outlier" else 1e5)
+        if what == "V outlier":
+            v[5] = size
+    elif what == "K channels":
+        f = torch.where(torch.arange(heads * 128, device=dev) % 2 == 0, size, 1.0 / size)
+        q, k = q / f, k * f
+    elif what == "V channels":
+        v = v * (size ** -(torch.arange(heads * 128, device=dev) % 8).double()).float()
+    elif what == "tiny Q and K":
+        q, k = q * size, k * size
+    elif what == "tiny start":
+        k[:40] *= size
+        v[:40] *= size
+    elif what == "subnormal V":
+        v = v * size
+    for n in (heads, 256):   # 6 rows (split) and 768 (whole rows, persistent walk)
+        qq, kk, vv = (x if n == heads else x[:, :128].repeat(1, n).contiguous() for x in (q, k, v))
+        m = torch.ones((n, lqb, nkb), device=dev)
+        m[:, 1, 2] = 0.0
+        o = fvsr_lcsa.kernel_block_attention(qq, kk, vv, m, n)
+        keep = m[0].bool().repeat_interleave(128, 0)[:lq].repeat_interleave(128, 1)[:, :lk]
+        for h in (0, n - 1):
+            c = slice(h * 128, (h + 1) * 128)
+            s = (qq[:, c].double() @ kk[:, c].double().t().contiguous() / 128 ** 0.5).masked_fill(~keep, -float("inf"))
+            ref = torch.softmax(s, -1) @ vv[:, c].double()
+            err = (o[:, c].double() - ref).abs().amax(0)
+            # half a unit of the smallest fp32 number, where the result itself is one
+            err = (err - 2.0 ** -149).clamp_min(0.0) / ref.abs().amax(0)
+            assert float(err.max()) <= FP32_REL, (n, h, float(err.max()))
