@@ -311,7 +311,8 @@ __global__ __launch_bounds__(kScoreThreads) void scores_softmax_kernel(const flo
 // exact top-k threshold + mask / list emit
 // ------------------------------------------------------------------------------------------------------------
 // The (k+1)-th largest of each (head, query slice) row of s*Nk probs, k = min(n-1, topk), by an exact select over
-// the fp32 bit patterns (probs are >= 0, so bit order = value order and bit 31 is 0). kThrParts or more workgroups
+// the fp32 bit patterns (probs are >= 0, so bit order = value order and bit 31 is 0; a NaN, of a query block that sees no
+// key block or of NaN inputs, ranks above every number whatever its sign: kValueBits). kThrParts or more workgroups
 // share a row. Each reads the row's top-12-bit histogram (built by scores_softmax_kernel), finds the bin that holds the
 // threshold and its rank in the bin (all of them find the same), then scans its share of the row and gathers the
 // elements of that bin into the row's candidate area of the workspace. The candidates and the arrival count move
@@ -321,6 +322,7 @@ __global__ __launch_bounds__(kScoreThreads) void scores_softmax_kernel(const flo
 // candidate area (e.g. the threshold falls on the exact zeros outside the local window) makes that last workgroup
 // run a full-row radix select from memory instead: exponent [30:23], then mantissa [22:15], [14:7], [6:0], with the
 // zeros counted by a wave ballot instead of 64 colliding LDS atomics.
+constexpr unsigned kValueBits = 0x7fffffffu;
 constexpr int kThrParts = 16;           // workgroups per (head, query slice) row, at least (more for long rows)
 constexpr int kThrMaxParts = 64;
 constexpr int kThrThreads = 256;
@@ -468,13 +470,14 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
   // first, so one atomic per workgroup reserves its slots (a returning device-scope atomic per wave and step would
   // put a memory round trip on every step).
   if (gather) {
+    auto bin_of = [&](unsigned u) { return (u & kValueBits) >> 19; };   // the histogram's bin
     auto in_share = [&](int i) { return e0 + tid + (int64_t)i * kThrThreads < e1; };
     unsigned mine = 0;
     if (in_regs) {
 #pragma unroll
-      for (int i = 0; i < kThrRegs; ++i) mine += (rv[i] >> 19) == bin && in_share(i) ? 1u : 0u;
+      for (int i = 0; i < kThrRegs; ++i) mine += bin_of(rv[i]) == bin && in_share(i) ? 1u : 0u;
     } else {
-      for (int64_t e = e0 + tid; e < e1; e += kThrThreads) mine += (bits[e] >> 19) == bin ? 1u : 0u;
+      for (int64_t e = e0 + tid; e < e1; e += kThrThreads) mine += bin_of(bits[e]) == bin ? 1u : 0u;
     }
     const unsigned minc = wave_incl_scan(mine);
     if (lane == 63) wsum[wave] = minc;
@@ -493,16 +496,16 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
       if (in_regs) {
 #pragma unroll
         for (int i = 0; i < kThrRegs; ++i) {
-          if ((rv[i] >> 19) == bin && in_share(i)) {
-            if (at < cap) __hip_atomic_store(cw + at, rv[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (bin_of(rv[i]) == bin && in_share(i)) {
+            if (at < cap) __hip_atomic_store(cw + at, rv[i] & kValueBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             ++at;
           }
         }
       } else {
         for (int64_t e = e0 + tid; e < e1; e += kThrThreads) {
           const unsigned u = bits[e];
-          if ((u >> 19) == bin) {
-            if (at < cap) __hip_atomic_store(cw + at, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (bin_of(u) == bin) {
+            if (at < cap) __hip_atomic_store(cw + at, u & kValueBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             ++at;
           }
         }
@@ -558,7 +561,7 @@ __global__ __launch_bounds__(kThrThreads) void topk_threshold_kernel(const float
       radix_digit<kThrThreads>(hist, tot, prefix, rk, pmask, shifts[pass], dmask, [&](auto&& f) {
         for (int64_t b0 = 0; b0 < n; b0 += kThrThreads) {
           const int64_t e = b0 + tid;
-          f(e < n ? bits[e] : 0xffffffffu);
+          f(e < n ? bits[e] & kValueBits : 0xffffffffu);
         }
       }, &s_prefix, &s_rank);
       pmask |= dmask << shifts[pass];
@@ -737,7 +740,7 @@ __global__ __launch_bounds__(kSmallThreads) void select_small_kernel(const float
     radix_digit<kSmallThreads>(hist, tot, prefix, rk, pmask, shifts[pass], dmask, [&](auto&& f) {
       for (int b0 = 0; b0 < n; b0 += kSmallThreads) {
         const int e = b0 + tid;
-        f(e < n ? __float_as_uint(ss[e]) & 0x7fffffffu : 0xffffffffu);   // the mask: NaN inputs
+        f(e < n ? __float_as_uint(ss[e]) & kValueBits : 0xffffffffu);
       }
     }, &s_prefix, &s_rank);
     pmask |= dmask << shifts[pass];

@@ -274,3 +274,31 @@ def test_small_selection_equals_the_general_one(dev, s, nk, dtype):
                                                                q_slices, s, local, topk, lq=q.shape[0], lk=lk)
             assert O.compare(small[1].cpu().numpy(), ref_probs)["rel"] <= 1e-5
             check_mask(small[0], ref_mask, ref_probs, q_slices, topk)
+
+
+@pytest.mark.parametrize("s,nk", [(32, 64), (17, 120), (3, 512)])
+def test_small_selection_of_rows_without_a_visible_block(dev, s, nk):
+    """A query block that sees no key block has NaN probabilities, which rank above every other one and are never selected
+    (parity unpinned: the reference's sort order of NaN is its library's). The one-launch selection and the general kernels
+    treat them alike: the general path is the same call with one more, hidden, key block, whose own NaN in that row shifts
+    the rank by one."""
+    gen = torch.Generator(device=dev).manual_seed(s)
+    heads, q_slices = 2, 2
+    q = torch.randn((q_slices * s * 128, heads * 128), generator=gen, device=dev)
+    k = torch.randn(((nk + 1) * 128, heads * 128), generator=gen, device=dev)
+    local = np.random.default_rng(nk).random((s, s)) < 0.8
+    local[:, nk % s] = False
+    local[:, (nk + 1) % s] = True
+    blind = s // 2
+    local[blind] = False
+    lk = nk * 128
+    for topk in (0, nk - 1, nk, nk + 7, s * nk // 2):
+        small = fvsr_lcsa.draft_block_mask_and_probs(q, k[:lk], heads, q_slices, s, local, topk)
+        large = fvsr_lcsa.draft_block_mask_and_probs(q, k, heads, q_slices, s, local, topk + (1 if topk >= nk else 0))
+        assert torch.equal(small[1].isnan(), large[1][..., :nk].isnan())
+        assert bool(small[1][:, [blind, s + blind]].isnan().all())
+        assert torch.equal(small[1].nan_to_num(-1.0), large[1][..., :nk].nan_to_num(-1.0))
+        assert torch.equal(small[0], large[0][..., :nk]), topk
+        assert bool((small[0][:, [blind, s + blind]] == 0).all())
+        assert bool((small[0] > 0).any()) == (topk > nk), topk
+        check_lists(small[0], small[2], small[3])
