@@ -1,7 +1,9 @@
 """GPU parity of the block-sparse attention (lcsa_attn) through the C ABI, against the oracle.
 
 Bars (written in each test): fp32 rel <= 1e-5, bf16 rel <= 1e-2 against the float64 oracle on the same (bf16-valued)
-inputs, rel = max|got - ref| / max|ref| (Gates.swift:19-29). The kernel and its dense fallback must agree exactly.
+inputs, rel = max|got - ref| / max|ref| (Gates.swift:19-29). The dense entry point walks the selected blocks too and must
+return the kernel's bits; where a test says "everywhere", the whole output is held against a float64 softmax over all keys
+with the unselected blocks at -inf.
 The reference's own probe protocol (Diag.swift:86-121: random masks at 0.3-0.6 density with a forced empty query
 block, fp32 and bf16) is reproduced.
 """
@@ -13,6 +15,7 @@ import torch
 
 import fvsr_lcsa
 from fvsr_lcsa import synth
+from gpu_reference import rel_everywhere
 from oracle import lcsa as O
 
 pytestmark = pytest.mark.gpu
@@ -94,7 +97,8 @@ def test_rows_around_the_persistent_grid(dev, heads, lqb, oracle):
     """Row counts (heads x query blocks) just below, just above and twice the persistent grid of the bf16 walk
     (2 workgroups per CU): every workgroup's first row is dealt by XCD, the rest come from the longest-first queue.
     Row lengths vary from empty to full. The outputs start as NaN, so a row the walk skipped or repeated into the
-    wrong place fails; kernel == dense fallback everywhere, and both against the oracle where it is quick."""
+    wrong place fails; both entry points against the float64 masked softmax everywhere, and against the oracle where it is
+    quick."""
     lk = 3 * 128 + 50
     gen = torch.Generator().manual_seed(heads * 1000 + lqb)
     q = torch.randn((lqb * 128, heads * 128), generator=gen).to(torch.bfloat16)
@@ -111,6 +115,7 @@ def test_rows_around_the_persistent_grid(dev, heads, lqb, oracle):
     torch.cuda.synchronize()
     assert not torch.isnan(o).any()
     assert torch.equal(o, od)
+    assert rel_everywhere(od, qd, kd, vd, heads, md) <= BF16_REL
     empty = (m.sum(-1) == 0)                          # (heads, lqb): rows with no listed block are zeros
     ov = o.float().cpu().view(lqb, 128, heads, 128)
     for h, i in empty.nonzero().tolist():
@@ -238,13 +243,15 @@ def _torch_fp32_attention(q, k, v, heads, hsel):
 
 
 def test_c2_full_mask_sparse_equals_dense_bf16(dev):
-    """1280x768 bf16, every block kept: kernel == dense fallback exactly, and both within 1e-2 of torch fp32."""
+    """1280x768 bf16, every block kept: both entry points return the same bits, within 1e-2 of the float64 softmax
+    everywhere and of torch fp32 on two heads."""
     wl = synth.WORKLOADS["dense_1280x768_bf16"]
     q, k, v = synth.make_qkv(wl, seed=0, device=dev)
     m = torch.ones((wl.heads, wl.nq, wl.nk), device=dev)
     o = fvsr_lcsa.kernel_block_attention(q, k, v, m, wl.heads)
     od = fvsr_lcsa.block_masked_attention(q, k, v, m, wl.heads)
     assert torch.equal(o, od)
+    assert rel_everywhere(od, q, k, v, wl.heads, m) <= BF16_REL
     hsel = [0, 7]
     ref = _torch_fp32_attention(q, k, v, wl.heads, hsel)
     got = torch.cat([o[:, h * 128:(h + 1) * 128] for h in hsel], dim=1)
@@ -267,8 +274,8 @@ def _rows_vs_oracle(q, k, v, mask_np, heads, o, pairs):
 
 def test_c2_full_mask_every_head_vs_oracle(dev):
     """1280x768 bf16, every block kept (DiT.swift:279-313 with a full mask): three query blocks of EVERY head (the
-    first, a middle and the last of the 60) against the float64 oracle at rel <= 1e-2, for the sparse kernel and
-    for the dense fallback; the two are equal bit for bit."""
+    first, a middle and the last of the 60) against the float64 oracle at rel <= 1e-2, which holds for the kernel's and
+    the dense entry point's output alike: they are equal bit for bit."""
     wl = synth.WORKLOADS["dense_1280x768_bf16"]
     q, k, v = synth.make_qkv(wl, seed=0, device=dev)
     m = torch.ones((wl.heads, wl.nq, wl.nk), device=dev)
@@ -284,7 +291,8 @@ def test_c2_full_mask_every_head_vs_oracle(dev):
 def test_c4_bf16_subset_vs_oracle(dev):
     """1920x1152 bf16 (Lq 17280, Lk 43200 with a ragged last key block), the oracle's block mask (equal to the
     GPU selection's, which test_gpu_select checks bit for bit): three query blocks of every head against the float64
-    oracle at rel <= 1e-2 (each row non-empty, lists of different lengths), kernel == dense fallback everywhere."""
+    oracle at rel <= 1e-2 (each row non-empty, lists of different lengths), the dense entry point against the float64
+    masked softmax everywhere."""
     wl = synth.WORKLOADS["sparse_1920x1152_bf16"]
     q, k, v = synth.make_qkv(wl)
     local = synth.local_mask(wl).numpy()
@@ -297,6 +305,7 @@ def test_c4_bf16_subset_vs_oracle(dev):
     od = fvsr_lcsa.block_masked_attention(qd, kd, vd, md, wl.heads)
     assert torch.equal(o, od)
     assert torch.isfinite(o.float()).all()
+    assert rel_everywhere(od, qd, kd, vd, wl.heads, md, step=16) <= BF16_REL
     # per head: the query blocks with the shortest and the longest list, and one in the middle of the grid
     kc = mask_np.sum(-1)
     pairs = []
@@ -310,7 +319,7 @@ def test_c4_bf16_subset_vs_oracle(dev):
 def test_c3_bf16_attention_vs_oracle(dev):
     """1280x768 bf16 block-sparse (local range 3, 60% of in-window pairs; tie-free smooth Q/K at the workload's
     seed), the oracle's own mask: two query blocks of every head against the float64 oracle at rel <= 1e-2
-    (DiT.swift:279-313), kernel == dense fallback everywhere."""
+    (DiT.swift:279-313), the dense entry point against the float64 masked softmax everywhere."""
     wl = synth.WORKLOADS["sparse_1280x768_bf16"]
     q, k, v = synth.make_qkv(wl)
     local = synth.local_mask(wl).numpy()
@@ -323,13 +332,14 @@ def test_c3_bf16_attention_vs_oracle(dev):
     o = fvsr_lcsa.kernel_block_attention(qd, kd, vd, md, wl.heads)
     od = fvsr_lcsa.block_masked_attention(qd, kd, vd, md, wl.heads)
     assert torch.equal(o, od)
+    assert rel_everywhere(od, qd, kd, vd, wl.heads, md) <= BF16_REL
     pairs = [(h, b) for h in range(wl.heads) for b in ((7 * h) % wl.nq, (7 * h + 31) % wl.nq)]
     assert _rows_vs_oracle(q, k, v, mask_np, wl.heads, o, pairs) <= BF16_REL
 
 
 def test_c4_iid_workload_subset(dev):
-    """The i.i.d. 1920x1152 workload (960 of 1620 rows select nothing): empty rows are zeros, non-empty rows match
-    the oracle, kernel == dense fallback."""
+    """The i.i.d. 1920x1152 workload (960 of 1620 rows select nothing): empty rows are zeros, some non-empty rows match
+    the oracle, and the dense entry point the float64 masked softmax everywhere."""
     wl = synth.WORKLOADS["sparse_1920x1152_bf16_iid"]
     q, k, v = synth.make_qkv(wl)
     qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
@@ -339,6 +349,7 @@ def test_c4_iid_workload_subset(dev):
     o = fvsr_lcsa.kernel_block_attention(qd, kd, vd, mask, wl.heads)
     od = fvsr_lcsa.block_masked_attention(qd, kd, vd, mask, wl.heads)
     assert torch.equal(o, od)
+    assert rel_everywhere(od, qd, kd, vd, wl.heads, mask, step=16) <= BF16_REL
     kc = kcnt.cpu().numpy()
     ov = o.float().cpu().view(wl.nq, 128, wl.heads, 128)
     empty = np.argwhere(kc == 0)
@@ -355,8 +366,8 @@ def test_reference_raise_on_sharp_scores(dev, density):
     """Scores that grow along the walk far past the first tile's max: key block j is scaled by s_j (0.05 .. 8), so a
     row's logits span about 90 in log2 units and the reference is raised several times per row (each raise rescales
     O and l and recomputes the tile). The scores are scaled in fp32 (a bf16-rounded prescaled Q would misplace the
-    dominant weights by up to 2^0.2 at these magnitudes). bf16 within its bar of the float64 oracle; the kernel
-    equal to the dense fallback (which raises at the same tiles) and to the list entry point, bit for bit."""
+    dominant weights by up to 2^0.2 at these magnitudes). bf16 within its bar of the float64 oracle; the three entry
+    points (mask, dense, lists) return the same bits."""
     heads, lqb, nkb = 2, 3, 6
     gen = torch.Generator().manual_seed(77)
     scale = torch.tensor([0.05, 0.5, 2.0, 4.0, 6.0, 8.0]).repeat_interleave(128).view(-1, 1)
@@ -396,13 +407,16 @@ np.savez(sys.argv[2], o=o.float().cpu().numpy(), od=od.float().cpu().numpy())
 """
 
 
-def test_64_query_waves_equal_32_query_waves(dev, tmp_path):
+@pytest.mark.parametrize("heads,lqb", [(4, 20), (7, 20), (14, 20)])
+def test_64_query_waves_equal_32_query_waves(dev, tmp_path, heads, lqb):
     """The bf16 walk's 64-queries-per-wave lane (FVSR_ATTN_QG=2, one wave per SIMD; read once per process, so it runs
-    in a child) does the same arithmetic per 32-query group as the default lane: kernel and dense walk bit-identical
-    to the default's, on ragged rows with an empty one and listed blocks of every length."""
+    in a child) does the same arithmetic per 32-query group as the default lane: the same bits as the default's, within the
+    bar of the float64 masked softmax everywhere, on ragged rows with an empty one and listed blocks of every length. 80
+    rows are split in equal pieces, 140 in pieces of one length (128 threads plan them here, 256 in the default), 280 are
+    whole (one workgroup each)."""
     import subprocess
     import sys
-    heads, lqb, nkb = 4, 20, 60
+    nkb = 60
     gen = torch.Generator().manual_seed(2024)
     q = torch.randn((lqb * 128 - 37, heads * 128), generator=gen).to(torch.bfloat16)
     k = torch.randn((nkb * 128 - 90, heads * 128), generator=gen).to(torch.bfloat16)
@@ -425,6 +439,7 @@ def test_64_query_waves_equal_32_query_waves(dev, tmp_path):
     assert np.array_equal(z["o"], _np(o))
     assert np.array_equal(z["od"], _np(od))
     assert torch.equal(o, od)
+    assert rel_everywhere(od, qd, kd, vd, heads, md) <= BF16_REL
 
 
 def _rows_vs_torch(q, k, v, m, heads, o, pairs):
@@ -450,8 +465,8 @@ def test_row_counts_beyond_the_order_kernels_lds(dev, heads, lqb, uniform):
     """More rows than the row-order kernel keeps in LDS (8192: the sorted order is staged in the workspace) and, at
     140,000 rows, more than its row-id bitmap covers (131,072: each wave is ranked by scanning its rows). Lists of
     mixed lengths (0 .. 4 blocks) and of one length (2 blocks each: the order is dealt without the sort). Outputs
-    start as NaN, so a row the walk skipped fails; kernel == dense fallback everywhere, empty rows are zeros, and a
-    few rows match a float32 torch softmax."""
+    start as NaN, so a row the walk skipped fails; the dense entry point against the float64 masked softmax everywhere, empty
+    rows are zeros, and a few rows match a float32 torch softmax."""
     lk = 3 * 128 + 50
     g = torch.Generator(device=dev).manual_seed(lqb + int(uniform))
     q = torch.randn((lqb * 128, heads * 128), generator=g, device=dev).to(torch.bfloat16)
@@ -472,6 +487,7 @@ def test_row_counts_beyond_the_order_kernels_lds(dev, heads, lqb, uniform):
     torch.cuda.synchronize()
     assert not torch.isnan(o).any()
     assert torch.equal(o, od)
+    assert rel_everywhere(od, q, k, v, heads, m, step=1024) <= BF16_REL
     empty = (m.sum(-1) == 0).nonzero().tolist()
     ov = o.view(lqb, 128, heads, 128)
     for h, i in empty[:64]:

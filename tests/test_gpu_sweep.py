@@ -9,8 +9,8 @@ most rows have a clear threshold; V is noise.
 Bars, as in test_gpu_select.py and test_gpu_attention.py: probs rel <= 1e-5; the mask bit-exact where the (head,
 query slice) threshold margin exceeds 1e-4, else flips only at the reference's legitimate near-ties
 (Gates.swift:239-277); kcnt / kidx are the mask's lists (SparseAttention.swift:175-177); the attention over the
-GPU's lists against the float64 oracle on the GPU's mask: fp32 rel <= 1e-5, bf16 rel <= 1e-2; the block-sparse
-kernel and the dense fallback agree bit for bit.
+GPU's lists against the float64 oracle on the GPU's mask: fp32 rel <= 1e-5, bf16 rel <= 1e-2; the call from the
+selection's lists and the dense entry point from its mask agree bit for bit.
 """
 import numpy as np
 import pytest
