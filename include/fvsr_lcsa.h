@@ -102,7 +102,7 @@ int fvsr_lcsa_select(fvsr_ctx* ctx, int dtype, const void* qW, int64_t lq, const
  * v per head over the first kcnt[h][i] key blocks listed in kidx[h][i][*] (row stride nk_stride); a query block
  * with kcnt 0 writes zeros. q (lq, H*128), k/v (lk, H*128), o (lq, H*128), all `dtype`. lq, lk need not be
  * multiples of 128: keys past lk are excluded, rows past lq are not written. fp32 operands may have any size; query
- * blocks that meet magnitudes above 2^59 (infinities among them) are computed twice and take several times as long. */
+ * blocks that meet magnitudes above 2^59 (infinities among them) take two to three times as long. */
 int fvsr_lcsa_attention(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
                         int64_t lk, int heads, const int32_t* kidx, const int32_t* kcnt, int nk_stride, void* o,
                         void* stream);

@@ -1020,8 +1020,10 @@ __global__ __launch_bounds__(1024) void attn_order_kernel(const int32_t* __restr
 // list, elements far below the largest lose their bits, also where the largest has no weight in the result.)
 //
 // At the ends of the range:
-//   magnitudes above 2^59 (infinities among them): the item is redone on the fp32 matrix instructions (f32_exact_walk). Up
-//      to there no partial product or sum of a score that fp32 holds overflows.
+//   magnitudes above 2^59 (infinities among them): the walk stops and the item is computed on the fp32 matrix instructions
+//      (f32_exact_walk; 576 rows x 24 blocks with one such key a block 1750 us, where the split takes 630 without them, a whole
+//      walk before the exact one 2300 and a kernel for these instructions alone 1184). Up to there no partial product or sum
+//      of a score that fp32 holds overflows.
 //   V is multiplied by 2^24 before the split, so that every part of the smallest fp32 number is a normal bf16; the
 //      output takes the power back, exactly. Parts of Q and K below 2^-126 may be lost: at most 2^-126 2^59 128 = 2^-60 of a
 //      score, an absolute error that the exponential does not see.
@@ -1141,6 +1143,8 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
   __shared__ __attribute__((aligned(1024))) char smem[6 * kF32Plane];   // K planes h, m, l, then V planes h, m, l
   static_assert(sizeof(float) * 2 * kTileKeys * kExactLd <= 6 * kF32Plane, "the exact walk's tiles fit");
   __shared__ int item_s;
+  __shared__ int huge_s;   // a magnitude above kSplitMax was met: the walk stops after the block
+
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
@@ -1355,6 +1359,7 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
     static_for<0, 8>([&](auto i_c) { split_raw(i_c, 1.f, lds, st_k); });
     load_half(vrs, I0{}, o0);
     load_half(vrs, I1{}, o0);
+    if (tid == 0) huge_s = 0;
     __syncthreads();   // K is stored
     for (int b = 0; b < nblocks; ++b) {
       const int n0 = entry_keys(e0);
@@ -1362,8 +1367,11 @@ void attn_f32_kernel(AttnArgs a, const int32_t* __restrict__ kidx, const int32_t
       e0 = e1;
       e1 = walk_entry(b + 2);
 #pragma nounroll   // one copy of the step: it fills the instruction cache
-      for (int sub = 0; sub < 4; ++sub)
+      for (int sub = 0; sub < 4; ++sub) {
+        if (sub == 2 && !(mag <= kSplitMax)) huge_s = 1;   // barriers on both sides: every wave reads the same below
         step(n0 - sub * kTileKeys, sub_off(sub < 3 ? o0 : o1, (sub + 1) & 3));
+      }
+      if (huge_s != 0) break;
       o0 = o1;
     }
     if (__syncthreads_or(!(mag <= kSplitMax))) {
