@@ -150,7 +150,8 @@ struct AttnArgs {
                          // the order kernel)
   int pieces;                   // > 1: each row's key list is split into that many items, in a workgroup each
   int split_items, split_min;   // split_items > 0: the rows' key lists are split into at most that many items of at least
-                                // split_min blocks, in a workgroup each (set by launch_attention)
+                                // split_min blocks, in a workgroup each (set by launch_attention),
+  int split_slow, split_cost;   // unless the longest list is at most split_slow / 16 pieces + split_cost blocks long
   float* part_o;         // workspace of part_items partial results (kPartialFloats each): the accumulators of the items
   float* part_ml;        // (128 x 128 floats each), then their references and sums (2 x 128 floats each)
   int64_t part_items;

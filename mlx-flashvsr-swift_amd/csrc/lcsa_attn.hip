@@ -175,8 +175,9 @@ struct AttnItem {
 
 // Splits the rows' key lists into at most G pieces of about the same length: T, the most blocks of a piece, is the smallest
 // of 64 candidates from max(min_blocks, longest / kMaxPieces, blocks / G) up to the longest list with sum max(1, ceil(len / T)) <= G
-// (rows <= G, so the last always fits), and a row of n = ceil(len / T) pieces is cut at len p / n. The pieces number the
-// rows in order. Every workgroup finds the same T and then its own piece; a row's first piece leaves (n << 16 | number) in
+// (2 rows <= G, so the last always fits), and a row of n = ceil(len / T) pieces is cut at len p / n. The pieces number the
+// rows in order. Where the longest list is at most split_slow / 16 T + split_cost blocks, pieces do not pay and every row is
+// one. Every workgroup finds the same T and then its own piece; a row's first piece leaves (n << 16 | number) in
 // plan[row] for the merge. `sm` is LDS for kMaxSplitRows + 4 x 64 + 8 ints. Called by the whole workgroup of THREADS; false for a
 // workgroup without an item. Costs about a microsecond: one round trip for the lengths and four barriers.
 template <int THREADS>
@@ -213,7 +214,9 @@ __device__ __forceinline__ bool split_item(const AttnArgs& a, const int32_t* __r
   const int G = a.split_items;
   const int t0 = max(max(a.split_min, (mx + kMaxPieces - 1) / kMaxPieces), (sum + G - 1) / G);
   const int dt = max(1, (mx - t0 + 62) / 63);   // t0 + 63 dt >= mx
-  // ceil(len / T) in fp32: floor((len + T - 1/2) / T) is at least 1 / (2 T) from an integer, and len + T < 2^18
+  // ceil(len / T) in fp32: floor((len + T - 1/2) / T), at least 1 / (2 T) from an integer, so exact up to lists of a million
+  // entries; beyond, a count may be one too many, alike in every workgroup, which the cuts do not mind (the last candidate
+  // still fits: G >= 2 rows)
   auto pieces_of = [](int len, float t, float inv) -> int { return max(1, (int)((len + t - 0.5f) * inv)); };
   const float tc = (float)(t0 + lane * dt), ic = 1.f / tc;
   // lane l tries T = t0 + l dt; each wave counts the pieces of its own rows
@@ -234,8 +237,10 @@ __device__ __forceinline__ bool split_item(const AttnArgs& a, const int32_t* __r
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) n += cand[w * 64 + lane];
   const int best = __ffsll((unsigned long long)__ballot(n <= G)) - 1;   // lane 63 fits
-  const int items = __builtin_amdgcn_readlane(n, best);
-  const float T = (float)(t0 + best * dt), iT = 1.f / T;
+  const int Tb = t0 + best * dt;
+  const bool whole = 16ll * mx <= (int64_t)a.split_slow * Tb + 16 * a.split_cost;
+  const int items = whole ? rows : __builtin_amdgcn_readlane(n, best);
+  const float T = (float)Tb, iT = 1.f / T;
   // XCD x (workgroups b with b % 8 = x) takes a contiguous range of the pieces, whose key blocks overlap
   const int xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
   const int q = items / kXcds, rem = items % kXcds;
@@ -244,12 +249,12 @@ __device__ __forceinline__ bool split_item(const AttnArgs& a, const int32_t* __r
   int c[kPer], csum = 0;
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
-    c[i] = kPer * tid + i < rows ? pieces_of(len[i], T, iT) : 0;
+    c[i] = kPer * tid + i < rows ? (whole ? 1 : pieces_of(len[i], T, iT)) : 0;
     csum += c[i];
   }
   int at = wave_scan_dpp(csum) - csum;
-  // pieces of the waves before: their candidates' counts
-  for (int w = 0; w < wave; ++w) at += __builtin_amdgcn_readfirstlane(cand[w * 64 + best]);
+  // pieces of the waves before: their rows, or their candidates' counts
+  for (int w = 0; w < wave; ++w) at += whole ? kPer * 64 : __builtin_amdgcn_readfirstlane(cand[w * 64 + best]);
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     if (mine >= at && mine < at + c[i]) {
@@ -275,6 +280,9 @@ __device__ __forceinline__ bool split_item(const AttnArgs& a, const int32_t* __r
   return true;
 }
 
+// the pieces of a row that lists n blocks, where rows are cut in a.pieces equal ones: a single block stays whole
+__device__ __forceinline__ int row_pieces(const AttnArgs& a, int n) { return n <= 1 ? 1 : a.pieces; }
+
 // The next item of this workgroup. DIRECT (every item has a workgroup of its own): one item, a piece of the split or the
 // XCD-remapped workgroup index as piece (index / rows of a.pieces) of row (index % rows). Else the row at its position of the order's first wave, then of its XCD's
 // queue. Called by the whole workgroup; false when nothing is left.
@@ -289,11 +297,11 @@ __device__ __forceinline__ bool next_item(const AttnArgs& a, const int32_t* __re
     it.row = it.slot - piece * rows;
     it.h = it.row / a.nq;
     it.qb = it.row - it.h * a.nq;
-    it.pieces = a.pieces;
     const int n = max(0, min(kcnt[it.row], a.nk_stride));
-    it.b0 = (int)((int64_t)n * piece / a.pieces);
-    it.nblocks = (int)((int64_t)n * (piece + 1) / a.pieces) - it.b0;
-    return true;
+    it.pieces = row_pieces(a, n);
+    it.b0 = (int)((int64_t)n * piece / it.pieces);
+    it.nblocks = (int)((int64_t)n * (piece + 1) / it.pieces) - it.b0;
+    return piece < it.pieces;
   } else {
     int p = blockIdx.x;
     if (!first) {
@@ -1405,6 +1413,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, const int32
   const bool planned = a.split_items > 0;
   const int pieces = planned ? plan[row] >> 16 : a.pieces, first = planned ? plan[row] & 0xffff : row;
   if (pieces <= 1) return;
+  const int listed = planned ? 0 : min(a.kcnt[row], a.nk_stride);
   const int h = row / a.nq, qb = row - h * a.nq;
   const float* const ml = a.part_ml + (int64_t)first * 2 * kBlock + group * 32 + l32;
   const float* const po = a.part_o + ((int64_t)first * 4 + group) * (32 * kHeadDim) + 1024 * dt + 4 * lane;
@@ -1416,6 +1425,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, const int32
     const float m = ml[p * ml_step];
     M = fmaxf(M, ml[p * ml_step + kBlock] != 0.f ? m : -INFINITY);
   }
+  if (!planned && row_pieces(a, listed) <= 1) return;   // written already; here, where the count has arrived with the weights
   f32x4 acc[4] = {};
   float l = 0.f;
 #pragma unroll 4
@@ -1535,26 +1545,32 @@ static int attn_query_groups() {
 // How a call's rows are split. Few rows leave workgroup slots idle and make each row's key list one serial chain, so their
 // lists are split into pieces; a piece costs 65 KB of partial result written and read again, and the merge a launch. Measured (12
 // heads, us a call with its merge; whole rows, the rows halved .. in equal pieces, pieces of one length):
-//   bf16, up to half a row per CU: one workgroup per CU already runs at 70 % of what two reach together, so one item per CU of
-//   at least 4 blocks, in equal pieces: planning costs about a microsecond and gains nothing there (48 rows x 16 of 16 blocks
-//   31.4, 21.3, 23.0; 72 x 19 of 24 42.3, 26.4, 28.1; 108 x 9 of 19 31.3, 25.6, 26.9).
+//   bf16, up to half a row per CU: one workgroup per CU already runs at 70 % of what two reach together, so one item per CU,
+//   for every 4 blocks held at most, in equal pieces: planning costs about a microsecond and gains nothing there (48 rows x 16
+//   of 16 blocks 31.4, 21.3, 23.0; 72 x 19 of 24 42.3, 26.4, 28.1; 108 x 9 of 19 31.3, 25.6, 26.9). A row of one block
+//   stays whole (108 rows x 1 of 27 16.4 with an empty piece to merge, 11.8).
 //   bf16, up to a row per CU: two items per CU where lists are long, in pieces of one length of at least 8 blocks (192 rows x
-//   32 of 64 78.8, 72.7, 67.9; x 29 of 48 64.3, 63.5, 64.7); short lists stay whole (216 x 16 of 18 37.3, 44.4).
+//   32 of 64 78.8, 72.7, 67.9); short lists stay whole (216 x 16 of 18 37.3, 44.4). Two items on a CU take 1.8 times as long
+//   a block as one, and the partial results and their merge as long as 5 or 6 blocks, so pieces pay only where they cut the
+//   longest list past that, and split_item keeps the rows whole where they don't (all in pieces, now: lists of one length, 240
+//   rows x 10 of 60 40.1, 32.8; 192 x 16 of 64 45.2, 41.1; 132 x 30 of 60, in pieces still, 52.4, 52.0 and whole 63.7; lists
+//   of about 29 of 48, 192 rows, in pieces still, 65.8, 65.9 and whole 80.9).
 //   fp32, where a block costs five times as much: every slot is filled, pieces of one length, down to a block (48 x 16 of 16
 //   157, 53, 55; 72 x 19 of 24 212, 92, 77; 108 x 9 of 19 153, 79, 69; 192 x 29 of 48 340, 301, 272; 192 x 32 of 64 423, 356,
 //   300).
 struct SplitRule {
   int pieces;              // equal pieces of every row (1: whole rows)
   int items, min_blocks;   // or, if items > 0, pieces of one length (split_item)
+  int slow, cost;          // unless the longest list is at most slow / 16 pieces + cost blocks long
 };
 static SplitRule split_rule(int dtype, int64_t rows, int nk, int cus, int64_t max_items) {
   const int64_t one = std::min<int64_t>(cus, max_items), two = std::min<int64_t>(2 * cus, max_items);
-  if (rows > kMaxSplitRows) return SplitRule{1, 0, 0};
-  if (dtype != FVSR_DTYPE_BF16) return 2 * rows <= two && nk >= 2 ? SplitRule{1, (int)two, 1} : SplitRule{1, 0, 0};
+  if (rows > kMaxSplitRows) return SplitRule{1};
+  if (dtype != FVSR_DTYPE_BF16) return 2 * rows <= two && nk >= 2 ? SplitRule{1, (int)two, 1} : SplitRule{1};
   if (2 * rows <= one && nk >= 8)
-    return SplitRule{(int)std::min<int64_t>(std::min<int64_t>(one / rows, nk / 4), kMaxPieces), 0, 0};
-  if (2 * rows <= two && nk >= 48) return SplitRule{1, (int)two, 8};
-  return SplitRule{1, 0, 0};
+    return SplitRule{(int)std::min<int64_t>(std::min<int64_t>(one / rows, nk / 4), kMaxPieces)};
+  if (2 * rows <= two && nk >= 48) return SplitRule{1, (int)two, 8, 29, 5};
+  return SplitRule{1};
 }
 
 // the most items that attentions over up to `rows` rows and nk key blocks split into
@@ -1568,10 +1584,12 @@ int launch_attention(int dtype, AttnArgs a, hipStream_t stream) {
   const bool half = dtype == FVSR_DTYPE_BF16;
   // two workgroups are resident per CU (64 KB of LDS each in the bf16 walk, 48 KB in the fp32 one)
   const int slots = std::min(2 * device_cus(), kMaxPersistentWgs);
-  const SplitRule rule = a.order ? split_rule(dtype, rows, a.nk, device_cus(), a.part_items) : SplitRule{1, 0, 0};
+  const SplitRule rule = a.order ? split_rule(dtype, rows, a.nk, device_cus(), a.part_items) : SplitRule{1};
   a.pieces = rule.pieces;
   a.split_items = rule.items;
   a.split_min = rule.min_blocks;
+  a.split_slow = rule.slow;
+  a.split_cost = rule.cost;
   a.part_ml = a.part_o + a.part_items * kBlock * kHeadDim;
   const bool direct = rows * a.pieces <= slots || !a.order;   // a workgroup per item
   const dim3 grid(a.split_items > 0 ? a.split_items : direct ? rows * a.pieces : slots);

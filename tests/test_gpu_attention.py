@@ -528,6 +528,26 @@ def test_split_key_lists(dev, dtype, heads, lqb, nkb):
         assert float((o[:, c].double() - ref).abs().max() / ref.abs().max()) <= bar, h
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,lqb,nkb,longest", [(12, 9, 27, 1), (12, 1, 64, 3), (12, 16, 50, 8), (12, 16, 50, 19),
+                                                   (12, 16, 50, 20), (12, 16, 50, 50), (16, 16, 48, 10)])
+def test_split_rows_of_short_lists(dev, dtype, heads, lqb, nkb, longest):
+    """Calls whose keys allow more pieces than their lists have blocks, or whose longest list (of 1 block, of about where
+    pieces begin to pay, of all blocks) decides between whole rows and pieces: the other lists hold up to a third of it, one
+    row none. Every row against the float64 masked softmax, outputs start as NaN."""
+    gen = torch.Generator(device=dev).manual_seed(heads * 1000 + nkb + longest)
+    lq, lk = lqb * 128 - 5, nkb * 128 - 77
+    q, k, v = (torch.randn((n, heads * 128), generator=gen, device=dev).to(dtype) for n in (lq, lk, lk))
+    n = torch.randint(0, longest // 3 + 1, (heads, lqb, 1), generator=gen, device=dev)
+    n[::2, ::3] = longest
+    n[-1, -1] = 0
+    m = (torch.rand((heads, lqb, nkb), generator=gen, device=dev).argsort(-1).argsort(-1) < n).float()
+    o = torch.full_like(q, float("nan"))
+    fvsr_lcsa.kernel_block_attention(q, k, v, m, heads, out=o)
+    bar = BF16_REL if dtype == torch.bfloat16 else FP32_REL
+    assert rel_everywhere(o, q, k, v, heads, m) <= bar
+
+
 @pytest.mark.parametrize("heads,lqb", [(2, 2), (8, 66)])
 def test_fp32_values_outside_the_split(dev, heads, lqb):
     """fp32 operands that the split into 16-bit parts cannot hold: an infinite V column stays infinite and leaves the others alone,
