@@ -41,7 +41,7 @@ typedef enum fvsr_dtype { FVSR_DTYPE_F32 = 0, FVSR_DTYPE_BF16 = 1 } fvsr_dtype;
 /* Attention implementation, mirroring `FlashVSRAttention` (DiT.swift:193-203). `gathered` (2) is not built: the
  * reference documents it as 2-4x slower than dense and keeps it for study only. */
 typedef enum fvsr_attn_mode {
-  FVSR_ATTN_AUTO = 0,    /* kernel when the expected kept fraction <= threshold, else dense (DiT.swift:517-522) */
+  FVSR_ATTN_AUTO = 0,    /* of the layer calls: either (DiT.swift:517-522); their results are the same, so nothing is chosen */
   FVSR_ATTN_DENSE = 1,   /* blockMaskedAttention's result: softmax over all keys, unselected blocks masked */
   FVSR_ATTN_KERNEL = 3   /* only the selected key blocks visited (kernelBlockAttention) */
 } fvsr_attn_mode;
@@ -76,8 +76,9 @@ size_t fvsr_workspace_size(int heads, int64_t lq, int64_t lk, int channels);
  * (kr, kc) visible to query block (qr, qc), i.e. kr in [qr - r/2, qr - r/2 + r - 1] and likewise for columns. */
 int fvsr_local_block_mask(int bh, int bw, int range, uint8_t* out);
 
-/* Expected kept fraction min(1, (topk+1)/(s*nk)) and the `auto` choice against `threshold` (the reference uses
- * 0.45, DiT.swift:210,517-522). HOST function. Returns FVSR_ATTN_KERNEL or FVSR_ATTN_DENSE in *mode. */
+/* Expected kept fraction min(1, (topk+1)/(s*nk)) and the reference's `auto` choice against `threshold` (it uses
+ * 0.45, DiT.swift:210,517-522). HOST function. Returns FVSR_ATTN_KERNEL or FVSR_ATTN_DENSE in *mode: what the
+ * reference would run; here both walk the selected blocks at the same cost. */
 int fvsr_attention_mode_auto(int topk, int s, int nk, double threshold, double* expected, int* mode);
 
 /* ---- (a3 + a7 list build) block selection ----------------------------------------------------------------- */
@@ -123,7 +124,9 @@ int fvsr_lcsa_attention_noalloc(fvsr_ctx* ctx, int dtype, const void* q, int64_t
 /* Replaces `FlashVSRAttentionOps.kernel` / `.dense` (SparseAttention.swift:190-202): attention under a block mask
  * (H, Nq, Nk) f32 tested > 0.5. FVSR_ATTN_DENSE is the dense fallback of
  * `blockMaskedAttention` (DiT.swift:279-313). A masked block's weights are exactly 0, so both modes walk the selected
- * blocks only and return the same values. */
+ * blocks only and return the same values. Unselected blocks are not read: a NaN or an infinity in one does not reach
+ * the output, where a softmax over all keys multiplies it by 0 to a NaN in every row that selects another block. The
+ * ring's mode DENSE and the layer calls do the same. */
 int fvsr_lcsa_attention_mask(fvsr_ctx* ctx, int dtype, const void* q, int64_t lq, const void* k, const void* v,
                              int64_t lk, int heads, const float* block_mask, int mode, void* o, void* stream);
 
@@ -160,7 +163,7 @@ int fvsr_lcsa_attention_ring(fvsr_ctx* ctx, fvsr_kv_ring* ring, int layer, const
                              void* stream);
 
 /* One LCSA layer call — the self-attention core of `blockForward` (DiT.swift:504-538) after the projections:
- * append the chunk's new K/V, select over cache ++ new, attend (mode AUTO uses threshold 0.45 like the reference),
+ * append the chunk's new K/V, select over cache ++ new, attend (any mode: the selected blocks are walked),
  * then evict. qW (lq, C) window order; k_new/v_new as fvsr_kv_ring_append. mask_out/probs_out may be NULL. */
 int fvsr_lcsa_layer(fvsr_ctx* ctx, fvsr_kv_ring* ring, int layer, const void* qW, int64_t lq, const void* k_new,
                     const void* v_new, int n_new_slices, int layout, int q_slices, const uint8_t* local_dev,
@@ -190,7 +193,7 @@ int fvsr_kv_ring_append_qkv(fvsr_kv_ring* ring, int layer, const void* q, const 
 
 /* The LCSA layer call from the projections: the self-attention core of `blockForward` (DiT.swift:496-539) between
  * the q/k/v projections and the o projection. fvsr_kv_ring_append_qkv (normQ/normK + RoPE + window partition +
- * cache append), selection over cache ++ new, attention (mode AUTO: threshold 0.45), evict; the attention output
+ * cache append), selection over cache ++ new, attention (any mode, as above), evict; the attention output
  * is written in natural (f, h, w) token order, i.e. the reference's windowReverse (DiT.swift:121-126,539) is fused
  * into the attention kernel's store. q, k, v: (2*n_new_slices*8bh*8bw, C) projections in natural order; q_work:
  * (same shape) receives q' in window order; o: (same shape) the attention output in natural order. The queries

@@ -1582,7 +1582,7 @@ int launch_attention(int dtype, AttnArgs a, hipStream_t stream) {
   const int rows = a.heads * a.nq;
   if (rows <= 0) return FVSR_OK;
   const bool half = dtype == FVSR_DTYPE_BF16;
-  // two workgroups are resident per CU (64 KB of LDS each in the bf16 walk, 48 KB in the fp32 one)
+  // two workgroups are resident per CU (64 KB of LDS each in the bf16 walk, 48 in the fp32 one; two waves per SIMD)
   const int slots = std::min(2 * device_cus(), kMaxPersistentWgs);
   const SplitRule rule = a.order ? split_rule(dtype, rows, a.nk, device_cus(), a.part_items) : SplitRule{1};
   a.pieces = rule.pieces;

@@ -183,7 +183,8 @@ def local_block_mask(bh: int, bw: int, r: int) -> np.ndarray:
 
 
 def attention_mode_auto(topk: int, s: int, nk: int, threshold: float = 0.45):
-    """(expected kept fraction, ATTN_KERNEL | ATTN_DENSE): the `auto` rule of DiT.swift:517-522."""
+    """(expected kept fraction, ATTN_KERNEL | ATTN_DENSE): the `auto` rule of DiT.swift:517-522. The layer calls return
+    the same in every mode: they walk the selected blocks."""
     e = C.c_double()
     m = C.c_int()
     call("fvsr_attention_mode_auto", topk, s, nk, threshold, C.byref(e), C.byref(m))
@@ -285,7 +286,8 @@ def kernel_block_attention(q, k, v, block_mask, heads: int, stream=None, out=Non
 
 
 def block_masked_attention(q, k, v, block_mask, heads: int, stream=None, out=None) -> torch.Tensor:
-    """The dense fallback's result (unselected blocks weigh exactly 0, so they are not visited). DiT.swift:279-313."""
+    """The dense fallback's result (unselected blocks weigh exactly 0, so they are not read: a NaN or an infinity in one
+    does not reach the output). DiT.swift:279-313."""
     return _attn_mask(q, k, v, block_mask, heads, ATTN_DENSE, stream, out)
 
 

@@ -63,7 +63,8 @@ public func localBlockMask(bh: Int, bw: Int, range r: Int) -> [UInt8] {
     return m
 }
 
-/// The `auto` rule of blockForward (DiT.swift:517-522): kernel when the expected kept fraction is <= 0.45.
+/// The `auto` rule of blockForward (DiT.swift:517-522): kernel when the expected kept fraction is <= 0.45. The layer
+/// calls return the same in every mode.
 public func attentionModeAuto(topk: Int, spatialBlocks s: Int, keyBlocks nk: Int,
                               threshold: Double = 0.45) -> (expected: Double, mode: fvsr_attn_mode) {
     var e = 0.0
@@ -100,7 +101,8 @@ public func kernelBlockAttention(_ c: LCSAContext, q: DeviceTensor, k: DeviceTen
                                        stream), "fvsr_lcsa_attention_mask")
 }
 
-/// `blockMaskedAttention` (DiT.swift:279-313): the dense fallback (same values and, here, the same walk).
+/// `blockMaskedAttention` (DiT.swift:279-313): the dense fallback (same values and, here, the same walk: unselected
+/// blocks are not read, so a NaN or an infinity in one does not reach the output).
 public func blockMaskedAttention(_ c: LCSAContext, q: DeviceTensor, k: DeviceTensor, v: DeviceTensor,
                                  blockMask: DeviceTensor, heads: Int, out: DeviceTensor, stream: HIPStream = nil) {
     fvsrCheck(fvsr_lcsa_attention_mask(c.ctx, q.dtype, q.ptr, Int64(q.rows), k.ptr, v.ptr, Int64(k.rows),

@@ -670,3 +670,23 @@ def test_fp32_error_is_relative_to_what_counts(dev, what, size):
             # half a unit of the smallest fp32 number, where the result itself is one
             err = (err - 2.0 ** -149).clamp_min(0.0) / ref.abs().amax(0)
             assert float(err.max()) <= FP32_REL, (n, h, float(err.max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,lqb,nkb", [(2, 3, 6), (12, 43, 6)])
+def test_unselected_blocks_are_not_read(dev, dtype, heads, lqb, nkb):
+    """NaN and infinities in a block that no row selects, and in one that only the first row selects, reach neither mode's
+    output elsewhere: the same bits as without them (6 rows, split; 516, past the resident workgroups)."""
+    gen = torch.Generator(device=dev).manual_seed(lqb)
+    q, k, v = (torch.randn((n * 128, heads * 128), generator=gen, device=dev).to(dtype) for n in (lqb, nkb, nkb))
+    m = (torch.rand((heads, lqb, nkb), generator=gen, device=dev) < 0.6).float()
+    m[:, :, 2] = 0.0
+    m[:, :, 4] = 0.0
+    m[:, 0, 4] = 1.0
+    clean = fvsr_lcsa.kernel_block_attention(q, k, v, m, heads)
+    k[2 * 128:3 * 128], v[2 * 128:3 * 128] = float("nan"), float("inf")
+    v[4 * 128 + 7] = float("nan")
+    for call in (fvsr_lcsa.kernel_block_attention, fvsr_lcsa.block_masked_attention):
+        o = call(q, k, v, m, heads)
+        assert torch.equal(o[128:], clean[128:])
+        assert bool(o[:128].isnan().all())
