@@ -84,6 +84,7 @@ static Carve carve(int heads, int64_t nq, int64_t nk, int C) {
   c.thr = off; off += align256((size_t)heads * nq * 4);   // per (head, query slice) thresholds (nq >= slices)
   c.hist = off; off += align256(hist12_bytes(heads, (int)nq));   // nq >= query slices
   c.cand = off; off += align256(topk_cand_bytes(heads, nq));
+  // grows with rows and keys, also past the rows that are split: a stream's later, smaller chunks fit its first one's carve
   c.part = off; off += align256((size_t)attn_partial_items(heads * nq, (int)nk) * kPartialFloats * 4);
   c.total = off;
   return c;

@@ -128,7 +128,7 @@ __device__ __forceinline__ int swz_v(int r) { return (r & 3) << 2; }
 // the end of the walk, whose block offset is the buffer's size) load zeros without touching memory.
 template <int OFF>
 __device__ __forceinline__ void dma16(u32x4 rsrc, uint32_t lds_base, int voff, int boff) {
-  const uint32_t off = (uint32_t)voff + (uint32_t)boff;   // < 2^31 + 2^17: no wrap
+  const uint32_t off = (uint32_t)voff + (uint32_t)boff;   // voff holds the head's offset, inside the buffer: < 2^32
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base + OFF),
                "v"(off), "s"(rsrc));
 }
